@@ -99,12 +99,6 @@ __device__ __forceinline__ uint64_t insert_zero(uint64_t t, uint32_t h)
 	return ((t >> h) << (h + 1)) | lo;
 }
 
-__device__ __forceinline__ uint32_t insert_zero32(uint32_t t, uint32_t h)
-{
-	const uint32_t lo = t & ((1u << h) - 1);
-	return ((t >> h) << (h + 1)) | lo;
-}
-
 // Update of one pair (a_i, a_j), i < j, P|i> = i^r4 |j>:
 //   a_i <- c a_i + i conj(s i^r4) a_j,   a_j <- c a_j + i (s i^r4) a_i.
 // For odd r4 the partner enters as itself, for even r4 as i*partner
@@ -237,422 +231,119 @@ __global__ __launch_bounds__(kBlock) void k_rot_diag(
 //
 // LDS slots are XOR-swizzled (bits >= 4 folded into bits 0..3) so that the
 // strided cosets of a wave spread over the banks.
-
-// The descriptors are kernel arguments read with wave-uniform indices.
-// Every field the kernels read is an aligned 32-bit word (byte fields are
-// read through the word that holds them), so all of them come in through
-// scalar loads: a byte or unaligned read would become a vector-memory load
-// that shares the wait counter with the tile's HBM traffic.
-struct alignas(16) FusedTerm {
+//
+// The host plans a pass in the structures below (FusedPass) and packs what
+// the kernels read into a compact descriptor (DevPass, pack_pass).  Every
+// map the kernels need is linear over GF(2) in the thread index: the tile
+// coordinate of a thread's coset, with it the HBM index of the coset, its
+// LDS slot and the parity of the coset with a term's phase mask.  So the
+// descriptor holds one column per thread-index bit for each map, and a
+// kernel forms a value as the XOR of the columns of its set bits: two
+// vector operations per lane bit, scalar ones for the bits that select a
+// wave.  Spreading the index over the free tile bits and gathering the
+// basis vectors bit by bit took about 60 vector and 100 scalar
+// instructions per exchange and two chains of about ten dependent scalar
+// loads per tile, and a scalar instruction costs a wave as much issue time
+// as a vector one (measured on gfx950: one scalar instruction per 4.3
+// clocks per SIMD, one FP64 instruction per 4.5).
+struct FusedTerm {
 	uint64_t z;    // physical phase mask (per-tile parity)
 	double c, s;
 	uint32_t zt;   // phase mask in tile coordinates (bits 0..15) and the
 	               // per-register signs parity(w & ztp) (bits 16..31)
-	union {
-		struct {
-			uint8_t xtp;   // flip mask in group coordinates
-			uint8_t ztp;   // parity(u_i & zt), group coordinates
-			uint8_t y;     // popcount(x & z) & 3
-			uint8_t pad;
-		};
-		uint32_t meta;
-	};
+	uint8_t xtp;   // flip mask in group coordinates
+	uint8_t ztp;   // parity(u_i & zt), group coordinates
+	uint8_t y;     // popcount(x & z) & 3
 };
 
-struct alignas(16) FusedGroup {
-	union {
-		uint16_t u[4];   // group basis, tile coordinates
-		uint32_t uw[2];
-	};
-	union {
-		uint8_t piv[4];  // its leading bits, ascending
-		uint32_t pivw;
-	};
-	union {
-		uint8_t jpos[12];// tile bit of each coset-index bit (the free bits)
-		uint32_t jposw[3];
-	};
-	union {
-		struct {
-			// terms first .. first + count; for a half-tile pass,
-			// the exchange to the next group splits the tile by tile
-			// bit xh, carried by coset-index bit xk
-			uint8_t first, count, xh, xk;
-		};
-		uint32_t fcw;
-	};
-	uint32_t pad3[1];
+struct FusedGroup {
+	uint16_t u[4];   // group basis, tile coordinates
+	uint8_t piv[4];  // its leading bits, ascending
+	uint8_t jpos[12];// tile bit of each coset-index bit (the free bits)
+	// terms first .. first + count; for a half-tile pass, the exchange to
+	// the next group splits the tile by tile bit xh, carried by
+	// coset-index bit xk
+	uint8_t first, count, xh, xk;
 };
-
-constexpr int kMaxPer = (1 << PH2HIP_TILE_MAX) / kBlock;
 
 struct FusedPass {
 	uint64_t w[PH2HIP_TILE_MAX];   // gathered basis vectors
-	uint64_t roff[kMaxPer];        // gathered offset of load/store step m
-	// Offset (row part ^ column part) of coset element w of the first
-	// ([0]) and last ([1]) micro-group, for groups that move their cosets
-	// straight between HBM and registers (dflags).
-	uint64_t dcw[2][16];
 	uint32_t piv[PH2HIP_TILE_MAX]; // their leading bits, ascending
-	union {
-		struct {
-			uint8_t L, g, ngroups, nterms;
-		};
-		uint32_t hdr;
-	};
+	uint8_t L, g, ngroups, nterms;
 	// bit 0: the first group loads its cosets from HBM (the tile is not
-	// staged in LDS first); bit 1: the last group stores them to HBM.
+	// staged in LDS first); bit 1: the last group stores them to HBM;
+	// bit 2: the half-tile form.
 	uint32_t dflags;
 	FusedGroup grp[PH2HIP_PASS_MAX];
 	FusedTerm t[PH2HIP_PASS_MAX];
 };
 
-// Device-side reads of the packed fields.
-__device__ __forceinline__ uint32_t pass_L(const FusedPass &P)
-{
-	return P.hdr & 0xffu;
-}
-__device__ __forceinline__ uint32_t pass_g(const FusedPass &P)
-{
-	return (P.hdr >> 8) & 0xffu;
-}
-__device__ __forceinline__ uint32_t pass_ngroups(const FusedPass &P)
-{
-	return (P.hdr >> 16) & 0xffu;
-}
+// Packed descriptor: a head, the groups, the terms, without gaps.  Read
+// through scalar loads only.
+constexpr int kThreadBits = 10;   // thread-index bits a column set covers
+constexpr int kSegMax = PH2HIP_TILE_MAX + 1;
 
-static_assert(sizeof(FusedPass) <= 4000, "kernel argument too large");
+struct DevHead {
+	uint32_t ngroups;
+	uint32_t nseg;
+	// tile index -> base index: bits [src, src + width) move to dst;
+	// src | dst << 8 | width << 16 (width 0: unused)
+	uint32_t seg[kSegMax];
+	// HBM index columns of the first and last group's cosets, and of
+	// their basis vectors
+	uint64_t col[2][kThreadBits];
+	uint64_t dc[2][4];
+};
+
+struct DevGroup {
+	uint32_t count;      // terms
+	uint32_t xk;         // half-tile exchange: wave bit of the half
+	uint32_t toff;       // byte offset of the first term
+	// LDS byte offsets (>> kShift) of the exchange to the next group:
+	// where this group's cosets are written (low half) and the next
+	// group's are read (high half), per thread-index bit and per basis
+	// vector
+	uint32_t col[kThreadBits];
+	uint32_t g[4];
+};
+
+struct DevTerm {
+	uint64_t z;          // phase mask (per-tile parity)
+	double c, s;         // s negated where bit 1 of y is set
+	uint32_t zt;         // phase mask in thread-index bits (low half) and
+	                     // the per-register signs (high half)
+	uint32_t code;       // handler: even patterns, odd patterns, diagonal
+};
+
+static_assert(sizeof(DevTerm) == 32, "term stride of the kernels");
+
+// Two more groups than the pass has: the ones that only move the tile
+// between HBM and LDS (pack_pass).  One term more: the kernels fetch the
+// term after the one they run.
+constexpr size_t kDevMax = sizeof(DevHead) +
+	(PH2HIP_PASS_MAX + 2) * sizeof(DevGroup) +
+	(PH2HIP_PASS_MAX + 1) * sizeof(DevTerm);
+
+struct alignas(16) DevPass {
+	uint8_t b[(kDevMax + 15) & ~size_t{15}];
+};
+
+#define PH2_CONST __attribute__((address_space(4)))
+typedef const PH2_CONST DevHead *cHead;
+typedef const PH2_CONST DevGroup *cGroup;
+
+typedef double v2d __attribute__((ext_vector_type(2)));
 
 // LDS slot of tile coordinate v: bits >= 4 folded into bits 0..3.  The map
 // is GF(2)-linear, so slot(a ^ b) = slot(a) ^ slot(b).
-typedef double v2d __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ uint32_t lds_slot(uint32_t v)
+constexpr uint32_t lds_slot(uint32_t v)
 {
 	return v ^ (((v >> 4) ^ (v >> 8)) & 15u);
 }
 
-__device__ __forceinline__ double flip_sign(double v, uint32_t f)
-{
-	return __hiloint2double(__double2hiint(v) ^ (int)(f << 31),
-		__double2loint(v));
-}
-
-// One pair update in place: (x, y) of one coset pair, c uniform, si the
-// per-thread signed sine, si = sb * sg with sg = +-1.0 uniform.  ODD:
-// x <- c x + si y,  y <- c y - si x;  even:  x <- c x + si (i y),
-// y <- c y + si (i x), per component as in rot_pair.  Each result is
-// round(round(c u) +- round(si v)), the same roundings as
-// add(mul(c, u), mul(+-si, v)) (negation is exact).  Written as one block
-// with the four values read and written in place: as plain code the
-// compiler gives each term's results new registers and then copies the
-// whole coset back once per term at the loop back-edge.  The real and the
-// imaginary halves are two independent 2x2 updates sharing four
-// temporaries, and si is formed inside the block, so a pair holds five
-// temporaries at most (the scheduler would otherwise form the signed
-// sines of all pairs of a term early and keep them live).
-template <bool ODD>
-__device__ __forceinline__ void pair_inplace(double &xr, double &xi,
-	double &yr, double &yi, double c, double sb, double sg)
-{
-	double si, t0, t1, t2, t3;
-	if (ODD)
-		__asm__(
-			"v_mul_f64 %[si], %[sg], %[sb]\n\t"
-			"v_mul_f64 %[t0], %[c], %[xr]\n\t"
-			"v_mul_f64 %[t2], %[c], %[yr]\n\t"
-			"v_mul_f64 %[t1], %[si], %[yr]\n\t"
-			"v_mul_f64 %[t3], %[si], %[xr]\n\t"
-			"v_add_f64 %[xr], %[t0], %[t1]\n\t"
-			"v_add_f64 %[yr], %[t2], -%[t3]\n\t"
-			"v_mul_f64 %[t0], %[c], %[xi]\n\t"
-			"v_mul_f64 %[t2], %[c], %[yi]\n\t"
-			"v_mul_f64 %[t1], %[si], %[yi]\n\t"
-			"v_mul_f64 %[t3], %[si], %[xi]\n\t"
-			"v_add_f64 %[xi], %[t0], %[t1]\n\t"
-			"v_add_f64 %[yi], %[t2], -%[t3]"
-			: [xr] "+v"(xr), [xi] "+v"(xi), [yr] "+v"(yr),
-			  [yi] "+v"(yi), [si] "=&v"(si), [t0] "=&v"(t0),
-			  [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3)
-			: [c] "s"(c), [sb] "v"(sb), [sg] "s"(sg));
-	else
-		__asm__(
-			"v_mul_f64 %[si], %[sg], %[sb]\n\t"
-			"v_mul_f64 %[t0], %[c], %[xr]\n\t"
-			"v_mul_f64 %[t2], %[c], %[yi]\n\t"
-			"v_mul_f64 %[t1], %[si], %[yi]\n\t"
-			"v_mul_f64 %[t3], %[si], %[xr]\n\t"
-			"v_add_f64 %[xr], %[t0], -%[t1]\n\t"
-			"v_add_f64 %[yi], %[t2], %[t3]\n\t"
-			"v_mul_f64 %[t0], %[c], %[xi]\n\t"
-			"v_mul_f64 %[t2], %[c], %[yr]\n\t"
-			"v_mul_f64 %[t1], %[si], %[yr]\n\t"
-			"v_mul_f64 %[t3], %[si], %[xi]\n\t"
-			"v_add_f64 %[xi], %[t0], %[t1]\n\t"
-			"v_add_f64 %[yr], %[t2], -%[t3]"
-			: [xr] "+v"(xr), [xi] "+v"(xi), [yr] "+v"(yr),
-			  [yi] "+v"(yi), [si] "=&v"(si), [t0] "=&v"(t0),
-			  [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3)
-			: [c] "s"(c), [sb] "v"(sb), [sg] "s"(sg));
-}
-
-// Diagonal update in place: a <- c a + sj (i a) with sj = sb * sg, i.e.
-// (c re - sj im, c im + sj re), the roundings of rot_diag.
-__device__ __forceinline__ void diag_inplace(double &re, double &im,
-	double c, double sb, double sg)
-{
-	double sj, t0, t1, t2, t3;
-	__asm__(
-		"v_mul_f64 %[sj], %[sg], %[sb]\n\t"
-		"v_mul_f64 %[t0], %[c], %[re]\n\t"
-		"v_mul_f64 %[t2], %[c], %[im]\n\t"
-		"v_mul_f64 %[t1], %[sj], %[im]\n\t"
-		"v_mul_f64 %[t3], %[sj], %[re]\n\t"
-		"v_add_f64 %[re], %[t0], -%[t1]\n\t"
-		"v_add_f64 %[im], %[t2], %[t3]"
-		: [re] "+v"(re), [im] "+v"(im), [sj] "=&v"(sj), [t0] "=&v"(t0),
-		  [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3)
-		: [c] "s"(c), [sb] "v"(sb), [sg] "s"(sg));
-}
-
-// High word of +-1.0 for coset register w: -1.0 if bit w of the term's
-// sign mask is set.  A bit test and a select on the scalar unit.
-__device__ __forceinline__ double reg_sign(uint32_t sgn, int w)
-{
-	return __hiloint2double((sgn >> w & 1u) ? (int)0xbff00000 :
-		0x3ff00000, 0);
-}
-
-// +-1.0 with the sign bit f (an exact multiplier)
-__device__ __forceinline__ double unit_sign(uint32_t f)
-{
-	return __hiloint2double(0x3ff00000 | (int)(f << 31), 0);
-}
-
-// One term with compile-time flip pattern XT on a coset of 2^D amplitudes
-// held as (re, im) register quads, so that the 16-byte HBM and LDS moves
-// read and write them in place (with re and im in separate arrays the
-// compiler pairs them up with two copies per move).  r4 = y + 2*par (mod 4)
-// with par = bpt ^ parity(w & ztp).  Odd y: the partner enters as itself
-// and s_j = -s_i; even y: as i*partner and s_j = s_i.  s_i = s with its
-// sign flipped by par ^ bit1(y); sb already carries bpt ^ bit1(y), so per
-// pair only parity(w & ztp) (uniform) flips.
-template <int D, int XT, bool ODD>
-__device__ __forceinline__ void coset_term(v2d (&a)[1 << D], uint32_t sgn,
-	double sb, double c)
-{
-	constexpr int H = 31 - __builtin_clz(XT);
-#pragma unroll
-	for (int q = 0; q < (1 << (D - 1)); q++) {
-		const int w = ((q >> H) << (H + 1)) | (q & ((1 << H) - 1));
-		double xr = a[w].x, xi = a[w].y, yr = a[w ^ XT].x,
-			yi = a[w ^ XT].y;
-		// per pair only the uniform sign (scalar unit) changes: one
-		// exact multiply by +-1.0 held in scalar registers
-		pair_inplace<ODD>(xr, xi, yr, yi, c, sb, reg_sign(sgn, w));
-		a[w].x = xr;
-		a[w].y = xi;
-		a[w ^ XT].x = yr;
-		a[w ^ XT].y = yi;
-	}
-}
-
-// xtp is in 1 .. 2^D - 1 (built so on the host); the last pattern takes
-// every value not matched before it, so that no path leaves the coset
-// unchanged: such a path makes the compiler copy all 2^(D+1) coset
-// registers once per term at the loop back-edge.
-template <int D, bool ODD, int XT = 1>
-__device__ __forceinline__ void coset_dispatch(v2d (&a)[1 << D],
-	uint32_t xtp, uint32_t sgn, double sb, double c)
-{
-	if constexpr (XT == (1 << D) - 1) {
-		coset_term<D, XT, ODD>(a, sgn, sb, c);
-	} else {
-		if (xtp == XT) {
-			coset_term<D, XT, ODD>(a, sgn, sb, c);
-			return;
-		}
-		coset_dispatch<D, ODD, XT + 1>(a, xtp, sgn, sb, c);
-	}
-}
-
-__device__ __forceinline__ uint64_t tile_base(const FusedPass &P, uint64_t t)
-{
-	uint64_t base = t << pass_L(P);
-	const uint32_t g = pass_g(P);
-	for (uint32_t b = 0; b < g; b++)
-		base = insert_zero(base, P.piv[b]);
-	return base;
-}
-
-// The terms of one micro-group (P.t[first .. first + count), fcw) on one
-// coset of 2^D registers with base coordinate bu in the tile at base.
-template <int D>
-__device__ __forceinline__ void group_terms(v2d (&a)[1 << D],
-	const FusedPass &P, uint32_t fcw, uint32_t bu, uint64_t base)
-{
-	const uint32_t kfirst = fcw & 0xffu;
-	const uint32_t kend = kfirst + ((fcw >> 8) & 0xffu);
-	// term k + 1 is loaded (scalar loads) while term k runs
-	uint64_t tz = P.t[kfirst].z;
-	double c = P.t[kfirst].c, ts = P.t[kfirst].s;
-	uint32_t tzt = P.t[kfirst].zt, meta = P.t[kfirst].meta;
-	for (uint32_t k = kfirst; k < kend; k++) {
-		const uint32_t kn = k + 1 < kend ? k + 1 : k;
-		const uint64_t tz_n = P.t[kn].z;
-		const double c_n = P.t[kn].c, ts_n = P.t[kn].s;
-		const uint32_t tzt_n = P.t[kn].zt,
-			meta_n = P.t[kn].meta;
-		const uint32_t xtp = meta & 0xffu;
-		const uint32_t ty = (meta >> 16) & 0xffu;
-		const uint32_t sgn = tzt >> 16;
-		const uint32_t bpt = (__popc(bu & (tzt & 0xffffu)) ^
-			__popcll(base & tz)) & 1u;
-		if (xtp == 0) {
-			// diagonal: a <- c a + s_j (i a), s_j = +-s
-			const double sb = flip_sign(ts, bpt);
-#pragma unroll
-			for (int w = 0; w < (1 << D); w++) {
-				double re = a[w].x, im = a[w].y;
-				diag_inplace(re, im, c, sb, reg_sign(sgn, w));
-				a[w].x = re;
-				a[w].y = im;
-			}
-		} else {
-			const double sb = flip_sign(ts,
-				bpt ^ ((ty >> 1) & 1u));
-			if (ty & 1)
-				coset_dispatch<D, true>(a, xtp, sgn, sb,
-					c);
-			else
-				coset_dispatch<D, false>(a, xtp, sgn, sb,
-					c);
-		}
-		tz = tz_n;
-		c = c_n;
-		ts = ts_n;
-		tzt = tzt_n;
-		meta = meta_n;
-		// each quad stays one register quad across terms: without this
-		// the D = 3 coset was copied whole at the loop back-edge
-#pragma unroll
-		for (int w = 0; w < (1 << D); w++)
-			__asm__ volatile("" : "+v"(a[w]));
-	}
-}
-
-// Tile coordinate of coset j's base: j's bits spread over the free tile
-// bits jpos (three packed words).
-template <int TB, int D>
-__device__ __forceinline__ uint32_t coset_base(uint32_t j, uint32_t jw0,
-	uint32_t jw1, uint32_t jw2)
-{
-	const uint32_t jw[3] = { jw0, jw1, jw2 };
-	uint32_t bu = 0;
-#pragma unroll
-	for (int k = 0; k < TB - D; k++)
-		bu |= (j >> k & 1u) << ((jw[k >> 2] >> (8 * (k & 3))) & 0xffu);
-	return bu;
-}
-
-// HBM index of tile coordinate bu (row part ^ column part).
-__device__ __forceinline__ uint64_t hbm_index(const FusedPass &P,
-	uint64_t base, uint32_t bu, uint32_t L, uint32_t g)
-{
-	uint64_t abu = base ^ (bu & ((1u << L) - 1));
-	for (uint32_t b = 0; b < g; b++)
-		if ((bu >> (L + b)) & 1u)
-			abu ^= P.w[b];
-	return abu;
-}
-
-// All micro-groups of a pass on one tile.  Each group's cosets come from
-// and go back to the LDS tile, except that with dflags bit 0 the first
-// group reads its cosets straight from HBM (the tile was not staged) and
-// with bit 1 the last group writes them straight to HBM (the tile is not
-// stored from LDS afterwards).  Those groups map coset-index bits 0..3 to
-// tile bits 0..3 (checked on the host, with L >= 4), so 16 lanes move one
-// 256-byte run; a pass of one group then never touches LDS.
-template <int TB, int D>
-__device__ __forceinline__ void tile_groups(v2d *__restrict__ a, v2d *tile,
-	const FusedPass &P, uint64_t base, uint32_t tid, uint32_t dflags)
-{
-	constexpr uint32_t NSUB = (1u << TB) >> D;    // cosets per group
-	static_assert(NSUB % kBlock == 0, "cosets must cover the block");
-	const uint32_t ngroups = pass_ngroups(P);
-	const uint32_t L = pass_L(P), g = pass_g(P);
-	for (uint32_t gi = 0; gi < ngroups; gi++) {
-		const uint32_t uw0 = P.grp[gi].uw[0], uw1 = P.grp[gi].uw[1];
-		const uint32_t jw0 = P.grp[gi].jposw[0], jw1 = P.grp[gi].jposw[1],
-			jw2 = P.grp[gi].jposw[2];
-		const uint32_t fcw = P.grp[gi].fcw;
-		const uint32_t gu[4] = { uw0 & 0xffffu, uw0 >> 16, uw1 & 0xffffu,
-			uw1 >> 16 };
-		// byte offsets of the basis vectors' LDS slots (the slot map is
-		// linear, so an element's offset is the XOR of these)
-		uint32_t gs[4];
-#pragma unroll
-		for (int i = 0; i < 4; i++)
-			gs[i] = lds_slot(gu[i]) << 4;
-		const bool gload = gi == 0 && (dflags & 1u);
-		const bool gstore = gi + 1 == ngroups && (dflags & 2u);
-		if (!gload)
-			__syncthreads();
-		for (uint32_t j = tid; j < NSUB; j += kBlock) {
-			const uint32_t bu = coset_base<TB, D>(j, jw0, jw1, jw2);
-			// byte offset of the coset base's slot: the per-element
-			// offsets (uniform) are XORed in pre-shifted, one VALU
-			// operation per LDS access
-			uint32_t sbu16 = lds_slot(bu) << 4;
-			__asm__("" : "+v"(sbu16));   // keeps the shift out of
-			                             // the per-access XOR
-			const uint64_t abu = (gload || gstore) ?
-				hbm_index(P, base, bu, L, g) : 0;
-			v2d cs[1 << D];
-			if (gload) {
-#pragma unroll
-				for (int w = 0; w < (1 << D); w++)
-					cs[w] = a[abu ^ P.dcw[0][w]];
-			} else {
-#pragma unroll
-				for (int w = 0; w < (1 << D); w++) {
-					uint32_t cw16 = 0;
-#pragma unroll
-					for (int i = 0; i < D; i++)
-						if (w >> i & 1)
-							cw16 ^= gs[i];
-					cs[w] = *reinterpret_cast<const v2d *>(
-						reinterpret_cast<const char *>(tile) +
-						(sbu16 ^ cw16));
-				}
-			}
-			group_terms<D>(cs, P, fcw, bu, base);
-			if (gstore) {
-#pragma unroll
-				for (int w = 0; w < (1 << D); w++)
-					a[abu ^ P.dcw[1][w]] = cs[w];
-			} else {
-#pragma unroll
-				for (int w = 0; w < (1 << D); w++) {
-					uint32_t cw16 = 0;
-#pragma unroll
-					for (int i = 0; i < D; i++)
-						if (w >> i & 1)
-							cw16 ^= gs[i];
-					*reinterpret_cast<v2d *>(
-						reinterpret_cast<char *>(tile) +
-						(sbu16 ^ cw16)) = cs[w];
-				}
-			}
-		}
-	}
-	if (!(dflags & 2u))
-		__syncthreads();
-}
-
-// Slot of tile coordinate v in a buffer of half a tile: bits h and TB-1
+// Slot of tile coordinate v in a buffer of half a tile: bits h and tb-1
 // exchanged, then bits 4 and up folded into bits 0..3 through
-// y ^ (y >> 1) ^ (y >> 3) with y = v >> 4, then bit TB-1 dropped.  Linear,
+// y ^ (y >> 1) ^ (y >> 3) with y = v >> 4, then bit tb-1 dropped.  Linear,
 // and one-to-one on each half {v : bit h of v = const}.
 //
 // Banks, as measured on gfx950 with the LDS conflict counters: a 16-byte
@@ -665,216 +356,446 @@ __device__ __forceinline__ void tile_groups(v2d *__restrict__ a, v2d *tile,
 // mod 16.  The whole-tile fold (bank vector t mod 4 for tile bit t) runs
 // out of a residue for many groups: 15% of LDS cycles were conflicts at
 // tile 12 with it, 6% at tile 13.
-template <int TB>
-__device__ __forceinline__ uint32_t half_slot(uint32_t v, uint32_t h)
+constexpr uint32_t half_slot(uint32_t tb, uint32_t v, uint32_t h)
 {
-	const uint32_t t = ((v >> h) ^ (v >> (TB - 1))) & 1u;
-	v ^= t * ((1u << h) | (1u << (TB - 1)));
+	const uint32_t t = ((v >> h) ^ (v >> (tb - 1))) & 1u;
+	v ^= t * ((1u << h) | (1u << (tb - 1)));
 	v ^= ((v >> 4) ^ (v >> 5) ^ (v >> 7)) & 15u;
-	return v & ((1u << (TB - 1)) - 1);
+	return v & ((1u << (tb - 1)) - 1);
 }
 
-// Byte offsets in the half buffer of a group's basis vectors (uniform).
-template <int TB>
-__device__ __forceinline__ void half_offsets(const FusedGroup &G, uint32_t h,
-	uint32_t (&gs)[4])
+// LDS byte offsets are packed in 16 bits, shifted right by this: only the
+// whole-tile form of tile 13 (128 KiB) has larger ones.
+constexpr int lds_shift(int tb, bool half)
 {
-	const uint32_t uw0 = G.uw[0], uw1 = G.uw[1];
-	gs[0] = half_slot<TB>(uw0 & 0xffffu, h) << 4;
-	gs[1] = half_slot<TB>(uw0 >> 16, h) << 4;
-	gs[2] = half_slot<TB>(uw1 & 0xffffu, h) << 4;
-	gs[3] = half_slot<TB>(uw1 >> 16, h) << 4;
+	return tb == 13 && !half ? 1 : 0;
 }
 
-// All micro-groups of a pass on one tile with half a tile of LDS, from the
-// first group's cosets in cs (coset base bu of group 0, read from HBM by
-// the caller) to the last group's, which go back to HBM.  Between groups q
-// and q+1 the cosets move through the buffer in two rounds, one per half of
-// the tile (split bit xh of group q; the threads of one half are the waves
-// whose coset-index bit xk is that half).  One coset per thread: 2^(TB - D)
-// threads.  fresh: the buffer has no earlier readers in this workgroup (its
-// first tile), so the first exchange needs no barrier before writing.
-template <int TB, int D>
-__device__ __forceinline__ void half_groups(v2d *__restrict__ a, v2d *buf,
-	const FusedPass &P, uint64_t base, uint32_t tid, v2d (&cs)[1 << D],
-	uint32_t bu, bool fresh)
+// ---------------------------------------------------------------------------
+// the terms of one micro-group
+// ---------------------------------------------------------------------------
+//
+// A coset is 2^D amplitudes of one thread as (re, im) register quads in
+// fixed registers (v16 up), the form in which the 16-byte HBM and LDS moves
+// read and write them.  The terms run in one block of assembly, for what
+// surrounds the FP64 work costs as much as the work: with the term loop in
+// C++ each term took about 45 scalar instructions, nine vector ones and
+// eight branches besides its pair updates (a taken branch holds a wave for
+// about 20 clocks), here 15, three and one.  With the linear maps above, a
+// sweep of 1024 terms took 644, 2215 and 10993 us at 18, 22 and 25 qubits
+// before and 526, 1846 and 10536 us after; 1163 and 1133 ms at 31 qubits,
+// where HBM weighs more.
+//
+// Term k + 1 is fetched (one scalar load) while term k runs.  Dispatch: the
+// term's code picks its handler, one per flip pattern XT in 1 .. 2^D - 1,
+// first for even y, then for odd, then the diagonal one; the handlers of
+// the patterns have one size, so the address is a product.  A handler ends
+// with the next dispatch itself.
+//
+// Signs.  P|i> = i^r4 |i ^ x> with r4 = y + 2 par (mod 4), par the parity of
+// i & z.  Odd y: the partner enters as itself and s_j = -s_i; even y: as
+// i*partner and s_j = s_i.  par = parity(tile base & z) ^ parity(thread
+// index & zt) ^ parity(w & ztp), w the register.  The first is uniform and
+// the second per thread: both go into the sign bit of sg = +-1.0.  The
+// third is a bit of the term's sign mask: the uniform sine +-s of pair w is
+// picked by a bit test and a select on the scalar unit.  sg enters in the
+// sum: fma(sg, t, u) with sg = +-1.0 has an exact product, so it rounds
+// once, to round(u +- t), and each result is round(round(c u) +-
+// round(s v)), the same roundings as add(mul(c, u), mul(+-s, v)).  A pair
+// costs the 8 products and 4 sums of its definition, and nothing for signs.
+//
+// Registers: v[4:11] temporaries, v[12:13] sg, v14 scratch; s[72:79] the
+// next term, s80 terms left, s81 its offset, s[84:85] first handler,
+// s[86:87] scratch, s[88:89] c, s[90:91] the signed s of the pair, s92/s93
+// high words of s and -s, s94 sign masks.
+#define PH2_TERM_MACROS                                                     \
+	".ifndef ph2_macros\n"                                              \
+	".set ph2_macros, 1\n"                                              \
+	/* next term: its scalars, sg, the fetch of the one after, jump */  \
+	".macro PH2_NEXT id\n"                                              \
+	"s_sub_u32 s80, s80, 1\n"                                           \
+	"s_cbranch_scc1 .Lph2x\\id\n"                                       \
+	"s_waitcnt lgkmcnt(0)\n"                                            \
+	"s_and_b64 s[86:87], s[72:73], s[82:83]\n"                          \
+	"v_and_b32 v14, s78, v15\n"                                         \
+	"s_bcnt1_i32_b64 s86, s[86:87]\n"                                   \
+	"s_mov_b64 s[88:89], s[74:75]\n"                                    \
+	"v_bcnt_u32_b32 v14, v14, s86\n"                                    \
+	"s_mov_b64 s[90:91], s[76:77]\n"                                    \
+	"s_mov_b32 s92, s77\n"                                              \
+	"v_lshl_or_b32 v13, v14, 31, s95\n"                                 \
+	"s_xor_b32 s93, s77, 0x80000000\n"                                  \
+	"s_mov_b32 s94, s78\n"                                              \
+	"s_mul_i32 s86, s79, (.Lph2n\\id - .Lph2h\\id)\n"                   \
+	"s_add_u32 s86, s84, s86\n"                                         \
+	"s_addc_u32 s87, s85, 0\n"                                          \
+	"s_load_dwordx8 s[72:79], s[70:71], s81\n"                          \
+	"s_add_u32 s81, s81, 32\n"                                          \
+	"s_setpc_b64 s[86:87]\n"                                            \
+	".endm\n"                                                           \
+	/* one half of a pair update on doubles v[x], v[y], v[p], v[q]:     \
+	 * x <- c x +- sg s p, y <- c y +- sg s q with p, q the partners */ \
+	".macro PH2_HALF x, y, p, q, nx, ny\n"                              \
+	"v_mul_f64 v[4:5], s[90:91], v[\\p:\\p+1]\n"                        \
+	"v_mul_f64 v[6:7], s[90:91], v[\\q:\\q+1]\n"                        \
+	"v_mul_f64 v[8:9], s[88:89], v[\\x:\\x+1]\n"                        \
+	"v_mul_f64 v[10:11], s[88:89], v[\\y:\\y+1]\n"                      \
+	".if \\nx\n"                                                        \
+	"v_fma_f64 v[\\x:\\x+1], v[12:13], -v[4:5], v[8:9]\n"               \
+	".else\n"                                                           \
+	"v_fma_f64 v[\\x:\\x+1], v[12:13], v[4:5], v[8:9]\n"                \
+	".endif\n"                                                          \
+	".if \\ny\n"                                                        \
+	"v_fma_f64 v[\\y:\\y+1], v[12:13], -v[6:7], v[10:11]\n"             \
+	".else\n"                                                           \
+	"v_fma_f64 v[\\y:\\y+1], v[12:13], v[6:7], v[10:11]\n"              \
+	".endif\n"                                                          \
+	".endm\n"                                                           \
+	".macro PH2_SINE w\n"                                               \
+	".if \\w\n"                                                         \
+	"s_bitcmp1_b32 s94, 16+\\w\n"                                       \
+	"s_cselect_b32 s91, s93, s92\n"                                     \
+	".endif\n"                                                          \
+	".endm\n"                                                           \
+	/* a pattern: pairs (w, w ^ xt), bit h the top one of xt */         \
+	".macro PH2_PATTERN np, xt, h, odd\n"                               \
+	".set ph2_k, 0\n"                                                   \
+	".rept \\np\n"                                                      \
+	".set ph2_w, ((ph2_k>>\\h)<<(\\h+1))+(ph2_k&((1<<\\h)-1))\n"        \
+	".set ph2_a, 16+4*ph2_w\n"                                          \
+	".set ph2_b, 16+4*(ph2_w^\\xt)\n"                                   \
+	"PH2_SINE ph2_w\n"                                                  \
+	".if \\odd\n"                                                       \
+	"PH2_HALF ph2_a, ph2_b, ph2_b, ph2_a, 0, 1\n"                       \
+	"PH2_HALF ph2_a+2, ph2_b+2, ph2_b+2, ph2_a+2, 0, 1\n"               \
+	".else\n"                                                           \
+	"PH2_HALF ph2_a, ph2_b+2, ph2_b+2, ph2_a, 1, 0\n"                   \
+	"PH2_HALF ph2_a+2, ph2_b, ph2_b, ph2_a+2, 0, 1\n"                   \
+	".endif\n"                                                          \
+	".set ph2_k, ph2_k+1\n"                                             \
+	".endr\n"                                                           \
+	".endm\n"                                                           \
+	".macro PH2_PATTERNS d, odd, id\n"                                  \
+	".set ph2_x, 1\n"                                                   \
+	".rept (1<<\\d)-1\n"                                                \
+	".if ph2_x>7\n"                                                     \
+	"PH2_PATTERN 1<<(\\d-1), ph2_x, 3, \\odd\n"                         \
+	".elseif ph2_x>3\n"                                                 \
+	"PH2_PATTERN 1<<(\\d-1), ph2_x, 2, \\odd\n"                         \
+	".elseif ph2_x>1\n"                                                 \
+	"PH2_PATTERN 1<<(\\d-1), ph2_x, 1, \\odd\n"                         \
+	".else\n"                                                           \
+	"PH2_PATTERN 1<<(\\d-1), ph2_x, 0, \\odd\n"                         \
+	".endif\n"                                                          \
+	"PH2_NEXT \\id\n"                                                   \
+	".if (ph2_x==1)&&(\\odd==0)\n"                                      \
+	".Lph2n\\id:\n"                                                     \
+	".endif\n"                                                          \
+	".set ph2_x, ph2_x+1\n"                                             \
+	".endr\n"                                                           \
+	".endm\n"                                                           \
+	/* diagonal: re <- c re - sg s im, im <- c im + sg s re */          \
+	".macro PH2_DIAG d, id\n"                                           \
+	".set ph2_k, 0\n"                                                   \
+	".rept 1<<\\d\n"                                                    \
+	".set ph2_a, 16+4*ph2_k\n"                                          \
+	"PH2_SINE ph2_k\n"                                                  \
+	"PH2_HALF ph2_a, ph2_a+2, ph2_a+2, ph2_a, 1, 0\n"                   \
+	".set ph2_k, ph2_k+1\n"                                             \
+	".endr\n"                                                           \
+	"PH2_NEXT \\id\n"                                                   \
+	".endm\n"                                                           \
+	".endif\n"
+
+// The block for depth d: the term pointer, count and tile base arrive in
+// s[70:71], s80 and s[82:83], the thread index in v15.
+#define PH2_TERMS(d)                                                        \
+	PH2_TERM_MACROS                                                     \
+	"s_load_dwordx8 s[72:79], s[70:71], 0x0\n"                          \
+	"v_mov_b32 v12, 0\n"                                                \
+	"s_mov_b32 s81, 32\n"                                               \
+	"s_mov_b32 s95, 0x3ff00000\n"                                       \
+	"s_getpc_b64 s[84:85]\n"                                            \
+	".Lph2p%=:\n"                                                       \
+	"s_add_u32 s84, s84, (.Lph2h%= - .Lph2p%=)\n"                       \
+	"s_addc_u32 s85, s85, 0\n"                                          \
+	"PH2_NEXT %=\n"                                                     \
+	".Lph2h%=:\n"                                                       \
+	"PH2_PATTERNS " #d ", 0, %=\n"                                      \
+	"PH2_PATTERNS " #d ", 1, %=\n"                                      \
+	"PH2_DIAG " #d ", %=\n"                                             \
+	".Lph2x%=:\n"                                                       \
+	"s_waitcnt lgkmcnt(0)"
+
+#define PH2_TERMS_IN                                                        \
+	"{s[70:71]}"(tp), "{s[82:83]}"(base), "{v15}"(tid)
+#define PH2_TERMS_CLOBBER                                                   \
+	"v4", "v5", "v6", "v7", "v8", "v9", "v10", "v11", "v12", "v13",     \
+	"v14", "s72", "s73", "s74", "s75", "s76", "s77", "s78", "s79",      \
+	"s81", "s84", "s85", "s86", "s87", "s88", "s89", "s90", "s91",      \
+	"s92", "s93", "s94", "s95", "scc"
+
+// The count terms at tp (uniform) on the coset a of thread tid, in the tile
+// at base.  count is at least 1.
+template <int D>
+__device__ __forceinline__ void group_terms(v2d (&a)[1 << D], uint64_t tp,
+	uint32_t count, uint32_t tid, uint64_t base)
 {
-	// the split index bits (the top two) must select whole 64-lane waves
-	static_assert(TB - D >= 8 && TB - D <= 10, "2^(TB-D) threads, 256..1024");
-	const uint32_t ngroups = pass_ngroups(P);
-	const uint32_t L = pass_L(P), g = pass_g(P);
-	for (uint32_t gi = 0;; gi++) {
-		const uint32_t fcw = P.grp[gi].fcw;
-		group_terms<D>(cs, P, fcw, bu, base);
-		if (gi + 1 == ngroups)
+	if constexpr (D == 1)
+		__asm__ volatile(PH2_TERMS(1)
+			: "+{v[16:19]}"(a[0]), "+{v[20:23]}"(a[1]),
+			  "+{s80}"(count)
+			: PH2_TERMS_IN : PH2_TERMS_CLOBBER);
+	else if constexpr (D == 2)
+		__asm__ volatile(PH2_TERMS(2)
+			: "+{v[16:19]}"(a[0]), "+{v[20:23]}"(a[1]),
+			  "+{v[24:27]}"(a[2]), "+{v[28:31]}"(a[3]),
+			  "+{s80}"(count)
+			: PH2_TERMS_IN : PH2_TERMS_CLOBBER);
+	else if constexpr (D == 3)
+		__asm__ volatile(PH2_TERMS(3)
+			: "+{v[16:19]}"(a[0]), "+{v[20:23]}"(a[1]),
+			  "+{v[24:27]}"(a[2]), "+{v[28:31]}"(a[3]),
+			  "+{v[32:35]}"(a[4]), "+{v[36:39]}"(a[5]),
+			  "+{v[40:43]}"(a[6]), "+{v[44:47]}"(a[7]),
+			  "+{s80}"(count)
+			: PH2_TERMS_IN : PH2_TERMS_CLOBBER);
+	else
+		__asm__ volatile(PH2_TERMS(4)
+			: "+{v[16:19]}"(a[0]), "+{v[20:23]}"(a[1]),
+			  "+{v[24:27]}"(a[2]), "+{v[28:31]}"(a[3]),
+			  "+{v[32:35]}"(a[4]), "+{v[36:39]}"(a[5]),
+			  "+{v[40:43]}"(a[6]), "+{v[44:47]}"(a[7]),
+			  "+{v[48:51]}"(a[8]), "+{v[52:55]}"(a[9]),
+			  "+{v[56:59]}"(a[10]), "+{v[60:63]}"(a[11]),
+			  "+{v[64:67]}"(a[12]), "+{v[68:71]}"(a[13]),
+			  "+{v[72:75]}"(a[14]), "+{v[76:79]}"(a[15]),
+			  "+{s80}"(count)
+			: PH2_TERMS_IN : PH2_TERMS_CLOBBER);
+}
+
+// All ones where bit k of tid is set.
+__device__ __forceinline__ uint32_t bit_mask(uint32_t tid, int k)
+{
+	return (uint32_t)((int)(tid << (31 - k)) >> 31);
+}
+
+// Base index of tile t: its bits moved to the index bits that the tile
+// does not gather, a run of them at a time.
+__device__ __forceinline__ uint64_t tile_base(cHead H, uint64_t t)
+{
+	uint64_t base = 0;
+	const uint32_t n = H->nseg;
+#pragma unroll
+	for (int i = 0; i < kSegMax; i++) {
+		if ((i == 4 || i == 8) && n <= (uint32_t)i)
 			break;
-		const FusedGroup &N = P.grp[gi + 1];
-		const uint32_t h = (fcw >> 16) & 0xffu, xk = fcw >> 24;
-		const uint32_t half = __builtin_amdgcn_readfirstlane(
-			(tid >> xk) & 1u);
-		// the thread index is re-read per exchange: hoisted out of
-		// the loop, its bit extractions would hold 8 VGPRs throughout
-		uint32_t jt = tid;
-		__asm__ volatile("" : "+v"(jt));
-		const uint32_t bn = coset_base<TB, D>(jt, N.jposw[0],
-			N.jposw[1], N.jposw[2]);
-		uint32_t gw[4], gr[4];
-		half_offsets<TB>(P.grp[gi], h, gw);
-		half_offsets<TB>(N, h, gr);
-		uint32_t sw = half_slot<TB>(bu, h) << 4;
-		uint32_t sr = half_slot<TB>(bn, h) << 4;
-		__asm__("" : "+v"(sw), "+v"(sr));
-		for (uint32_t q = 0; q < 2; q++) {
-			// the buffer's previous readers are done (it has none before
-			// the first exchange of a workgroup's first tile)
-			if (gi > 0 || q > 0 || !fresh)
-				__syncthreads();
-			if (half == q) {
-#pragma unroll
-				for (int w = 0; w < (1 << D); w++) {
-					uint32_t c16 = 0;
-#pragma unroll
-					for (int i = 0; i < D; i++)
-						if (w >> i & 1)
-							c16 ^= gw[i];
-					*reinterpret_cast<v2d *>(
-						reinterpret_cast<char *>(buf) +
-						(sw ^ c16)) = cs[w];
-				}
-			}
-			__syncthreads();
-			if (half == q) {
-#pragma unroll
-				for (int w = 0; w < (1 << D); w++) {
-					uint32_t c16 = 0;
-#pragma unroll
-					for (int i = 0; i < D; i++)
-						if (w >> i & 1)
-							c16 ^= gr[i];
-					cs[w] = *reinterpret_cast<const v2d *>(
-						reinterpret_cast<const char *>(buf) +
-						(sr ^ c16));
-				}
-			}
-		}
-		bu = bn;
+		const uint32_t sg = H->seg[i];
+		uint64_t f;
+		__asm__("s_bfe_u64 %0, %1, %2" : "=s"(f) : "s"(t), "s"(sg) :
+			"scc");
+		base |= f << ((sg >> 8) & 63u);
 	}
-	const uint64_t abu = hbm_index(P, base, bu, L, g);
-#pragma unroll
-	for (int w = 0; w < (1 << D); w++)
-		a[abu ^ P.dcw[1][w]] = cs[w];
+	return base;
 }
 
-// One tile in the half-tile form: the first group's cosets from HBM, then
-// half_groups.
+// HBM index, within the tile at base, of the coset base of thread tid in
+// the first (side 0) or last (side 1) group.
+template <int NB>
+__device__ __forceinline__ uint64_t coset_index(cHead H, int side,
+	uint64_t base, uint32_t tid, uint32_t wave)
+{
+#pragma unroll
+	for (int k = 6; k < NB; k++)
+		base ^= H->col[side][k] & (0 - (uint64_t)(wave >> (k - 6) & 1u));
+	uint32_t lo = (uint32_t)base, hi = (uint32_t)(base >> 32);
+	// the thread index is re-read per use: kept from one to the next, the
+	// masks of its bits would hold registers throughout
+	__asm__ volatile("" : "+v"(tid));
+#pragma unroll
+	for (int k = 0; k < 6; k++) {
+		const uint32_t m = bit_mask(tid, k);
+		const uint64_t c = H->col[side][k];
+		lo ^= m & (uint32_t)c;
+		hi ^= m & (uint32_t)(c >> 32);
+	}
+	return (uint64_t)hi << 32 | lo;
+}
+
+// Coset element of step i of a walk that changes one basis vector at a
+// time, and the vector changed after it.
+constexpr int gray(int i)
+{
+	return i ^ (i >> 1);
+}
+constexpr int gray_bit(int i)
+{
+	return __builtin_ctz(i + 1);
+}
+
+// The cosets of the first group from HBM: elements with index in [E0, E1).
 template <int TB, int D>
-__device__ __forceinline__ void tile_groups_half(v2d *__restrict__ a,
-	v2d *buf, const FusedPass &P, uint64_t base, uint32_t tid)
+__device__ __forceinline__ void load_coset(const v2d *__restrict__ a,
+	cHead H, uint64_t base, uint32_t tid, uint32_t wave, v2d (&cs)[1 << D])
 {
-	const uint32_t bu = coset_base<TB, D>(tid, P.grp[0].jposw[0],
-		P.grp[0].jposw[1], P.grp[0].jposw[2]);
-	const uint64_t abu = hbm_index(P, base, bu, pass_L(P), pass_g(P));
-	v2d cs[1 << D];
+	uint64_t i = coset_index<TB - D>(H, 0, base, tid, wave);
 #pragma unroll
-	for (int w = 0; w < (1 << D); w++)
-		cs[w] = a[abu ^ P.dcw[0][w]];
-	half_groups<TB, D>(a, buf, P, base, tid, cs, bu, true);
-}
-
-// Direct HBM->LDS tile loads (gfx950 global_load_lds_dwordx4): the data
-// does not pass through registers, so all of a thread's loads of the tile
-// are in flight at once whatever the register pressure of the rotation
-// code.  Lane l of wave w in load step m fills LDS slot s = m*256 + 64w + l,
-// i.e. tile coordinate lds_slot(s) = s ^ f with f = ((s >> 4) ^ (s >> 8)) &
-// 15 (the swizzle is an involution).  f only touches coordinate bits 0..3,
-// which lie inside a row when L >= 4, so the lane reads column (s ^ f) &
-// lmask of the row of s: every 16 lanes still cover one 256-byte run.
-// Requires L >= 4.
-#define PH2_LDS(p) ((__attribute__((address_space(3))) void *)(p))
-
-// s_waitcnt with vmcnt <= N and no wait on the other counters (gfx9
-// encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
-template <uint32_t N>
-__device__ __forceinline__ void vm_wait()
-{
-	static_assert(N < 64, "vmcnt field");
-	__asm__ volatile("" ::: "memory");
-	__builtin_amdgcn_s_waitcnt((N & 15u) | ((N >> 4) << 14) | (7u << 4) |
-		(15u << 8));
-	__asm__ volatile("" ::: "memory");
-}
-
-template <int TB>
-__device__ __forceinline__ void dma_tile(const v2d *__restrict__ a,
-	v2d *__restrict__ buf,
-	const FusedPass &P, uint64_t bo, uint32_t tid)
-{
-	constexpr uint32_t PER = (1u << TB) / kBlock;
-	const uint32_t lmask = (1u << pass_L(P)) - 1;
-	const uint32_t wave0 = __builtin_amdgcn_readfirstlane(tid & ~63u);
-#pragma unroll
-	for (uint32_t m = 0; m < PER; m++) {
-		const uint32_t u = tid + m * kBlock;
-		const uint32_t f = ((tid >> 4) ^ m) & 15u;
-		__builtin_amdgcn_global_load_lds(
-			(const void *)(a + (bo ^ P.roff[m] ^ ((u ^ f) & lmask))),
-			PH2_LDS(buf + m * kBlock + wave0), 16, 0, 0);
+	for (int e = 0; e < (1 << D); e++) {
+		cs[gray(e)] = a[i];
+		if (e + 1 < (1 << D))
+			i ^= H->dc[0][gray_bit(e)];
 	}
 }
 
-template <int TB>
-__device__ __forceinline__ void store_tile(v2d *__restrict__ a,
-	const v2d *buf, const FusedPass &P, uint64_t bo, uint32_t tid)
+template <int TB, int D>
+__device__ __forceinline__ void store_coset(v2d *__restrict__ a, cHead H,
+	uint64_t base, uint32_t tid, uint32_t wave, const v2d (&cs)[1 << D])
 {
-	constexpr uint32_t PER = (1u << TB) / kBlock;
-	const uint32_t lmask = (1u << pass_L(P)) - 1;
+	uint64_t i = coset_index<TB - D>(H, 1, base, tid, wave);
 #pragma unroll
-	for (uint32_t m = 0; m < PER; m++)
-		a[bo ^ P.roff[m] ^ ((tid + m * kBlock) & lmask)] =
-			buf[lds_slot(tid + m * kBlock)];
+	for (int e = 0; e < (1 << D); e++) {
+		a[i] = cs[gray(e)];
+		if (e + 1 < (1 << D))
+			i ^= H->dc[1][gray_bit(e)];
+	}
 }
 
-// Load one tile from HBM into LDS, apply the pass, write it back.
-template <int TB, int D>
-__device__ __forceinline__ void fused_tile(v2d *__restrict__ a,
-	v2d *tile, const FusedPass &P, uint64_t t)
+// The walks keep one address: it is opaque on entry and the accesses stay
+// in order (left free, the compiler forms all of them ahead and keeps them
+// for both rounds of a half-tile exchange, 32 registers).
+template <int D>
+__device__ __forceinline__ void lds_write(char *buf, uint32_t at,
+	const uint32_t (&g)[4], const v2d (&cs)[1 << D])
 {
-	constexpr uint32_t PER = (1u << TB) / kBlock;
-	const uint32_t L = pass_L(P), lmask = (1u << L) - 1, tid = threadIdx.x;
-	const uint32_t g = pass_g(P);
-	uint64_t wt = 0;   // gathered offset of this thread's row part
-	for (uint32_t b = 0; b < g; b++)
-		if ((tid >> L) >> b & 1)
-			wt ^= P.w[b];
-	const uint64_t base = tile_base(P, t);
-	const uint64_t bo = base ^ wt;
-	const uint32_t dflags = P.dflags;
-	if (dflags & 1u) {
-		// the first group reads its cosets from HBM itself
-	} else if (L >= 4) {
-		dma_tile<TB>(a, tile, P, bo, tid);
-		vm_wait<0>();
+	__asm__ volatile("" : "+v"(at));
+#pragma unroll
+	for (int e = 0; e < (1 << D); e++) {
+		if (e && e % 4 == 0)
+			__builtin_amdgcn_sched_barrier(0);
+		*reinterpret_cast<v2d *>(buf + at) = cs[gray(e)];
+		if (e + 1 < (1 << D))
+			at ^= g[gray_bit(e)];
+	}
+}
+
+template <int D>
+__device__ __forceinline__ void lds_read(const char *buf, uint32_t at,
+	const uint32_t (&g)[4], v2d (&cs)[1 << D])
+{
+	__asm__ volatile("" : "+v"(at));
+#pragma unroll
+	for (int e = 0; e < (1 << D); e++) {
+		if (e && e % 4 == 0)
+			__builtin_amdgcn_sched_barrier(0);
+		cs[gray(e)] = *reinterpret_cast<const v2d *>(buf + at);
+		if (e + 1 < (1 << D))
+			at ^= g[gray_bit(e)];
+	}
+}
+
+// The cosets of one group, in cs, become those of the next through LDS.
+//
+// Whole tile: every thread writes, a barrier, every thread reads.  The slot
+// map is the same for all exchanges, so a thread writes only the slots it
+// read in the exchange before: no barrier ahead of the writes.
+//
+// Half tile (HALF): a buffer of half a tile and two rounds, one per half of
+// the tile (split bit xh of the host's plan; the threads of one half are
+// the waves whose coset-index bit xk is that half).  lead: the buffer has
+// earlier readers in this workgroup.
+template <int TB, int D, bool HALF>
+__device__ __forceinline__ void exchange(char *buf, cGroup G, uint32_t tid,
+	uint32_t wave, bool lead, v2d (&cs)[1 << D])
+{
+	constexpr int NB = TB - D, SH = lds_shift(TB, HALF);
+	uint32_t acc = 0;
+#pragma unroll
+	for (int k = 6; k < NB; k++)
+		acc ^= G->col[k] & (0 - (wave >> (k - 6) & 1u));
+	__asm__ volatile("" : "+v"(tid));   // as in coset_index
+#pragma unroll
+	for (int k = 0; k < 6; k++)
+		acc ^= bit_mask(tid, k) & G->col[k];
+	const uint32_t sw = (acc & 0xffffu) << SH, sr = (acc >> 16) << SH;
+	uint32_t gw[4], gr[4];
+#pragma unroll
+	for (int i = 0; i < D; i++) {
+		gw[i] = (G->g[i] & 0xffffu) << SH;
+		gr[i] = (G->g[i] >> 16) << SH;
+	}
+	if constexpr (!HALF) {
+		lds_write<D>(buf, sw, gw, cs);
+		__syncthreads();
+		lds_read<D>(buf, sr, gr, cs);
 	} else {
-		// staged through registers, a few loads in flight at a time
-#pragma unroll 4
-		for (uint32_t m = 0; m < PER; m++)
-			tile[lds_slot(tid + m * kBlock)] =
-				a[bo ^ P.roff[m] ^ ((tid + m * kBlock) & lmask)];
+		const uint32_t half = wave >> G->xk & 1u;
+		for (uint32_t q = 0; q < 2; q++) {
+			// the buffer's previous readers are done
+			if (lead || q > 0)
+				__syncthreads();
+			if (half == q)
+				lds_write<D>(buf, sw, gw, cs);
+			__syncthreads();
+			if (half == q)
+				lds_read<D>(buf, sr, gr, cs);
+		}
 	}
-	tile_groups<TB, D>(a, tile, P, base, tid, dflags);
-	if (!(dflags & 2u))
-		store_tile<TB>(a, tile, P, bo, tid);
 }
 
-// Waves per SIMD that the LDS of the whole-tile form allows (160 KiB per
-// CU, 2^TB x 16 B per 256-thread workgroup), given to the compiler as its
-// register target: left free it spends registers that cost occupancy (114
-// VGPRs at tile 11, where five workgroups fit the LDS).
-constexpr int lds_waves(int TB)
+// All micro-groups of a pass on one tile, from the first group's cosets in
+// cs (read from HBM by the caller) to the last group's, which go back to
+// HBM.  One coset per thread: 2^(TB - D) threads.  fresh: the buffer has no
+// earlier readers in this workgroup (its first tile).
+template <int TB, int D, bool HALF>
+__device__ __forceinline__ void run_groups(v2d *__restrict__ a, char *buf,
+	cHead H, uint64_t base, uint32_t tid, uint32_t wave, bool fresh,
+	v2d (&cs)[1 << D])
 {
-	// 160 KiB / (2^TB * 16 B) workgroups, one wave per SIMD each; tiles
-	// 12 and 13 fit at most two workgroups, so no target there
-	return TB > 11 ? 1 : (10240 >> TB) < 8 ? (10240 >> TB) : 8;
+	// the index bits that select the half must select whole 64-lane waves
+	static_assert(TB - D >= 8 && TB - D <= kThreadBits,
+		"2^(TB-D) threads, 256..1024");
+	cGroup G = reinterpret_cast<cGroup>(H + 1);
+	const uint64_t at = reinterpret_cast<uint64_t>(H);
+	const uint32_t n = H->ngroups;
+	// one copy of the loop body (a peeled first round would double the
+	// 28 KiB of handlers at D = 4, beyond the instruction cache)
+#pragma clang loop unroll(disable)
+	for (uint32_t gi = 0;; gi++, G++) {
+		if (G->count)
+			group_terms<D>(cs, at + G->toff, G->count, tid, base);
+		if (gi + 1 == n)
+			break;
+		// a whole tile has its slots to itself after the first
+		// exchange of a tile; the first one overwrites what the tile
+		// before it left
+		if (!HALF && gi == 0 && !fresh)
+			__syncthreads();
+		exchange<TB, D, HALF>(buf, G, tid, wave, gi > 0 || !fresh, cs);
+	}
+	store_coset<TB, D>(a, H, base, tid, wave, cs);
+}
+
+// Load one tile from HBM, apply the pass, write it back.
+template <int TB, int D, bool HALF>
+__device__ __forceinline__ void fused_tile(v2d *__restrict__ a, char *buf,
+	cHead H, uint64_t t)
+{
+	const uint32_t tid = threadIdx.x;
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const uint64_t base = tile_base(H, t);
+	v2d cs[1 << D];
+	load_coset<TB, D>(a, H, base, tid, wave, cs);
+	run_groups<TB, D, HALF>(a, buf, H, base, tid, wave, true, cs);
+}
+
+// The descriptor of the kernels that take it by value: a DevPass after the
+// first pointer argument.  Read in place: taken through the argument
+// itself, its address would make the compiler copy it to scratch.
+__device__ __forceinline__ cHead arg_head()
+{
+	static_assert(alignof(DevPass) == 16, "argument offset");
+	return reinterpret_cast<cHead>(reinterpret_cast<uint64_t>(
+		__builtin_amdgcn_kernarg_segment_ptr()) + 16);
 }
 
 // Workgroups are dealt to the 8 XCDs round-robin (workgroup w to XCD
@@ -891,84 +812,95 @@ __device__ __forceinline__ uint64_t xcd_tile(uint64_t w, uint64_t ntiles)
 // One tile per workgroup (grid = number of tiles); HBM latency is hidden
 // by the co-resident workgroups of the CU.
 template <int TB, int D>
-__global__ __launch_bounds__(kBlock)
-__attribute__((amdgpu_waves_per_eu(lds_waves(TB))))
-void k_rot_fused(
-	double2 *__restrict__ amp, const FusedPass P, uint64_t ntiles)
+__global__ __launch_bounds__((1 << TB) >> D) void k_rot_fused(
+	double2 *__restrict__ amp, const DevPass P, uint64_t ntiles)
 {
 	__shared__ v2d tile[1u << TB];
 	// 2-D grid when the tiles outnumber kMaxGrid (gridDim.x * 256 < 2^32)
 	const uint64_t w = (uint64_t)blockIdx.y * gridDim.x + blockIdx.x;
 	if (w >= ntiles)
 		return;           // whole workgroup: no barrier is left waiting
-	const uint64_t t = xcd_tile(w, ntiles);
 	// clang vector type: plain 16-byte accesses that stay in registers
-	fused_tile<TB, D>(reinterpret_cast<v2d *>(amp), tile, P, t);
+	fused_tile<TB, D, false>(reinterpret_cast<v2d *>(amp),
+		reinterpret_cast<char *>(tile), arg_head(), xcd_tile(w, ntiles));
+}
+
+// Waves per SIMD that the LDS of the half-tile form allows (160 KiB per CU,
+// 2^TB * 8 B per workgroup): five workgroups of four waves at tile 12, two
+// of eight at tile 13.  Given to the compiler as its register target.
+constexpr int half_waves(int TB)
+{
+	return TB == 12 ? 5 : 4;
 }
 
 // Half-tile form of k_rot_fused (descriptor flag 4): half the LDS, so
 // twice the workgroups per CU.  One coset per thread: 256 threads at tile
 // 12, 512 at tile 13.
 template <int TB, int D>
-__global__ __launch_bounds__((1 << TB) >> D) void k_rot_fused_half(
-	double2 *__restrict__ amp, const FusedPass P, uint64_t ntiles)
+__global__ __launch_bounds__((1 << TB) >> D)
+__attribute__((amdgpu_waves_per_eu(half_waves(TB))))
+void k_rot_fused_half(
+	double2 *__restrict__ amp, const DevPass P, uint64_t ntiles)
 {
 	__shared__ v2d buf[1u << (TB - 1)];
 	const uint64_t w = (uint64_t)blockIdx.y * gridDim.x + blockIdx.x;
 	if (w >= ntiles)
 		return;           // whole workgroup: no barrier is left waiting
-	const uint64_t t = xcd_tile(w, ntiles);
-	tile_groups_half<TB, D>(reinterpret_cast<v2d *>(amp), buf, P,
-		tile_base(P, t), threadIdx.x);
+	fused_tile<TB, D, true>(reinterpret_cast<v2d *>(amp),
+		reinterpret_cast<char *>(buf), arg_head(), xcd_tile(w, ntiles));
 }
 
-// Persistent half-tile form with the next tile's first-group cosets loaded
-// into registers while the current tile is rotated: PF of the 2^D
+// Persistent walk over tiles with the next tile's first-group cosets
+// loaded into registers while the current tile is rotated: PF of the 2^D
 // amplitudes of each coset (the rest are loaded when the tile starts), so
 // each workgroup keeps HBM reads in flight through its compute phase
 // instead of only at its start.  Workgroup b walks virtual workgroups
-// b, b + G, b + 2G, ... (G = gridDim.x, a multiple of 8, so each stays on
-// its XCD and the XCD's workgroups take neighbouring tiles, as xcd_tile
-// orders them).  Every workgroup leaves the loop once its next virtual
-// index reaches ntiles.
-template <int TB, int D, int PF>
-__global__ __launch_bounds__((1 << TB) >> D)
-void k_rot_fused_hpipe(double2 *__restrict__ amp, const FusedPass P,
-	uint64_t ntiles)
+// b, b + G, b + 2G, ... (G = gridDim.x; where it is a multiple of 8 each
+// stays on its XCD and the XCD's workgroups take neighbouring tiles, as
+// xcd_tile orders them).  Every workgroup leaves the loop once its next
+// virtual index reaches ntiles.
+template <int TB, int D, int PF, bool HALF>
+__device__ __forceinline__ void walk_tiles(v2d *__restrict__ a, char *buf,
+	cHead H, uint64_t ntiles)
 {
 	static_assert(PF > 0 && PF <= (1 << D), "prefetched amplitudes");
-	__shared__ v2d buf[1u << (TB - 1)];
-	v2d *__restrict__ a = reinterpret_cast<v2d *>(amp);
 	const uint32_t tid = threadIdx.x;
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	uint64_t v = blockIdx.x;
 	if (v >= ntiles)
 		return;           // whole workgroup: no barrier is left waiting
-	const uint32_t bu0 = coset_base<TB, D>(tid, P.grp[0].jposw[0],
-		P.grp[0].jposw[1], P.grp[0].jposw[2]);
 	// HBM offset of the first group's coset base within any tile
-	// (hbm_index is base ^ a function of bu)
-	const uint64_t off0 = hbm_index(P, 0, bu0, pass_L(P), pass_g(P));
-	uint64_t base = tile_base(P, xcd_tile(v, ntiles));
+	const uint64_t off0 = coset_index<TB - D>(H, 0, 0, tid, wave);
+	uint64_t base = tile_base(H, xcd_tile(v, ntiles));
 	v2d cs[1 << D], pre[PF];
+	uint64_t i = base ^ off0;
 #pragma unroll
-	for (int w = 0; w < PF; w++)
-		pre[w] = a[(base ^ off0) ^ P.dcw[0][w]];
+	for (int e = 0; e < PF; e++) {
+		pre[e] = a[i];
+		i ^= H->dc[0][gray_bit(e) & 3];
+	}
 	for (bool fresh = true;; fresh = false) {
+		i = base ^ off0;
 #pragma unroll
-		for (int w = 0; w < PF; w++)
-			cs[w] = pre[w];
-#pragma unroll
-		for (int w = PF; w < (1 << D); w++)
-			cs[w] = a[(base ^ off0) ^ P.dcw[0][w]];
+		for (int e = 0; e < (1 << D); e++) {
+			if (e < PF)
+				cs[gray(e)] = pre[e < PF ? e : 0];
+			else
+				cs[gray(e)] = a[i];
+			i ^= H->dc[0][gray_bit(e) & 3];
+		}
 		const uint64_t vn = v + gridDim.x;
 		const bool more = vn < ntiles;
-		const uint64_t bn = more ? tile_base(P, xcd_tile(vn, ntiles)) : 0;
+		const uint64_t bn = more ? tile_base(H, xcd_tile(vn, ntiles)) : 0;
 		if (more) {
+			i = bn ^ off0;
 #pragma unroll
-			for (int w = 0; w < PF; w++)
-				pre[w] = a[(bn ^ off0) ^ P.dcw[0][w]];
+			for (int e = 0; e < PF; e++) {
+				pre[e] = a[i];
+				i ^= H->dc[0][gray_bit(e) & 3];
+			}
 		}
-		half_groups<TB, D>(a, buf, P, base, tid, cs, bu0, fresh);
+		run_groups<TB, D, HALF>(a, buf, H, base, tid, wave, fresh, cs);
 		if (!more)
 			break;
 		v = vn;
@@ -976,9 +908,30 @@ void k_rot_fused_hpipe(double2 *__restrict__ amp, const FusedPass P,
 	}
 }
 
+template <int TB, int D, int PF>
+__global__ __launch_bounds__((1 << TB) >> D)
+void k_rot_fused_hpipe(double2 *__restrict__ amp, const DevPass P,
+	uint64_t ntiles)
+{
+	__shared__ v2d buf[1u << (TB - 1)];
+	walk_tiles<TB, D, PF, true>(reinterpret_cast<v2d *>(amp),
+		reinterpret_cast<char *>(buf), arg_head(), ntiles);
+}
+
+// The same in the whole-tile form, every amplitude prefetched.
+template <int TB, int D>
+__global__ __launch_bounds__((1 << TB) >> D) void k_rot_fused_pipe(
+	double2 *__restrict__ amp, const DevPass P, uint64_t ntiles)
+{
+	__shared__ v2d tile[1u << TB];
+	walk_tiles<TB, D, 1 << D, false>(reinterpret_cast<v2d *>(amp),
+		reinterpret_cast<char *>(tile), arg_head(), ntiles);
+}
+
 // Batched pass: pass p of many registers in one launch.  Work item i covers
 // tiles [tile0_i, tile0_{i+1}) of register i (amplitudes at amp_off_i) with
-// descriptor desc_i; a workgroup finds its item by a uniform binary search.
+// the packed descriptor at byte desc_i; a workgroup finds its item by a
+// uniform binary search.
 struct BatchItem {
 	uint64_t amp_off;
 	uint64_t tile0;
@@ -986,12 +939,12 @@ struct BatchItem {
 };
 
 // HALF: every descriptor of the launch has the half-tile form (half the
-// LDS and one coset per thread, as k_rot_fused_half).
+// LDS).
 template <int TB, int D, bool HALF = false>
-__global__ __launch_bounds__(HALF ? (1 << TB) >> D : kBlock)
-__attribute__((amdgpu_waves_per_eu(HALF ? 1 : lds_waves(TB))))
+__global__ __launch_bounds__((1 << TB) >> D)
+__attribute__((amdgpu_waves_per_eu(HALF ? half_waves(TB) : 1)))
 void k_rot_fused_batch(
-	double2 *__restrict__ amp, const FusedPass *__restrict__ descs,
+	double2 *__restrict__ amp, const uint8_t *__restrict__ descs,
 	const BatchItem *__restrict__ items, uint32_t nitems, uint64_t ntiles)
 {
 	__shared__ v2d tile[1u << (HALF ? TB - 1 : TB)];
@@ -1010,62 +963,10 @@ void k_rot_fused_batch(
 			hi = mid;
 	}
 	const BatchItem it = items[lo];
-	if constexpr (HALF) {
-		const FusedPass &P = descs[it.desc];
-		tile_groups_half<TB, D>(reinterpret_cast<v2d *>(amp) + it.amp_off,
-			tile, P, tile_base(P, t - it.tile0), threadIdx.x);
-	} else {
-		fused_tile<TB, D>(reinterpret_cast<v2d *>(amp) + it.amp_off, tile,
-			descs[it.desc], t - it.tile0);
-	}
-}
-
-// Persistent, software-pipelined pass: each workgroup walks tiles
-// blockIdx.x, +gridDim.x, ...; the next tile's HBM reads are in flight in
-// registers while the current tile is rotated in LDS, and its writes are
-// issued without waiting.  The groups always go through LDS here.
-template <int TB, int D>
-__global__ __launch_bounds__(kBlock) void k_rot_fused_pipe(
-	double2 *__restrict__ amp, const FusedPass P, uint64_t ntiles)
-{
-	constexpr uint32_t PER = (1u << TB) / kBlock;
-	__shared__ v2d tile[1u << TB];
-	v2d *__restrict__ a = reinterpret_cast<v2d *>(amp);
-	const uint32_t L = pass_L(P), lmask = (1u << L) - 1, tid = threadIdx.x;
-	const uint32_t g = pass_g(P);
-	uint64_t wt = 0;
-	for (uint32_t b = 0; b < g; b++)
-		if ((tid >> L) >> b & 1)
-			wt ^= P.w[b];
-	v2d pre[PER];
-	uint64_t t = blockIdx.x;
-	if (t < ntiles) {
-		const uint64_t bn = tile_base(P, t) ^ wt;
-#pragma unroll
-		for (uint32_t m = 0; m < PER; m++)
-			pre[m] = a[bn ^ P.roff[m] ^ ((tid + m * kBlock) & lmask)];
-	}
-	for (; t < ntiles; t += gridDim.x) {
-		const uint64_t base = tile_base(P, t);
-		__syncthreads();          // previous tile fully written out
-#pragma unroll
-		for (uint32_t m = 0; m < PER; m++)
-			tile[lds_slot(tid + m * kBlock)] = pre[m];
-		const uint64_t tn = t + gridDim.x;
-		if (tn < ntiles) {
-			const uint64_t bn = tile_base(P, tn) ^ wt;
-#pragma unroll
-			for (uint32_t m = 0; m < PER; m++)
-				pre[m] = a[bn ^ P.roff[m] ^
-					((tid + m * kBlock) & lmask)];
-		}
-		tile_groups<TB, D>(a, tile, P, base, tid, 0u);
-		const uint64_t bo = base ^ wt;
-#pragma unroll
-		for (uint32_t m = 0; m < PER; m++)
-			a[bo ^ P.roff[m] ^ ((tid + m * kBlock) & lmask)] =
-				tile[lds_slot(tid + m * kBlock)];
-	}
+	fused_tile<TB, D, HALF>(reinterpret_cast<v2d *>(amp) + it.amp_off,
+		reinterpret_cast<char *>(tile),
+		reinterpret_cast<cHead>(reinterpret_cast<uint64_t>(descs) +
+			it.desc), t - it.tile0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1522,11 +1423,19 @@ void pipe_init()
 	g_pipe_init = true;
 }
 
+size_t pack_pass(const FusedPass &P, uint32_t tb, bool half, uint8_t *out);
+
 template <int TB>
 int launch_fused(double2 *a, uint32_t nqb, const FusedPass &P,
 	uint64_t xunion, uint64_t zunion)
 {
+	constexpr int D = group_depth(TB);
+	const dim3 blk((1u << TB) >> D);
 	pipe_init();
+	const bool pipe = g_pipe_mask >> TB & 1;
+	DevPass dp;
+	memset(&dp, 0, sizeof dp);
+	pack_pass(P, TB, !pipe && (P.dflags & 4u) != 0, dp.b);
 	const uint64_t ntiles = UINT64_C(1) << (nqb - TB);
 	hipEvent_t stop;
 	ph2hip_launch_rec meta{};
@@ -1542,49 +1451,40 @@ int launch_fused(double2 *a, uint32_t nqb, const FusedPass &P,
 	meta.zunion = zunion;
 	if (prof_begin(2, P.nterms, UINT64_C(1) << nqb, &stop, &meta))
 		return -1;
-	if (g_pipe_mask >> TB & 1) {
-		const uint64_t grid = ntiles < g_persist_wgs ? ntiles
+	const uint64_t gx = ntiles < kMaxGrid ? ntiles : kMaxGrid;
+	const dim3 grid((uint32_t)gx, (uint32_t)((ntiles + gx - 1) / gx));
+	if (pipe) {
+		const uint64_t pg = ntiles < g_persist_wgs ? ntiles
 			: g_persist_wgs;
-		hipLaunchKernelGGL((k_rot_fused_pipe<TB, group_depth(TB)>),
-			dim3((uint32_t)grid), dim3(kBlock), 0, g_stream, a, P,
-			ntiles);
-	} else {
-		const uint64_t gx = ntiles < kMaxGrid ? ntiles : kMaxGrid;
-		const uint64_t gy = (ntiles + gx - 1) / gx;
-		if constexpr ((kHalfTiles >> TB & 1) != 0) {
-			const uint32_t pf = g_hpipe_pf[TB];
-			uint64_t pg = (uint64_t)g_hpipe_wpc[TB] * g_ncu;
-			pg = pg < ntiles ? pg : ntiles;
-			if (pg >= 8)
-				pg &= ~UINT64_C(7);   // whole rounds over the XCDs
-			if ((P.dflags & 4u) && pf && pg) {
-				constexpr int D = group_depth(TB);
-				const dim3 blk((1u << TB) >> D);
-				if (pf == 16)
-					hipLaunchKernelGGL((k_rot_fused_hpipe<TB, D, 16>),
-						dim3((uint32_t)pg), blk, 0, g_stream, a, P,
-						ntiles);
-				else
-					hipLaunchKernelGGL((k_rot_fused_hpipe<TB, D, 8>),
-						dim3((uint32_t)pg), blk, 0, g_stream, a, P,
-						ntiles);
-				HIPCHK(hipGetLastError());
-				return prof_end(stop);
-			}
-			if (P.dflags & 4u) {
-				hipLaunchKernelGGL(
-					(k_rot_fused_half<TB, group_depth(TB)>),
-					dim3((uint32_t)gx, (uint32_t)gy),
-					dim3((1u << TB) >> group_depth(TB)), 0,
-					g_stream, a, P, ntiles);
-				HIPCHK(hipGetLastError());
-				return prof_end(stop);
-			}
-		}
-		hipLaunchKernelGGL((k_rot_fused<TB, group_depth(TB)>),
-			dim3((uint32_t)gx, (uint32_t)gy), dim3(kBlock), 0, g_stream,
-			a, P, ntiles);
+		hipLaunchKernelGGL((k_rot_fused_pipe<TB, D>),
+			dim3((uint32_t)pg), blk, 0, g_stream, a, dp, ntiles);
+		HIPCHK(hipGetLastError());
+		return prof_end(stop);
 	}
+	if constexpr ((kHalfTiles >> TB & 1) != 0) {
+		const uint32_t pf = g_hpipe_pf[TB];
+		uint64_t pg = (uint64_t)g_hpipe_wpc[TB] * g_ncu;
+		pg = pg < ntiles ? pg : ntiles;
+		if (pg >= 8)
+			pg &= ~UINT64_C(7);   // whole rounds over the XCDs
+		if (P.dflags & 4u) {
+			if (pf == 16 && pg)
+				hipLaunchKernelGGL((k_rot_fused_hpipe<TB, D, 16>),
+					dim3((uint32_t)pg), blk, 0, g_stream, a,
+					dp, ntiles);
+			else if (pf && pg)
+				hipLaunchKernelGGL((k_rot_fused_hpipe<TB, D, 8>),
+					dim3((uint32_t)pg), blk, 0, g_stream, a,
+					dp, ntiles);
+			else
+				hipLaunchKernelGGL((k_rot_fused_half<TB, D>), grid,
+					blk, 0, g_stream, a, dp, ntiles);
+			HIPCHK(hipGetLastError());
+			return prof_end(stop);
+		}
+	}
+	hipLaunchKernelGGL((k_rot_fused<TB, D>), grid, blk, 0, g_stream, a, dp,
+		ntiles);
 	HIPCHK(hipGetLastError());
 	return prof_end(stop);
 }
@@ -1694,15 +1594,6 @@ int build_pass_mode(FusedPass &P, const struct ph2hip_rot *r, size_t len,
 	for (uint32_t b = 0; b < g; b++) {
 		P.w[b] = w[b];
 		P.piv[b] = (uint8_t)top_bit(w[b]);
-	}
-	// row part of element tid + m*kBlock that is uniform in m
-	for (uint32_t m = 0; m < (1u << tb) / kBlock; m++) {
-		const uint32_t rm = (m * kBlock) >> L;
-		uint64_t wm = 0;
-		for (uint32_t b = 0; b < g; b++)
-			if (rm >> b & 1)
-				wm ^= w[b];
-		P.roff[m] = wm;
 	}
 	const uint64_t lm = (UINT64_C(1) << L) - 1;
 	uint32_t xt[PH2HIP_PASS_MAX];
@@ -1936,23 +1827,114 @@ int build_pass_mode(FusedPass &P, const struct ph2hip_rot *r, size_t len,
 			if (!half && (G.jpos[0] != 0 || G.jpos[1] != 1 ||
 			    G.jpos[2] != 2 || G.jpos[3] != 3))
 				continue;
-			for (uint32_t e = 0; e < (1u << D); e++) {
-				uint32_t cw = 0;
-				for (uint32_t i = 0; i < D; i++)
-					if (e >> i & 1)
-						cw ^= G.u[i];
-				uint64_t off = cw & lm;
-				for (uint32_t b = 0; b < g; b++)
-					if ((cw >> (L + b)) & 1)
-						off ^= w[b];
-				P.dcw[side][e] = off;
-			}
 			P.dflags |= 1u << side;
 		}
 	}
 	if (half)
 		P.dflags |= 4u;
 	return 0;
+}
+
+// The kernels' descriptor of a planned pass in the half- or the whole-tile
+// form, written to out (kDevMax bytes of room); returns its size.  A first
+// or last group that does not move its cosets straight between HBM and
+// registers (dflags) gets a group without terms in front of or behind it,
+// whose cosets are the rows of the tile: it moves whole runs, and the
+// exchange with it takes them through LDS.
+size_t pack_pass(const FusedPass &P, uint32_t tb, bool half, uint8_t *out)
+{
+	const uint32_t D = (uint32_t)group_depth((int)tb), nb = tb - D;
+	const uint32_t sh = (uint32_t)lds_shift((int)tb, half);
+	FusedGroup rows;
+	memset(&rows, 0, sizeof rows);
+	for (uint32_t i = 0; i < D; i++)
+		rows.u[i] = (uint16_t)(1u << (nb + i));
+	for (uint32_t k = 0; k < nb; k++)
+		rows.jpos[k] = (uint8_t)k;
+	const FusedGroup *g[PH2HIP_PASS_MAX + 2];
+	uint32_t n = 0;
+	if (!(P.dflags & 1u))
+		g[n++] = &rows;
+	for (uint32_t i = 0; i < P.ngroups; i++)
+		g[n++] = &P.grp[i];
+	if (!(P.dflags & 2u))
+		g[n++] = &rows;
+
+	DevHead H;
+	memset(&H, 0, sizeof H);
+	H.ngroups = n;
+	uint64_t taken = (UINT64_C(1) << P.L) - 1;
+	for (uint32_t b = 0; b < P.g; b++)
+		taken |= UINT64_C(1) << P.piv[b];
+	for (uint32_t src = 0, bit = 0; bit < 48;) {
+		if (taken >> bit & 1) {
+			bit++;
+			continue;
+		}
+		uint32_t e = bit;
+		while (e < 48 && !(taken >> e & 1))
+			e++;
+		H.seg[H.nseg++] = src | bit << 8 | (e - bit) << 16;
+		src += e - bit;
+		bit = e;
+	}
+	const auto hbm = [&](uint32_t v) {
+		uint64_t i = v & ((1u << P.L) - 1);
+		for (uint32_t b = 0; b < P.g; b++)
+			if (v >> (P.L + b) & 1)
+				i ^= P.w[b];
+		return i;
+	};
+	for (int side = 0; side < 2; side++) {
+		const FusedGroup &G = *g[side ? n - 1 : 0];
+		for (uint32_t k = 0; k < nb; k++)
+			H.col[side][k] = hbm(1u << G.jpos[k]);
+		for (uint32_t i = 0; i < D; i++)
+			H.dc[side][i] = hbm(G.u[i]);
+	}
+	memcpy(out, &H, sizeof H);
+
+	size_t at = sizeof H, to = sizeof H + n * sizeof(DevGroup);
+	for (uint32_t q = 0; q < n; q++) {
+		const FusedGroup &G = *g[q];
+		DevGroup W;
+		memset(&W, 0, sizeof W);
+		W.count = G.count;
+		W.toff = (uint32_t)to;
+		if (q + 1 < n) {
+			const FusedGroup &N = *g[q + 1];
+			const auto slot = [&](uint32_t v) {
+				return (half ? half_slot(tb, v, G.xh) :
+					lds_slot(v)) << 4 >> sh;
+			};
+			if (half)
+				W.xk = G.xk - 6u;
+			for (uint32_t k = 0; k < nb; k++)
+				W.col[k] = slot(1u << G.jpos[k]) |
+					slot(1u << N.jpos[k]) << 16;
+			for (uint32_t i = 0; i < D; i++)
+				W.g[i] = slot(G.u[i]) | slot(N.u[i]) << 16;
+		}
+		memcpy(out + at, &W, sizeof W);
+		at += sizeof W;
+		for (uint32_t k = G.first; k < (uint32_t)G.first + G.count; k++) {
+			const FusedTerm &F = P.t[k];
+			DevTerm T;
+			T.z = F.z;
+			T.c = F.c;
+			T.s = F.xtp && (F.y & 2) ? -F.s : F.s;
+			T.zt = F.zt & 0xffff0000u;
+			for (uint32_t b = 0; b < nb; b++)
+				T.zt |= (F.zt >> G.jpos[b] & 1u) << b;
+			const uint32_t np = (1u << D) - 1;
+			T.code = F.xtp == 0 ? 2 * np :
+				(F.y & 1 ? np : 0) + F.xtp - 1;
+			memcpy(out + to, &T, sizeof T);
+			to += sizeof T;
+		}
+	}
+	memset(out + to, 0, sizeof(DevTerm));   // fetched, never run
+	return (to + sizeof(DevTerm) + 15) & ~size_t{15};
 }
 
 // Bit tb set: passes of tile width tb take the half-tile form where they
@@ -2007,25 +1989,26 @@ void *g_bdesc = nullptr, *g_bitem = nullptr;
 size_t g_bdesc_cap = 0, g_bitem_cap = 0;
 
 template <int TB>
-int launch_batch(double2 *amp, const FusedPass *descs, const BatchItem *items,
+int launch_batch(double2 *amp, const uint8_t *descs, const BatchItem *items,
 	uint32_t nitems, uint64_t ntiles, bool half)
 {
+	constexpr int D = group_depth(TB);
 	const uint64_t gx = ntiles < kMaxGrid ? ntiles : kMaxGrid;
 	const uint64_t gy = (ntiles + gx - 1) / gx;
 	if constexpr ((kBatchHalfTiles >> TB & 1) != 0) {
 		if (half) {
 			hipLaunchKernelGGL(
-				(k_rot_fused_batch<TB, group_depth(TB), true>),
+				(k_rot_fused_batch<TB, D, true>),
 				dim3((uint32_t)gx, (uint32_t)gy),
-				dim3((1u << TB) >> group_depth(TB)), 0, g_stream,
+				dim3((1u << TB) >> D), 0, g_stream,
 				amp, descs, items, nitems, ntiles);
 			HIPCHK(hipGetLastError());
 			return 0;
 		}
 	}
-	hipLaunchKernelGGL((k_rot_fused_batch<TB, group_depth(TB)>),
-		dim3((uint32_t)gx, (uint32_t)gy), dim3(kBlock), 0, g_stream, amp,
-		descs, items, nitems, ntiles);
+	hipLaunchKernelGGL((k_rot_fused_batch<TB, D>),
+		dim3((uint32_t)gx, (uint32_t)gy), dim3((1u << TB) >> D), 0,
+		g_stream, amp, descs, items, nitems, ntiles);
 	HIPCHK(hipGetLastError());
 	return 0;
 }
@@ -2135,7 +2118,8 @@ ReplaySlot *replay_slot(void *amp, uint32_t nqb, const struct ph2hip_rot *rot,
 } // namespace
 
 struct ph2hip_batch_plan {
-	FusedPass *desc;      // descriptors, job-major
+	uint8_t *desc;        // packed descriptors, job-major
+	size_t desc_bytes, desc_cap;
 	BatchItem *items;     // work items, launch-major
 	size_t ndesc, maxp;
 	size_t nlaunch;       // one or two per pass index (half-tile, whole)
@@ -2186,7 +2170,7 @@ void rg_clear()
 // Arguments of one batched node (k_rot_fused_batch's parameters).
 struct BatchArgs {
 	double2 *amp;
-	const FusedPass *descs;
+	const uint8_t *descs;
 	const BatchItem *items;
 	uint32_t nitems;
 	uint64_t ntiles;
@@ -2207,16 +2191,13 @@ void batch_node(hipKernelNodeParams &kp, BatchArgs &ba, bool half)
 	const uint64_t gy = nt == 0 ? 1 : (nt + gx - 1) / gx;
 	kp = hipKernelNodeParams{};
 	if constexpr ((kBatchHalfTiles >> TB & 1) != 0) {
-		if (half) {
+		if (half)
 			kp.func = reinterpret_cast<void *>(
 				&k_rot_fused_batch<TB, D, true>);
-			kp.blockDim = dim3((1u << TB) >> D);
-		}
 	}
-	if (!kp.func) {
+	if (!kp.func)
 		kp.func = reinterpret_cast<void *>(&k_rot_fused_batch<TB, D>);
-		kp.blockDim = dim3(kBlock);
-	}
+	kp.blockDim = dim3((1u << TB) >> D);
 	kp.gridDim = dim3((uint32_t)gx, (uint32_t)gy);
 	kp.sharedMemBytes = 0;
 	kp.kernelParams = ba.ptr;
@@ -2288,7 +2269,7 @@ int rg_launch(const struct ph2hip_batch_plan *pl, double2 *amp)
 	}
 	int rc = 0;
 	for (size_t i = 0; i < nn && !rc; i++) {
-		BatchArgs ba{ amp, static_cast<const FusedPass *>(g_bdesc),
+		BatchArgs ba{ amp, static_cast<const uint8_t *>(g_bdesc),
 			static_cast<const BatchItem *>(g_bitem), 0, 0, {} };
 		if (lof[i] >= 0) {
 			const size_t l = (size_t)lof[i];
@@ -3069,6 +3050,20 @@ void ph2hip_batch_plan_free(struct ph2hip_batch_plan *pl)
 	free(pl);
 }
 
+// Room for more bytes of packed descriptors.
+static int desc_reserve(struct ph2hip_batch_plan *pl, size_t more)
+{
+	if (pl->desc_bytes + more <= pl->desc_cap)
+		return 0;
+	const size_t cap = 2 * pl->desc_cap + 16 * more;
+	uint8_t *b = (uint8_t *)realloc(pl->desc, cap);
+	if (!b)
+		return fail("rotate_batched: out of host memory");
+	pl->desc = b;
+	pl->desc_cap = cap;
+	return 0;
+}
+
 int ph2hip_batch_plan_build(const struct ph2hip_batch_job *jobs, size_t njobs,
 	uint32_t tile_bits, uint32_t low_bits, uint64_t namp_total,
 	struct ph2hip_batch_plan **out)
@@ -3110,34 +3105,44 @@ int ph2hip_batch_plan_build(const struct ph2hip_batch_job *jobs, size_t njobs,
 		*out = pl;
 		return 0;
 	}
-	pl->desc = (FusedPass *)malloc(sizeof(FusedPass) * ndesc);
 	pl->items = (BatchItem *)malloc(sizeof(BatchItem) * ndesc);
 	pl->lstart = (size_t *)calloc(2 * maxp + 1, sizeof(size_t));
 	pl->ltiles = (uint64_t *)calloc(2 * maxp, sizeof(uint64_t));
 	pl->lhalf = (uint8_t *)calloc(2 * maxp, 1);
 	pl->lpass = (uint32_t *)calloc(2 * maxp, sizeof(uint32_t));
 	size_t *first = (size_t *)malloc(sizeof(size_t) * (njobs ? njobs : 1));
+	// per descriptor: its byte offset, times 2, plus 1 in the half-tile
+	// form
+	uint64_t *at = (uint64_t *)malloc(sizeof(uint64_t) * ndesc);
 	int rc = 0;
-	if (!pl->desc || !pl->items || !pl->lstart || !pl->ltiles ||
-	    !pl->lhalf || !pl->lpass || !first) {
+	if (!pl->items || !pl->lstart || !pl->ltiles || !pl->lhalf ||
+	    !pl->lpass || !first || !at) {
 		rc = fail("rotate_batched: out of host memory");
 	} else {
 		// descriptors, job-major
 		size_t d = 0;
+		FusedPass P;
 		for (size_t j = 0; j < njobs && !rc; j++) {
 			first[j] = d;
 			size_t k0 = 0;
 			for (size_t p = 0; p < jobs[j].npass && !rc; p++) {
 				rc = 1;
 				if (((half_mask() & kBatchHalfTiles) >> tile_bits) & 1)
-					rc = build_pass_mode(pl->desc[d],
-						jobs[j].rot + k0, jobs[j].pass_len[p],
-						tile_bits, low_bits, k0, true);
+					rc = build_pass_mode(P, jobs[j].rot + k0,
+						jobs[j].pass_len[p], tile_bits,
+						low_bits, k0, true);
 				if (rc > 0)
-					rc = build_pass_mode(pl->desc[d],
-						jobs[j].rot + k0, jobs[j].pass_len[p],
-						tile_bits, low_bits, k0, false);
-				d++;
+					rc = build_pass_mode(P, jobs[j].rot + k0,
+						jobs[j].pass_len[p], tile_bits,
+						low_bits, k0, false);
+				if (!rc && desc_reserve(pl, kDevMax))
+					rc = -1;
+				if (rc)
+					break;
+				const bool hf = (P.dflags & 4u) != 0;
+				at[d++] = 2 * pl->desc_bytes + hf;
+				pl->desc_bytes += pack_pass(P, tile_bits, hf,
+					pl->desc + pl->desc_bytes);
 				k0 += jobs[j].pass_len[p];
 			}
 		}
@@ -3154,12 +3159,12 @@ int ph2hip_batch_plan_build(const struct ph2hip_batch_job *jobs, size_t njobs,
 				for (size_t j = 0; j < njobs; j++) {
 					if (jobs[j].npass <= p)
 						continue;
-					const size_t dj = first[j] + p;
-					if (((pl->desc[dj].dflags & 4u) != 0) != (h != 0))
+					const uint64_t dj = at[first[j] + p];
+					if ((int)(dj & 1) != h)
 						continue;
 					pl->items[it].amp_off = jobs[j].amp_off;
 					pl->items[it].tile0 = t0;
-					pl->items[it].desc = dj;
+					pl->items[it].desc = dj >> 1;
 					t0 += UINT64_C(1) << (jobs[j].nqb - tile_bits);
 					it++;
 				}
@@ -3176,6 +3181,7 @@ int ph2hip_batch_plan_build(const struct ph2hip_batch_job *jobs, size_t njobs,
 		pl->nlaunch = l;
 	}
 	free(first);
+	free(at);
 	if (rc) {
 		ph2hip_batch_plan_free(pl);
 		return -1;
@@ -3197,10 +3203,10 @@ int ph2hip_batch_plan_launch(void *amp, struct ph2hip_batch_plan *pl,
 	const uint32_t tile_bits = pl->tile_bits;
 	// The upload follows the work already queued on the stream, so the
 	// launches of an earlier plan have read the buffers before they change.
-	if (dev_reserve(&g_bdesc, &g_bdesc_cap, sizeof(FusedPass) * ndesc) ||
+	if (dev_reserve(&g_bdesc, &g_bdesc_cap, pl->desc_bytes) ||
 	    dev_reserve(&g_bitem, &g_bitem_cap, sizeof(BatchItem) * ndesc))
 		return -1;
-	if (hipMemcpyAsync(g_bdesc, pl->desc, sizeof(FusedPass) * ndesc,
+	if (hipMemcpyAsync(g_bdesc, pl->desc, pl->desc_bytes,
 		    hipMemcpyHostToDevice, g_stream) != hipSuccess ||
 	    hipMemcpyAsync(g_bitem, pl->items, sizeof(BatchItem) * ndesc,
 		    hipMemcpyHostToDevice, g_stream) != hipSuccess)
@@ -3218,7 +3224,7 @@ int ph2hip_batch_plan_launch(void *amp, struct ph2hip_batch_plan *pl,
 	for (size_t l = 0; l < nlaunch && !rc; l++) {
 		const uint32_t ni = (uint32_t)(pl->lstart[l + 1] - pl->lstart[l]);
 		const BatchItem *it = (const BatchItem *)g_bitem + pl->lstart[l];
-		const FusedPass *dd = (const FusedPass *)g_bdesc;
+		const uint8_t *dd = (const uint8_t *)g_bdesc;
 		const bool hf = pl->lhalf[l] != 0;
 		hipEvent_t stop = nullptr;
 		ph2hip_launch_rec meta{};
