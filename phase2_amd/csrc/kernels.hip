@@ -278,31 +278,38 @@ struct FusedPass {
 	FusedTerm t[PH2HIP_PASS_MAX];
 };
 
-// Packed descriptor: a head, the groups, the terms, without gaps.  Read
-// through scalar loads only.
+// Packed descriptor: a head, the terms, one exchange record per group,
+// without gaps.  Read through scalar loads only.
 constexpr int kThreadBits = 10;   // thread-index bits a column set covers
 constexpr int kSegMax = PH2HIP_TILE_MAX + 1;
 
+// What a tile needs to start is in the first three 64-byte lines
+// (load_head).
 struct DevHead {
 	uint32_t ngroups;
+	uint32_t xoff;       // byte offset of the exchange records
+	uint32_t count;      // terms of the first group
 	uint32_t nseg;
 	// tile index -> base index: bits [src, src + width) move to dst;
 	// src | dst << 8 | width << 16 (width 0: unused)
 	uint32_t seg[kSegMax];
-	// HBM index columns of the first and last group's cosets, and of
-	// their basis vectors
-	uint64_t col[2][kThreadBits];
-	uint64_t dc[2][4];
+	// HBM index columns of the first group's cosets and of their basis
+	// vectors, low and high words
+	uint32_t col0[kThreadBits][2];
+	uint32_t dc0[4][2];
+	uint32_t pad[2];
+	// the same of the last group
+	uint64_t col1[kThreadBits];
+	uint64_t dc1[4];
 };
 
-struct DevGroup {
-	uint32_t count;      // terms
-	uint32_t xk;         // half-tile exchange: wave bit of the half
-	uint32_t toff;       // byte offset of the first term
-	// LDS byte offsets (>> kShift) of the exchange to the next group:
-	// where this group's cosets are written (low half) and the next
-	// group's are read (high half), per thread-index bit and per basis
-	// vector
+// Group q's record: the exchange to group q + 1.
+struct DevExchange {
+	uint32_t count;      // terms of group q + 1
+	uint32_t xk;         // half-tile form: wave bit of the half
+	// LDS byte offsets (>> lds_shift) of where group q's cosets are
+	// written (low half) and group q + 1's are read (high half), per
+	// thread-index bit and per basis vector
 	uint32_t col[kThreadBits];
 	uint32_t g[4];
 };
@@ -315,14 +322,19 @@ struct DevTerm {
 	uint32_t code;       // handler: even patterns, odd patterns, diagonal
 };
 
+static_assert(offsetof(DevHead, col1) == 192, "load_head");
+static_assert(sizeof(DevExchange) == 64, "one scalar load");
 static_assert(sizeof(DevTerm) == 32, "term stride of the kernels");
 
 // Two more groups than the pass has: the ones that only move the tile
 // between HBM and LDS (pack_pass).  One term more: the kernels fetch the
-// term after the one they run.
+// term after the one they run.  A kernel touches the first kWarm bytes of
+// every descriptor.
+constexpr size_t kWarm = 0x6c0;
 constexpr size_t kDevMax = sizeof(DevHead) +
-	(PH2HIP_PASS_MAX + 2) * sizeof(DevGroup) +
+	(PH2HIP_PASS_MAX + 2) * sizeof(DevExchange) +
 	(PH2HIP_PASS_MAX + 1) * sizeof(DevTerm);
+static_assert(kDevMax >= kWarm, "touched bytes");
 
 struct alignas(16) DevPass {
 	uint8_t b[(kDevMax + 15) & ~size_t{15}];
@@ -330,9 +342,14 @@ struct alignas(16) DevPass {
 
 #define PH2_CONST __attribute__((address_space(4)))
 typedef const PH2_CONST DevHead *cHead;
-typedef const PH2_CONST DevGroup *cGroup;
+// LDS by its own address space: with generic pointers the compiler merged
+// the first group's HBM loads and the exchange's LDS reads into one flat
+// load on a pointer of either kind.
+typedef __attribute__((address_space(3))) char *lds_t;
 
 typedef double v2d __attribute__((ext_vector_type(2)));
+typedef uint32_t v8u __attribute__((ext_vector_type(8)));
+typedef uint32_t v16u __attribute__((ext_vector_type(16)));
 
 // LDS slot of tile coordinate v: bits >= 4 folded into bits 0..3.  The map
 // is GF(2)-linear, so slot(a ^ b) = slot(a) ^ slot(b).
@@ -386,7 +403,9 @@ constexpr int lds_shift(int tb, bool half)
 // before and 526, 1846 and 10536 us after; 1163 and 1133 ms at 31 qubits,
 // where HBM weighs more.
 //
-// Term k + 1 is fetched (one scalar load) while term k runs.  Dispatch: the
+// Term k + 1 is fetched (one scalar load) while term k runs, and the
+// exchange record of the group with its first term; the fetched term that
+// ends a group's block is the next group's first.  Dispatch: the
 // term's code picks its handler, one per flip pattern XT in 1 .. 2^D - 1,
 // first for even y, then for odd, then the diagonal one; the handlers of
 // the patterns have one size, so the address is a product.  A handler ends
@@ -405,9 +424,9 @@ constexpr int lds_shift(int tb, bool half)
 // costs the 8 products and 4 sums of its definition, and nothing for signs.
 //
 // Registers: v[4:11] temporaries, v[12:13] sg, v14 scratch; s[72:79] the
-// next term, s80 terms left, s81 its offset, s[84:85] first handler,
-// s[86:87] scratch, s[88:89] c, s[90:91] the signed s of the pair, s92/s93
-// high words of s and -s, s94 sign masks.
+// next term, s80 terms left, s81 offset of the term after the next,
+// s[84:85] first handler, s[86:87] scratch, s[88:89] c, s[90:91] the
+// signed s of the pair, s92/s93 high words of s and -s, s94 sign masks.
 #define PH2_TERM_MACROS                                                     \
 	".ifndef ph2_macros\n"                                              \
 	".set ph2_macros, 1\n"                                              \
@@ -507,13 +526,12 @@ constexpr int lds_shift(int tb, bool half)
 	".endm\n"                                                           \
 	".endif\n"
 
-// The block for depth d: the term pointer, count and tile base arrive in
-// s[70:71], s80 and s[82:83], the thread index in v15.
+// The block for depth d: descriptor address, record address and tile base
+// arrive in s[70:71], s[68:69] and s[82:83], the thread index in v15.
 #define PH2_TERMS(d)                                                        \
 	PH2_TERM_MACROS                                                     \
-	"s_load_dwordx8 s[72:79], s[70:71], 0x0\n"                          \
+	"s_load_dwordx16 s[40:55], s[68:69], 0x0\n"                         \
 	"v_mov_b32 v12, 0\n"                                                \
-	"s_mov_b32 s81, 32\n"                                               \
 	"s_mov_b32 s95, 0x3ff00000\n"                                       \
 	"s_getpc_b64 s[84:85]\n"                                            \
 	".Lph2p%=:\n"                                                       \
@@ -527,30 +545,41 @@ constexpr int lds_shift(int tb, bool half)
 	".Lph2x%=:\n"                                                       \
 	"s_waitcnt lgkmcnt(0)"
 
+#define PH2_TERMS_INOUT                                                     \
+	"+{s[72:79]}"(C.term), "+{s80}"(C.count), "+{s81}"(C.off),          \
+	"=&{s[40:55]}"(x)
 #define PH2_TERMS_IN                                                        \
-	"{s[70:71]}"(tp), "{s[82:83]}"(base), "{v15}"(tid)
+	"{s[70:71]}"(C.desc), "{s[68:69]}"(C.rec), "{s[82:83]}"(base),      \
+	"{v15}"(tid)
 #define PH2_TERMS_CLOBBER                                                   \
 	"v4", "v5", "v6", "v7", "v8", "v9", "v10", "v11", "v12", "v13",     \
-	"v14", "s72", "s73", "s74", "s75", "s76", "s77", "s78", "s79",      \
-	"s81", "s84", "s85", "s86", "s87", "s88", "s89", "s90", "s91",      \
+	"v14", "s84", "s85", "s86", "s87", "s88", "s89", "s90", "s91",      \
 	"s92", "s93", "s94", "s95", "scc"
 
-// The count terms at tp (uniform) on the coset a of thread tid, in the tile
-// at base.  count is at least 1.
+// Where a tile is in its descriptor: address, current group's record, the
+// fetched term, terms left in the group, byte offset of the next fetch.
+struct Cursor {
+	uint64_t desc, rec;
+	v8u term;
+	uint32_t count, off;
+};
+
+// The terms of the current group on the coset a of thread tid, in the tile
+// at base; x receives the group's exchange record.
 template <int D>
-__device__ __forceinline__ void group_terms(v2d (&a)[1 << D], uint64_t tp,
-	uint32_t count, uint32_t tid, uint64_t base)
+__device__ __forceinline__ void group_terms(v2d (&a)[1 << D], Cursor &C,
+	uint32_t tid, uint64_t base, v16u &x)
 {
 	if constexpr (D == 1)
 		__asm__ volatile(PH2_TERMS(1)
 			: "+{v[16:19]}"(a[0]), "+{v[20:23]}"(a[1]),
-			  "+{s80}"(count)
+			  PH2_TERMS_INOUT
 			: PH2_TERMS_IN : PH2_TERMS_CLOBBER);
 	else if constexpr (D == 2)
 		__asm__ volatile(PH2_TERMS(2)
 			: "+{v[16:19]}"(a[0]), "+{v[20:23]}"(a[1]),
 			  "+{v[24:27]}"(a[2]), "+{v[28:31]}"(a[3]),
-			  "+{s80}"(count)
+			  PH2_TERMS_INOUT
 			: PH2_TERMS_IN : PH2_TERMS_CLOBBER);
 	else if constexpr (D == 3)
 		__asm__ volatile(PH2_TERMS(3)
@@ -558,7 +587,7 @@ __device__ __forceinline__ void group_terms(v2d (&a)[1 << D], uint64_t tp,
 			  "+{v[24:27]}"(a[2]), "+{v[28:31]}"(a[3]),
 			  "+{v[32:35]}"(a[4]), "+{v[36:39]}"(a[5]),
 			  "+{v[40:43]}"(a[6]), "+{v[44:47]}"(a[7]),
-			  "+{s80}"(count)
+			  PH2_TERMS_INOUT
 			: PH2_TERMS_IN : PH2_TERMS_CLOBBER);
 	else
 		__asm__ volatile(PH2_TERMS(4)
@@ -570,7 +599,7 @@ __device__ __forceinline__ void group_terms(v2d (&a)[1 << D], uint64_t tp,
 			  "+{v[56:59]}"(a[10]), "+{v[60:63]}"(a[11]),
 			  "+{v[64:67]}"(a[12]), "+{v[68:71]}"(a[13]),
 			  "+{v[72:75]}"(a[14]), "+{v[76:79]}"(a[15]),
-			  "+{s80}"(count)
+			  PH2_TERMS_INOUT
 			: PH2_TERMS_IN : PH2_TERMS_CLOBBER);
 }
 
@@ -580,17 +609,79 @@ __device__ __forceinline__ uint32_t bit_mask(uint32_t tid, int k)
 	return (uint32_t)((int)(tid << (31 - k)) >> 31);
 }
 
+// acc ^ (m & c), one instruction.
+__device__ __forceinline__ uint32_t xor_masked(uint32_t acc, uint32_t m,
+	uint32_t c)
+{
+	return __builtin_amdgcn_bitop3_b32(acc, m, c, 0x78);
+}
+
+// The start of a descriptor in registers: its first three lines, and the
+// cursor at its first group.  One wait for all of it: a tile would
+// otherwise begin with a chain of dependent scalar loads.  The waves also
+// touch the rest of the first kWarm bytes between them, so that the terms
+// and records of a pass come from the scalar cache: a launch starts with
+// that cache empty.
+struct Head {
+	v16u w[3];
+	__device__ __forceinline__ uint32_t at(size_t byte) const
+	{
+		return w[byte / 64][byte % 64 / 4];
+	}
+};
+
+template <int NT>
+__device__ __forceinline__ void load_head(cHead H, uint32_t wave, Head &h,
+	Cursor &C)
+{
+	C.desc = reinterpret_cast<uint64_t>(H);
+	uint32_t woff = wave * 64, t;
+	if constexpr (NT == 256)
+		__asm__ volatile(
+			"s_load_dwordx16 %[a], %[p], 0x0\n\t"
+			"s_load_dwordx16 %[b], %[p], 0x40\n\t"
+			"s_load_dwordx16 %[c], %[p], 0x80\n\t"
+			"s_load_dwordx8 %[f], %[p], %[first]\n\t"
+			"s_load_dword %[t], %[p], %[o] offset:0xc0\n\t"
+			"s_load_dword %[t], %[p], %[o] offset:0x1c0\n\t"
+			"s_load_dword %[t], %[p], %[o] offset:0x2c0\n\t"
+			"s_load_dword %[t], %[p], %[o] offset:0x3c0\n\t"
+			"s_load_dword %[t], %[p], %[o] offset:0x4c0\n\t"
+			"s_waitcnt lgkmcnt(0)"
+			: [a] "=&s"(h.w[0]), [b] "=&s"(h.w[1]),
+			  [c] "=&s"(h.w[2]), [f] "=&s"(C.term), [t] "=&s"(t)
+			: [p] "s"(C.desc), [o] "s"(woff),
+			  [first] "n"(sizeof(DevHead)));
+	else
+		__asm__ volatile(
+			"s_load_dwordx16 %[a], %[p], 0x0\n\t"
+			"s_load_dwordx16 %[b], %[p], 0x40\n\t"
+			"s_load_dwordx16 %[c], %[p], 0x80\n\t"
+			"s_load_dwordx8 %[f], %[p], %[first]\n\t"
+			"s_load_dword %[t], %[p], %[o] offset:0xc0\n\t"
+			"s_load_dword %[t], %[p], %[o] offset:0x2c0\n\t"
+			"s_load_dword %[t], %[p], %[o] offset:0x4c0\n\t"
+			"s_waitcnt lgkmcnt(0)"
+			: [a] "=&s"(h.w[0]), [b] "=&s"(h.w[1]),
+			  [c] "=&s"(h.w[2]), [f] "=&s"(C.term), [t] "=&s"(t)
+			: [p] "s"(C.desc), [o] "s"(woff),
+			  [first] "n"(sizeof(DevHead)));
+	C.rec = C.desc + h.at(offsetof(DevHead, xoff));
+	C.count = h.at(offsetof(DevHead, count));
+	C.off = sizeof(DevHead) + sizeof(DevTerm);
+}
+
 // Base index of tile t: its bits moved to the index bits that the tile
 // does not gather, a run of them at a time.
-__device__ __forceinline__ uint64_t tile_base(cHead H, uint64_t t)
+__device__ __forceinline__ uint64_t tile_base(const Head &h, uint64_t t)
 {
 	uint64_t base = 0;
-	const uint32_t n = H->nseg;
+	const uint32_t n = h.at(offsetof(DevHead, nseg));
 #pragma unroll
 	for (int i = 0; i < kSegMax; i++) {
-		if ((i == 4 || i == 8) && n <= (uint32_t)i)
+		if ((i == 3 || i == 5 || i == 7 || i == 10) && n <= (uint32_t)i)
 			break;
-		const uint32_t sg = H->seg[i];
+		const uint32_t sg = h.at(offsetof(DevHead, seg) + 4 * i);
 		uint64_t f;
 		__asm__("s_bfe_u64 %0, %1, %2" : "=s"(f) : "s"(t), "s"(sg) :
 			"scc");
@@ -599,15 +690,15 @@ __device__ __forceinline__ uint64_t tile_base(cHead H, uint64_t t)
 	return base;
 }
 
-// HBM index, within the tile at base, of the coset base of thread tid in
-// the first (side 0) or last (side 1) group.
-template <int NB>
-__device__ __forceinline__ uint64_t coset_index(cHead H, int side,
-	uint64_t base, uint32_t tid, uint32_t wave)
+// HBM index of thread tid's coset base from the columns col(k) of its index
+// bits, starting at base: the bits from 6 up are uniform in a wave.
+template <int NB, class F>
+__device__ __forceinline__ uint64_t coset_index(F col, uint64_t base,
+	uint32_t tid, uint32_t wave)
 {
 #pragma unroll
 	for (int k = 6; k < NB; k++)
-		base ^= H->col[side][k] & (0 - (uint64_t)(wave >> (k - 6) & 1u));
+		base ^= col(k) & (0 - (uint64_t)(wave >> (k - 6) & 1u));
 	uint32_t lo = (uint32_t)base, hi = (uint32_t)(base >> 32);
 	// the thread index is re-read per use: kept from one to the next, the
 	// masks of its bits would hold registers throughout
@@ -615,11 +706,26 @@ __device__ __forceinline__ uint64_t coset_index(cHead H, int side,
 #pragma unroll
 	for (int k = 0; k < 6; k++) {
 		const uint32_t m = bit_mask(tid, k);
-		const uint64_t c = H->col[side][k];
-		lo ^= m & (uint32_t)c;
-		hi ^= m & (uint32_t)(c >> 32);
+		const uint64_t c = col(k);
+		lo = xor_masked(lo, m, (uint32_t)c);
+		hi = xor_masked(hi, m, (uint32_t)(c >> 32));
 	}
 	return (uint64_t)hi << 32 | lo;
+}
+
+__device__ __forceinline__ uint64_t head_u64(const Head &h, size_t at)
+{
+	return (uint64_t)h.at(at + 4) << 32 | h.at(at);
+}
+
+// HBM index, from base, of thread tid's coset base in the first group.
+template <int NB>
+__device__ __forceinline__ uint64_t first_index(const Head &h, uint64_t base,
+	uint32_t tid, uint32_t wave)
+{
+	return coset_index<NB>([&](int k) {
+		return head_u64(h, offsetof(DevHead, col0) + 8 * k);
+	}, base, tid, wave);
 }
 
 // Coset element of step i of a walk that changes one basis vector at a
@@ -633,30 +739,34 @@ constexpr int gray_bit(int i)
 	return __builtin_ctz(i + 1);
 }
 
-// The cosets of the first group from HBM: elements with index in [E0, E1).
-template <int TB, int D>
+// The cosets of the first group from HBM, the coset base at index i.
+template <int D>
 __device__ __forceinline__ void load_coset(const v2d *__restrict__ a,
-	cHead H, uint64_t base, uint32_t tid, uint32_t wave, v2d (&cs)[1 << D])
+	const Head &h, uint64_t i, v2d (&cs)[1 << D])
 {
-	uint64_t i = coset_index<TB - D>(H, 0, base, tid, wave);
 #pragma unroll
 	for (int e = 0; e < (1 << D); e++) {
 		cs[gray(e)] = a[i];
 		if (e + 1 < (1 << D))
-			i ^= H->dc[0][gray_bit(e)];
+			i ^= head_u64(h, offsetof(DevHead, dc0) +
+				8 * gray_bit(e));
 	}
 }
 
+// The cosets of the last group to HBM.
 template <int TB, int D>
-__device__ __forceinline__ void store_coset(v2d *__restrict__ a, cHead H,
-	uint64_t base, uint32_t tid, uint32_t wave, const v2d (&cs)[1 << D])
+__device__ __forceinline__ void store_coset(v2d *__restrict__ a,
+	uint64_t desc, uint64_t base, uint32_t tid, uint32_t wave,
+	const v2d (&cs)[1 << D])
 {
-	uint64_t i = coset_index<TB - D>(H, 1, base, tid, wave);
+	cHead H = reinterpret_cast<cHead>(desc);
+	uint64_t i = coset_index<TB - D>([&](int k) { return H->col1[k]; },
+		base, tid, wave);
 #pragma unroll
 	for (int e = 0; e < (1 << D); e++) {
 		a[i] = cs[gray(e)];
 		if (e + 1 < (1 << D))
-			i ^= H->dc[1][gray_bit(e)];
+			i ^= H->dc1[gray_bit(e)];
 	}
 }
 
@@ -664,7 +774,7 @@ __device__ __forceinline__ void store_coset(v2d *__restrict__ a, cHead H,
 // in order (left free, the compiler forms all of them ahead and keeps them
 // for both rounds of a half-tile exchange, 32 registers).
 template <int D>
-__device__ __forceinline__ void lds_write(char *buf, uint32_t at,
+__device__ __forceinline__ void lds_write(lds_t buf, uint32_t at,
 	const uint32_t (&g)[4], const v2d (&cs)[1 << D])
 {
 	__asm__ volatile("" : "+v"(at));
@@ -672,14 +782,15 @@ __device__ __forceinline__ void lds_write(char *buf, uint32_t at,
 	for (int e = 0; e < (1 << D); e++) {
 		if (e && e % 4 == 0)
 			__builtin_amdgcn_sched_barrier(0);
-		*reinterpret_cast<v2d *>(buf + at) = cs[gray(e)];
+		*(__attribute__((address_space(3))) v2d *)(buf + at) =
+			cs[gray(e)];
 		if (e + 1 < (1 << D))
 			at ^= g[gray_bit(e)];
 	}
 }
 
 template <int D>
-__device__ __forceinline__ void lds_read(const char *buf, uint32_t at,
+__device__ __forceinline__ void lds_read(lds_t buf, uint32_t at,
 	const uint32_t (&g)[4], v2d (&cs)[1 << D])
 {
 	__asm__ volatile("" : "+v"(at));
@@ -687,7 +798,8 @@ __device__ __forceinline__ void lds_read(const char *buf, uint32_t at,
 	for (int e = 0; e < (1 << D); e++) {
 		if (e && e % 4 == 0)
 			__builtin_amdgcn_sched_barrier(0);
-		cs[gray(e)] = *reinterpret_cast<const v2d *>(buf + at);
+		cs[gray(e)] =
+			*(__attribute__((address_space(3))) v2d *)(buf + at);
 		if (e + 1 < (1 << D))
 			at ^= g[gray_bit(e)];
 	}
@@ -704,31 +816,33 @@ __device__ __forceinline__ void lds_read(const char *buf, uint32_t at,
 // the waves whose coset-index bit xk is that half).  lead: the buffer has
 // earlier readers in this workgroup.
 template <int TB, int D, bool HALF>
-__device__ __forceinline__ void exchange(char *buf, cGroup G, uint32_t tid,
-	uint32_t wave, bool lead, v2d (&cs)[1 << D])
+__device__ __forceinline__ void exchange(lds_t buf, const v16u &x,
+	uint32_t tid, uint32_t wave, bool lead, v2d (&cs)[1 << D])
 {
 	constexpr int NB = TB - D, SH = lds_shift(TB, HALF);
+	constexpr int COL = offsetof(DevExchange, col) / 4;
+	constexpr int GV = offsetof(DevExchange, g) / 4;
 	uint32_t acc = 0;
 #pragma unroll
 	for (int k = 6; k < NB; k++)
-		acc ^= G->col[k] & (0 - (wave >> (k - 6) & 1u));
+		acc ^= x[COL + k] & (0 - (wave >> (k - 6) & 1u));
 	__asm__ volatile("" : "+v"(tid));   // as in coset_index
 #pragma unroll
 	for (int k = 0; k < 6; k++)
-		acc ^= bit_mask(tid, k) & G->col[k];
+		acc = xor_masked(acc, bit_mask(tid, k), x[COL + k]);
 	const uint32_t sw = (acc & 0xffffu) << SH, sr = (acc >> 16) << SH;
 	uint32_t gw[4], gr[4];
 #pragma unroll
 	for (int i = 0; i < D; i++) {
-		gw[i] = (G->g[i] & 0xffffu) << SH;
-		gr[i] = (G->g[i] >> 16) << SH;
+		gw[i] = (x[GV + i] & 0xffffu) << SH;
+		gr[i] = (x[GV + i] >> 16) << SH;
 	}
 	if constexpr (!HALF) {
 		lds_write<D>(buf, sw, gw, cs);
 		__syncthreads();
 		lds_read<D>(buf, sr, gr, cs);
 	} else {
-		const uint32_t half = wave >> G->xk & 1u;
+		const uint32_t half = wave >> x[1] & 1u;
 		for (uint32_t q = 0; q < 2; q++) {
 			// the buffer's previous readers are done
 			if (lead || q > 0)
@@ -747,45 +861,49 @@ __device__ __forceinline__ void exchange(char *buf, cGroup G, uint32_t tid,
 // HBM.  One coset per thread: 2^(TB - D) threads.  fresh: the buffer has no
 // earlier readers in this workgroup (its first tile).
 template <int TB, int D, bool HALF>
-__device__ __forceinline__ void run_groups(v2d *__restrict__ a, char *buf,
-	cHead H, uint64_t base, uint32_t tid, uint32_t wave, bool fresh,
-	v2d (&cs)[1 << D])
+__device__ __forceinline__ void run_groups(v2d *__restrict__ a, lds_t buf,
+	Cursor C, uint32_t ngroups, uint64_t base, uint32_t tid, uint32_t wave,
+	bool fresh, v2d (&cs)[1 << D])
 {
 	// the index bits that select the half must select whole 64-lane waves
 	static_assert(TB - D >= 8 && TB - D <= kThreadBits,
 		"2^(TB-D) threads, 256..1024");
-	cGroup G = reinterpret_cast<cGroup>(H + 1);
-	const uint64_t at = reinterpret_cast<uint64_t>(H);
-	const uint32_t n = H->ngroups;
 	// one copy of the loop body (a peeled first round would double the
 	// 28 KiB of handlers at D = 4, beyond the instruction cache)
 #pragma clang loop unroll(disable)
-	for (uint32_t gi = 0;; gi++, G++) {
-		if (G->count)
-			group_terms<D>(cs, at + G->toff, G->count, tid, base);
-		if (gi + 1 == n)
+	for (uint32_t gi = 0;; gi++) {
+		v16u x;
+		group_terms<D>(cs, C, tid, base, x);
+		if (gi + 1 == ngroups)
 			break;
+		C.count = x[0];
+		C.rec += sizeof(DevExchange);
 		// a whole tile has its slots to itself after the first
 		// exchange of a tile; the first one overwrites what the tile
 		// before it left
 		if (!HALF && gi == 0 && !fresh)
 			__syncthreads();
-		exchange<TB, D, HALF>(buf, G, tid, wave, gi > 0 || !fresh, cs);
+		exchange<TB, D, HALF>(buf, x, tid, wave, gi > 0 || !fresh, cs);
 	}
-	store_coset<TB, D>(a, H, base, tid, wave, cs);
+	store_coset<TB, D>(a, C.desc, base, tid, wave, cs);
 }
 
 // Load one tile from HBM, apply the pass, write it back.
 template <int TB, int D, bool HALF>
-__device__ __forceinline__ void fused_tile(v2d *__restrict__ a, char *buf,
-	cHead H, uint64_t t)
+__device__ __forceinline__ void fused_tile(v2d *__restrict__ a, lds_t buf,
+	const Head &h, const Cursor &C, uint32_t wave, uint64_t t)
 {
 	const uint32_t tid = threadIdx.x;
-	const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-	const uint64_t base = tile_base(H, t);
+	const uint64_t base = tile_base(h, t);
 	v2d cs[1 << D];
-	load_coset<TB, D>(a, H, base, tid, wave, cs);
-	run_groups<TB, D, HALF>(a, buf, H, base, tid, wave, true, cs);
+	load_coset<D>(a, h, first_index<TB - D>(h, base, tid, wave), cs);
+	run_groups<TB, D, HALF>(a, buf, C, h.w[0][0], base, tid, wave, true,
+		cs);
+}
+
+__device__ __forceinline__ uint32_t wave_index()
+{
+	return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 }
 
 // The descriptor of the kernels that take it by value: a DevPass after the
@@ -816,13 +934,17 @@ __global__ __launch_bounds__((1 << TB) >> D) void k_rot_fused(
 	double2 *__restrict__ amp, const DevPass P, uint64_t ntiles)
 {
 	__shared__ v2d tile[1u << TB];
+	Head h;
+	Cursor C;
+	const uint32_t wave = wave_index();
+	load_head<((1 << TB) >> D)>(arg_head(), wave, h, C);
 	// 2-D grid when the tiles outnumber kMaxGrid (gridDim.x * 256 < 2^32)
 	const uint64_t w = (uint64_t)blockIdx.y * gridDim.x + blockIdx.x;
 	if (w >= ntiles)
 		return;           // whole workgroup: no barrier is left waiting
 	// clang vector type: plain 16-byte accesses that stay in registers
-	fused_tile<TB, D, false>(reinterpret_cast<v2d *>(amp),
-		reinterpret_cast<char *>(tile), arg_head(), xcd_tile(w, ntiles));
+	fused_tile<TB, D, false>(reinterpret_cast<v2d *>(amp), (lds_t)tile, h,
+		C, wave, xcd_tile(w, ntiles));
 }
 
 // Waves per SIMD that the LDS of the half-tile form allows (160 KiB per CU,
@@ -843,11 +965,15 @@ void k_rot_fused_half(
 	double2 *__restrict__ amp, const DevPass P, uint64_t ntiles)
 {
 	__shared__ v2d buf[1u << (TB - 1)];
+	Head h;
+	Cursor C;
+	const uint32_t wave = wave_index();
+	load_head<((1 << TB) >> D)>(arg_head(), wave, h, C);
 	const uint64_t w = (uint64_t)blockIdx.y * gridDim.x + blockIdx.x;
 	if (w >= ntiles)
 		return;           // whole workgroup: no barrier is left waiting
-	fused_tile<TB, D, true>(reinterpret_cast<v2d *>(amp),
-		reinterpret_cast<char *>(buf), arg_head(), xcd_tile(w, ntiles));
+	fused_tile<TB, D, true>(reinterpret_cast<v2d *>(amp), (lds_t)buf, h, C,
+		wave, xcd_tile(w, ntiles));
 }
 
 // Persistent walk over tiles with the next tile's first-group cosets
@@ -860,24 +986,29 @@ void k_rot_fused_half(
 // xcd_tile orders them).  Every workgroup leaves the loop once its next
 // virtual index reaches ntiles.
 template <int TB, int D, int PF, bool HALF>
-__device__ __forceinline__ void walk_tiles(v2d *__restrict__ a, char *buf,
+__device__ __forceinline__ void walk_tiles(v2d *__restrict__ a, lds_t buf,
 	cHead H, uint64_t ntiles)
 {
 	static_assert(PF > 0 && PF <= (1 << D), "prefetched amplitudes");
-	const uint32_t tid = threadIdx.x;
-	const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const uint32_t tid = threadIdx.x, wave = wave_index();
 	uint64_t v = blockIdx.x;
 	if (v >= ntiles)
 		return;           // whole workgroup: no barrier is left waiting
+	Head h;
+	Cursor C;
+	load_head<((1 << TB) >> D)>(H, wave, h, C);
+	const auto dc = [&](int e) {
+		return head_u64(h, offsetof(DevHead, dc0) + 8 * (gray_bit(e) & 3));
+	};
 	// HBM offset of the first group's coset base within any tile
-	const uint64_t off0 = coset_index<TB - D>(H, 0, 0, tid, wave);
-	uint64_t base = tile_base(H, xcd_tile(v, ntiles));
+	const uint64_t off0 = first_index<TB - D>(h, 0, tid, wave);
+	uint64_t base = tile_base(h, xcd_tile(v, ntiles));
 	v2d cs[1 << D], pre[PF];
 	uint64_t i = base ^ off0;
 #pragma unroll
 	for (int e = 0; e < PF; e++) {
 		pre[e] = a[i];
-		i ^= H->dc[0][gray_bit(e) & 3];
+		i ^= dc(e);
 	}
 	for (bool fresh = true;; fresh = false) {
 		i = base ^ off0;
@@ -887,20 +1018,21 @@ __device__ __forceinline__ void walk_tiles(v2d *__restrict__ a, char *buf,
 				cs[gray(e)] = pre[e < PF ? e : 0];
 			else
 				cs[gray(e)] = a[i];
-			i ^= H->dc[0][gray_bit(e) & 3];
+			i ^= dc(e);
 		}
 		const uint64_t vn = v + gridDim.x;
 		const bool more = vn < ntiles;
-		const uint64_t bn = more ? tile_base(H, xcd_tile(vn, ntiles)) : 0;
+		const uint64_t bn = more ? tile_base(h, xcd_tile(vn, ntiles)) : 0;
 		if (more) {
 			i = bn ^ off0;
 #pragma unroll
 			for (int e = 0; e < PF; e++) {
 				pre[e] = a[i];
-				i ^= H->dc[0][gray_bit(e) & 3];
+				i ^= dc(e);
 			}
 		}
-		run_groups<TB, D, HALF>(a, buf, H, base, tid, wave, fresh, cs);
+		run_groups<TB, D, HALF>(a, buf, C, h.w[0][0], base, tid, wave,
+			fresh, cs);
 		if (!more)
 			break;
 		v = vn;
@@ -915,7 +1047,7 @@ void k_rot_fused_hpipe(double2 *__restrict__ amp, const DevPass P,
 {
 	__shared__ v2d buf[1u << (TB - 1)];
 	walk_tiles<TB, D, PF, true>(reinterpret_cast<v2d *>(amp),
-		reinterpret_cast<char *>(buf), arg_head(), ntiles);
+		(lds_t)buf, arg_head(), ntiles);
 }
 
 // The same in the whole-tile form, every amplitude prefetched.
@@ -925,7 +1057,7 @@ __global__ __launch_bounds__((1 << TB) >> D) void k_rot_fused_pipe(
 {
 	__shared__ v2d tile[1u << TB];
 	walk_tiles<TB, D, 1 << D, false>(reinterpret_cast<v2d *>(amp),
-		reinterpret_cast<char *>(tile), arg_head(), ntiles);
+		(lds_t)tile, arg_head(), ntiles);
 }
 
 // Batched pass: pass p of many registers in one launch.  Work item i covers
@@ -963,10 +1095,13 @@ void k_rot_fused_batch(
 			hi = mid;
 	}
 	const BatchItem it = items[lo];
+	Head h;
+	Cursor C;
+	const uint32_t wave = wave_index();
+	load_head<((1 << TB) >> D)>(reinterpret_cast<cHead>(
+		reinterpret_cast<uint64_t>(descs) + it.desc), wave, h, C);
 	fused_tile<TB, D, HALF>(reinterpret_cast<v2d *>(amp) + it.amp_off,
-		reinterpret_cast<char *>(tile),
-		reinterpret_cast<cHead>(reinterpret_cast<uint64_t>(descs) +
-			it.desc), t - it.tile0);
+		(lds_t)tile, h, C, wave, t - it.tile0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1885,28 +2020,35 @@ size_t pack_pass(const FusedPass &P, uint32_t tb, bool half, uint8_t *out)
 				i ^= P.w[b];
 		return i;
 	};
-	for (int side = 0; side < 2; side++) {
-		const FusedGroup &G = *g[side ? n - 1 : 0];
-		for (uint32_t k = 0; k < nb; k++)
-			H.col[side][k] = hbm(1u << G.jpos[k]);
-		for (uint32_t i = 0; i < D; i++)
-			H.dc[side][i] = hbm(G.u[i]);
+	for (uint32_t k = 0; k < nb; k++) {
+		const uint64_t f = hbm(1u << g[0]->jpos[k]);
+		H.col0[k][0] = (uint32_t)f;
+		H.col0[k][1] = (uint32_t)(f >> 32);
+		H.col1[k] = hbm(1u << g[n - 1]->jpos[k]);
 	}
+	for (uint32_t i = 0; i < D; i++) {
+		const uint64_t f = hbm(g[0]->u[i]);
+		H.dc0[i][0] = (uint32_t)f;
+		H.dc0[i][1] = (uint32_t)(f >> 32);
+		H.dc1[i] = hbm(g[n - 1]->u[i]);
+	}
+	H.count = g[0]->count;
+	// the terms in order, then one that is fetched and never run
+	H.xoff = (uint32_t)(sizeof H + (P.nterms + 1u) * sizeof(DevTerm));
 	memcpy(out, &H, sizeof H);
 
-	size_t at = sizeof H, to = sizeof H + n * sizeof(DevGroup);
+	size_t to = sizeof H, at = H.xoff;
 	for (uint32_t q = 0; q < n; q++) {
 		const FusedGroup &G = *g[q];
-		DevGroup W;
+		DevExchange W;
 		memset(&W, 0, sizeof W);
-		W.count = G.count;
-		W.toff = (uint32_t)to;
 		if (q + 1 < n) {
 			const FusedGroup &N = *g[q + 1];
 			const auto slot = [&](uint32_t v) {
 				return (half ? half_slot(tb, v, G.xh) :
 					lds_slot(v)) << 4 >> sh;
 			};
+			W.count = N.count;
 			if (half)
 				W.xk = G.xk - 6u;
 			for (uint32_t k = 0; k < nb; k++)
@@ -1933,8 +2075,8 @@ size_t pack_pass(const FusedPass &P, uint32_t tb, bool half, uint8_t *out)
 			to += sizeof T;
 		}
 	}
-	memset(out + to, 0, sizeof(DevTerm));   // fetched, never run
-	return (to + sizeof(DevTerm) + 15) & ~size_t{15};
+	memset(out + to, 0, sizeof(DevTerm));
+	return (at + 15) & ~size_t{15};
 }
 
 // Bit tb set: passes of tile width tb take the half-tile form where they
@@ -3203,7 +3345,7 @@ int ph2hip_batch_plan_launch(void *amp, struct ph2hip_batch_plan *pl,
 	const uint32_t tile_bits = pl->tile_bits;
 	// The upload follows the work already queued on the stream, so the
 	// launches of an earlier plan have read the buffers before they change.
-	if (dev_reserve(&g_bdesc, &g_bdesc_cap, pl->desc_bytes) ||
+	if (dev_reserve(&g_bdesc, &g_bdesc_cap, pl->desc_bytes + kWarm) ||
 	    dev_reserve(&g_bitem, &g_bitem_cap, sizeof(BatchItem) * ndesc))
 		return -1;
 	if (hipMemcpyAsync(g_bdesc, pl->desc, pl->desc_bytes,
