@@ -87,10 +87,10 @@ int ph2hip_rotate_fused(void *amp, uint32_t nqb, const struct ph2hip_rot *rot,
  * workgroup per tile.  Initial mask from PHASE2_HIP_PIPE, else 0. */
 int ph2hip_set_fused_form(uint32_t pipe_mask, uint64_t persistent_wgs);
 
-/* Whether the first and last micro-group of a fused pass may move their
- * cosets straight between HBM and registers (when their lanes cover whole
- * 256-byte runs), skipping the LDS staging of the tile; on by default.
- * Every setting gives the same state. */
+/* Whether the first and last micro-group of a fused pass move their cosets
+ * straight between HBM and registers, skipping the LDS staging of the tile;
+ * on by default.  Passes in the half-tile form always do.  Every setting
+ * gives the same state. */
 int ph2hip_set_fused_direct(int on);
 
 /* Bit tb of tile_mask: fused passes of tile width tb take the half-tile

@@ -431,10 +431,12 @@ constexpr int lds_shift(int tb, bool half)
 	".ifndef ph2_macros\n"                                              \
 	".set ph2_macros, 1\n"                                              \
 	/* next term: its scalars, sg, the fetch of the one after, jump */  \
-	".macro PH2_NEXT id\n"                                              \
+	".macro PH2_NEXT id, wait\n"                                        \
 	"s_sub_u32 s80, s80, 1\n"                                           \
 	"s_cbranch_scc1 .Lph2x\\id\n"                                       \
+	".if \\wait\n"                                                      \
 	"s_waitcnt lgkmcnt(0)\n"                                            \
+	".endif\n"                                                          \
 	"s_and_b64 s[86:87], s[72:73], s[82:83]\n"                          \
 	"v_and_b32 v14, s78, v15\n"                                         \
 	"s_bcnt1_i32_b64 s86, s[86:87]\n"                                   \
@@ -506,7 +508,7 @@ constexpr int lds_shift(int tb, bool half)
 	".else\n"                                                           \
 	"PH2_PATTERN 1<<(\\d-1), ph2_x, 0, \\odd\n"                         \
 	".endif\n"                                                          \
-	"PH2_NEXT \\id\n"                                                   \
+	"PH2_NEXT \\id, 1\n"                                                \
 	".if (ph2_x==1)&&(\\odd==0)\n"                                      \
 	".Lph2n\\id:\n"                                                     \
 	".endif\n"                                                          \
@@ -522,7 +524,7 @@ constexpr int lds_shift(int tb, bool half)
 	"PH2_HALF ph2_a, ph2_a+2, ph2_a+2, ph2_a, 1, 0\n"                   \
 	".set ph2_k, ph2_k+1\n"                                             \
 	".endr\n"                                                           \
-	"PH2_NEXT \\id\n"                                                   \
+	"PH2_NEXT \\id, 1\n"                                                \
 	".endm\n"                                                           \
 	".endif\n"
 
@@ -537,7 +539,8 @@ constexpr int lds_shift(int tb, bool half)
 	".Lph2p%=:\n"                                                       \
 	"s_add_u32 s84, s84, (.Lph2h%= - .Lph2p%=)\n"                       \
 	"s_addc_u32 s85, s85, 0\n"                                          \
-	"PH2_NEXT %=\n"                                                     \
+	/* the first term is here already */                                \
+	"PH2_NEXT %=, 0\n"                                                  \
 	".Lph2h%=:\n"                                                       \
 	"PH2_PATTERNS " #d ", 0, %=\n"                                      \
 	"PH2_PATTERNS " #d ", 1, %=\n"                                      \
@@ -607,6 +610,21 @@ __device__ __forceinline__ void group_terms(v2d (&a)[1 << D], Cursor &C,
 __device__ __forceinline__ uint32_t bit_mask(uint32_t tid, int k)
 {
 	return (uint32_t)((int)(tid << (31 - k)) >> 31);
+}
+
+// acc ^ c if bit k of the uniform word w is set, on the scalar unit (in C++
+// the compiler takes it to the vector unit).
+template <int K>
+__device__ __forceinline__ uint32_t xor_bit(uint32_t acc, uint32_t w,
+	uint32_t c)
+{
+	uint32_t t;
+	__asm__("s_bitcmp1_b32 %[w], %[k]\n\t"
+		"s_cselect_b32 %[t], %[c], 0\n\t"
+		"s_xor_b32 %[a], %[a], %[t]"
+		: [a] "+s"(acc), [t] "=&s"(t)
+		: [w] "s"(w), [c] "s"(c), [k] "n"(K) : "scc");
+	return acc;
 }
 
 // acc ^ (m & c), one instruction.
@@ -823,9 +841,14 @@ __device__ __forceinline__ void exchange(lds_t buf, const v16u &x,
 	constexpr int COL = offsetof(DevExchange, col) / 4;
 	constexpr int GV = offsetof(DevExchange, g) / 4;
 	uint32_t acc = 0;
-#pragma unroll
-	for (int k = 6; k < NB; k++)
-		acc ^= x[COL + k] & (0 - (wave >> (k - 6) & 1u));
+	if constexpr (NB > 6)
+		acc = xor_bit<0>(acc, wave, x[COL + 6]);
+	if constexpr (NB > 7)
+		acc = xor_bit<1>(acc, wave, x[COL + 7]);
+	if constexpr (NB > 8)
+		acc = xor_bit<2>(acc, wave, x[COL + 8]);
+	if constexpr (NB > 9)
+		acc = xor_bit<3>(acc, wave, x[COL + 9]);
 	__asm__ volatile("" : "+v"(tid));   // as in coset_index
 #pragma unroll
 	for (int k = 0; k < 6; k++)
@@ -1953,18 +1976,15 @@ int build_pass_mode(FusedPass &P, const struct ph2hip_rot *r, size_t len,
 		}
 	}
 	P.ngroups = (uint8_t)ng;
-	// First and last group straight between HBM and registers when their
-	// coset-index bits 0..3 are tile bits 0..3 inside rows of >= 16; for a
+	// First and last group straight between HBM and registers; for a
 	// half-tile pass always (the tile is never staged whole in LDS).
-	if ((g_direct && L >= 4) || half) {
-		for (int side = 0; side < 2; side++) {
-			const FusedGroup &G = P.grp[side ? ng - 1 : 0];
-			if (!half && (G.jpos[0] != 0 || G.jpos[1] != 1 ||
-			    G.jpos[2] != 2 || G.jpos[3] != 3))
-				continue;
-			P.dflags |= 1u << side;
-		}
-	}
+	// Staging costs two exchanges a pass and buys coalesced rows where a
+	// group flips low qubits; without it a 1024-term sweep runs 8% faster
+	// at 16 and 18 qubits (379 -> 349, 454 -> 416 us, tile 10), 7% at 20
+	// (726 -> 677, tile 11), 4% at 22 and 3% at 24 at tile 11 (2084 ->
+	// 1991, 7884 -> 7660), and as fast at tile 12.
+	if (g_direct || half)
+		P.dflags |= 3u;
 	if (half)
 		P.dflags |= 4u;
 	return 0;

@@ -64,29 +64,28 @@ struct qreg_hip {
 #define AMP_QMAX ((size_t)1 << 20)   /* 24 MiB of queued writes */
 
 static int g_mode = -1;
-/* tile 0: auto_tile(); low 3 measured best of 3..5 for the greedy cut with
- * the half-tile kernel (33 qubits 0.7%, 26 qubits 3.5%, composite
- * integrator at 30 qubits 7% faster than 4) */
+/* tile 0: auto_tile() and auto_low() */
 static uint32_t g_tile = 0, g_low = 3;
 static ph2_sched_fn g_sched_fn;
 static void *g_sched_ctx;
 
-/* Tile width when none is set.
- *
- * Registers whose repeated sweeps replay from a captured graph (at most
- * ph2hip_replay_max_qb() qubits, 20 by default) are bound by each pass's
- * latency, not by launches.  Measured per step of a lex-ordered 470-611
- * term sweep replayed 64 times, tile 10 is best from 12 to 18 qubits and
- * tile 11 at 19 and 20.  Against the rule below, at 14, 16, 18 and 20
- * qubits: 0.287 vs 0.322, 0.318 vs 0.339, 0.390 vs 0.507 and 0.696 vs
- * 0.765 ms.  Never above nqb - 2.
- *
- * Otherwise: 13 from 26 qubits (the half-tile form at tile 13 sweeps 26
- * qubits 4.7% faster than at tile 12, and a pass still has 8192 tiles), 12
- * from 17, nqb - 5 below.  Small registers are latency-bound (a few dozen
- * workgroups per pass); without replay, at 16 qubits a whole Trotter run
- * takes 0.476 ms per step at tile 11, 0.503 at 10, 0.532 at 9 and 0.564 at
- * 12. */
+/* Tile width when none is set, from 1024-term blocks of lex-ordered sweeps
+ * timed at every tile width (us per block at the widths beside each line):
+ *   to 18 qubits, tile 10: 300, 349 and 416 at 13, 16 and 18 qubits
+ *     against 323, 369 and 421 at tile 11.  A few dozen workgroups, bound
+ *     by each pass's chain of terms and exchanges;
+ *   19 to 21, tile 11: 464, 676, 997 at 19, 20, 21 against 521, 786, 1257
+ *     at tile 10 and 609, 722, 1047 at tile 12;
+ *   22 and 23, tile 12: 1730 and 3371 against 1991 and 3749 at tile 11 and
+ *     1770 and 3385 at tile 13;
+ *   from 24, tile 13: 6748 and 15112 at 24 and 25 against 6841 and 17452 at
+ *     tile 12.  HBM traffic per pass weighs most and wider tiles need fewer
+ *     passes.
+ * Without replay of captured sweeps (ph2hip_replay_max_qb, 20 qubits by
+ * default) launches weigh more below: 12 from 17 qubits, nqb - 5 under
+ * that (at 16 qubits a Trotter step took 0.476 ms at tile 11, 0.503 at 10,
+ * 0.532 at 9 and 0.564 at 12).  Never above nqb - 2 in the replayed
+ * range. */
 static uint32_t auto_tile(uint32_t nqb)
 {
 	uint32_t t;
@@ -95,9 +94,21 @@ static uint32_t auto_tile(uint32_t nqb)
 		if (t + 2 > nqb)
 			t = nqb > 2 ? nqb - 2 : 0;
 	} else {
-		t = nqb >= 26 ? 13 : nqb > 16 ? 12 : (nqb > 5 ? nqb - 5 : 0);
+		t = nqb >= 24 ? 13 : nqb == 21 ? 11 : nqb > 16 ? 12 :
+			(nqb > 5 ? nqb - 5 : 0);
 	}
 	return t < PH2HIP_TILE_MIN ? PH2HIP_TILE_MIN : t;
+}
+
+/* Contiguous low bits the cut asks for under the automatic tile width: at
+ * most `low`, and 2 from 24 qubits, where rows of 64 bytes leave one more
+ * dimension to gather.  Same sweeps, low 2 against 3 at tile 13: 6547 and
+ * 6748 us at 24 qubits, 14874 and 15112 at 25, 62623 and 63233 at 27,
+ * 130562 and 134986 at 28, 538698 and 551383 at 30; low 1 is slower from
+ * 30.  Below 24 qubits the two are within 1%. */
+static uint32_t auto_low(uint32_t nqb, uint32_t low)
+{
+	return nqb >= 24 && low > 2 ? 2 : low;
 }
 
 static void load_defaults(void)
@@ -447,7 +458,8 @@ void qreg_paulirot(struct qreg *reg, struct paulis code_hi,
 		if (rc < 0)
 			rc = ph2_sched_greedy(h->rot, ncodes, nqb,
 				h->tile_bits ? h->tile_bits : auto_tile(nqb),
-				h->low_bits, &h->sched);
+				h->tile_bits ? h->low_bits :
+					auto_low(nqb, h->low_bits), &h->sched);
 		if (rc == 0)
 			rc = ph2hip_rotate_fused(h->damp, nqb, h->rot, ncodes,
 				h->sched.len, h->sched.tile_bits, h->sched.npass,
