@@ -62,6 +62,12 @@ struct ph2hip_rot {
 int ph2hip_rotate_plain(void *amp, uint32_t nqb, const struct ph2hip_rot *rot,
 	size_t n);
 
+/* The same on a register of 1..8 qubits, one workgroup that keeps it in LDS
+ * for up to 128 terms per launch.  Bit-identical to ph2hip_rotate_plain,
+ * which it calls while profiling is enabled (a record per term). */
+int ph2hip_rotate_small(void *amp, uint32_t nqb, const struct ph2hip_rot *rot,
+	size_t n);
+
 /* Plain-kernel variant: 2, 4 or 8 pairs per thread, plus 16 for
  * non-temporal stores (default 2).  All variants give the same state. */
 int ph2hip_set_plain_form(int form);

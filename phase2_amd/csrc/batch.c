@@ -373,9 +373,13 @@ static int run_round(struct batch *B, size_t r, size_t lim, int mode,
 		void *a = (char *)B->amp + g->off * 16;
 		const int small = nqb < PH2HIP_TILE_MIN;
 		if (mode == PH2_BATCH_PLAIN_EACH || small) {
-			if (ph2hip_rotate_plain(a, nqb, g->rot, g->nrot) < 0)
+			if ((mode == PH2_BATCH_PLAIN_EACH ?
+				    ph2hip_rotate_plain(a, nqb, g->rot, g->nrot) :
+				    ph2hip_rotate_small(a, nqb, g->rot,
+					    g->nrot)) < 0)
 				return -1;
-			B->launches += g->nrot;
+			B->launches += mode == PH2_BATCH_PLAIN_EACH ? g->nrot :
+				(g->nrot + 127) / 128;
 			continue;
 		}
 		const uint32_t t = tb < nqb ? tb : nqb;
@@ -408,13 +412,14 @@ static int run_round(struct batch *B, size_t r, size_t lim, int mode,
 	return 0;
 }
 
-/* Host half of a batched round: greedy schedules of every active register
- * and the pass descriptors of the whole round (no device work). */
-static int plan_round(struct batch *B, size_t r, uint32_t tb, uint32_t low,
-	struct ph2hip_batch_plan **plan)
+/* Host half of a batched round: greedy schedules of the first lim registers
+ * that are active in it and the pass descriptors of the whole round (no
+ * device work). */
+static int plan_round(struct batch *B, size_t r, size_t lim, uint32_t tb,
+	uint32_t low, struct ph2hip_batch_plan **plan)
 {
 	size_t nj = 0;
-	for (size_t i = 0; i < B->n; i++) {
+	for (size_t i = 0; i < lim; i++) {
 		struct breg *g = &B->b[i];
 		if (!active(g, r) || g->nrot == 0)
 			continue;
@@ -463,36 +468,78 @@ static int measure_round(struct batch *B, size_t r, double *out)
 	return 0;
 }
 
-/* Autotuner: time the first round of the first TUNE_REGS registers under
- * each candidate tile/low setting (every setting gives the same state) and
- * keep the fastest. */
+/* Seconds of the first round of the first lim registers under one setting:
+ * the launches alone for batched rounds (their plans are made while the
+ * device runs the round before), everything for the others. */
+static int time_round(struct batch *B, size_t lim, int batched, int mode,
+	uint32_t tb, uint32_t low, double *dt)
+{
+	struct ph2hip_batch_plan *plan = NULL;
+	uint64_t nl;
+	int rc = batched ? plan_round(B, 0, lim, tb, low, &plan) : 0;
+	if (rc < 0 || prep_round(B, 0, lim) < 0 || ph2hip_synchronize() < 0) {
+		ph2hip_batch_plan_free(plan);
+		return -1;
+	}
+	const double t0 = now_s();
+	rc = batched ? ph2hip_batch_plan_launch(B->amp, plan, 0, &nl) :
+		run_round(B, 0, lim, mode, tb, low);
+	if (ph2hip_synchronize() < 0)
+		rc = -1;
+	*dt = now_s() - t0;
+	ph2hip_batch_plan_free(plan);
+	return rc;
+}
+
+/* Autotuner: time the first round of some registers under each tile width,
+ * then the fastest with fewer and with more contiguous low bits (every
+ * setting gives the same state), and keep the fastest.  At most TUNE_REGS
+ * registers, and so few that the five rounds timed are at most a quarter of
+ * the work to come: over nine settings and always 16 registers, a batch of
+ * 40 registers and three samples spent 9 of its 17 ms here.  Tiles wider
+ * than the narrowest register take the batch off its pipeline (18 ms
+ * instead of 7), so they are timed, as what they are, only where the
+ * pipelined choice is a tile below 11. */
 static int autotune(struct batch *B, int mode, uint32_t *tb, uint32_t *low)
 {
-	static const uint32_t TB[] = { 11, 12, 13 };
-	static const uint32_t LOW[] = { 3, 4, 5 };
-	const size_t lim = B->n < TUNE_REGS ? B->n : TUNE_REGS;
+	size_t total = 0;
 	uint32_t minq = 64;
-	for (size_t i = 0; i < lim; i++)
+	for (size_t i = 0; i < B->n; i++) {
 		minq = B->b[i].nqb < minq ? B->b[i].nqb : minq;
-	double best = 1e300;
+		total += rounds_of(&B->b[i]);
+	}
+	size_t lim = total / 20;
+	lim = lim < 1 ? 1 : lim > TUNE_REGS ? TUNE_REGS : lim;
+	lim = lim > B->n ? B->n : lim;
+	double best = 1e300, dt;
 	*tb = 12;
 	*low = 3;
-	for (size_t a = 0; a < sizeof TB / sizeof *TB; a++) {
-		if (TB[a] > minq)
-			continue;
-		for (size_t c = 0; c < sizeof LOW / sizeof *LOW; c++) {
-			if (prep_round(B, 0, lim) < 0 || ph2hip_synchronize() < 0)
-				return -1;
-			const double t0 = now_s();
-			if (run_round(B, 0, lim, mode, TB[a], LOW[c]) < 0 ||
-			    ph2hip_synchronize() < 0)
-				return -1;
-			const double dt = now_s() - t0;
-			if (dt < best) {
-				best = dt;
-				*tb = TB[a];
-				*low = LOW[c];
-			}
+	uint32_t cand[4], nc = 0;
+	if (minq >= 11) {
+		for (uint32_t t = 11; t <= PH2HIP_TILE_MAX && t <= minq; t++)
+			cand[nc++] = t;
+	} else {
+		if (minq >= PH2HIP_TILE_MIN)
+			cand[nc++] = minq;
+		cand[nc++] = 12;
+	}
+	const int batched = mode == PH2_BATCH_FUSED_BATCHED;
+	for (uint32_t c = 0; c < nc; c++) {
+		if (time_round(B, lim, batched && cand[c] <= minq, mode,
+			    cand[c], 3, &dt) < 0)
+			return -1;
+		if (dt < best) {
+			best = dt;
+			*tb = cand[c];
+		}
+	}
+	for (uint32_t l = 2; l <= 4; l += 2) {
+		if (time_round(B, lim, batched && *tb <= minq, mode, *tb, l,
+			    &dt) < 0)
+			return -1;
+		if (dt < best) {
+			best = dt;
+			*low = l;
 		}
 	}
 	B->launches = B->passes = 0;
@@ -540,7 +587,7 @@ static int batch_run(struct batch *B, int mode, uint32_t tile_bits,
 	struct ph2hip_batch_plan *plan = NULL, *next = NULL;
 	if (pipelined && rc == 0 && rounds) {
 		const double tp = now_s();
-		rc = plan_round(B, 0, tile_bits, low_bits, &next);
+		rc = plan_round(B, 0, B->n, tile_bits, low_bits, &next);
 		prep += now_s() - tp;
 	}
 	for (size_t r = 0; r < rounds && rc == 0; r++) {
@@ -567,7 +614,8 @@ static int batch_run(struct batch *B, int mode, uint32_t tile_bits,
 		if (!rc && r + 1 < rounds) {
 			const double tp = now_s();
 			fill_all(B, r + 1);
-			rc = plan_round(B, r + 1, tile_bits, low_bits, &next);
+			rc = plan_round(B, r + 1, B->n, tile_bits, low_bits,
+				&next);
 			prep += now_s() - tp;
 		}
 		if (!rc)

@@ -13,6 +13,7 @@
 // Kernels:
 //   k_rot_pair    plain pass, one thread per amplitude pair (i, i^x), i<j
 //   k_rot_diag    plain pass for diagonal terms (x == 0)
+//   k_rot_small   a run of terms on a register of at most 2^8 amplitudes
 //   k_rot_fused   one HBM pass applying a run of terms in an LDS tile that is
 //                 a coset of span{low bits, flip masks of the run}
 //   k_fill        zeroing (no memset nodes, so the call is graph-safe)
@@ -30,6 +31,7 @@
 #include <cstring>
 #include <cstdarg>
 #include <algorithm>
+#include <mutex>
 
 #include "phase2_hip.h"
 
@@ -204,6 +206,69 @@ __global__ __launch_bounds__(kBlock) void k_rot_diag(
 			st16<NT>(&a[i], v[u]);
 		}
 	}
+	}
+}
+
+// ---------------------------------------------------------------------------
+// registers of at most 2^8 amplitudes
+// ---------------------------------------------------------------------------
+
+// A run of terms on a register too narrow for a tile, in one workgroup: the
+// amplitudes stay in LDS from the first term to the last, one thread per
+// pair.  The plain pass costs such a register a launch per term (2.3 us of
+// host time and as much on the device for a few hundred bytes of work);
+// here a term is one LDS round trip, and a launch takes kSmallTerms.
+constexpr uint32_t kSmallQb = 8, kSmallTerms = 128;
+
+struct SmallTerm {
+	double c, s;
+	uint16_t x, z;
+	uint8_t h, y;        // top bit of x; popcount(x & z) & 3
+	uint16_t pad;
+};
+
+struct SmallRun {
+	uint32_t n;
+	SmallTerm t[kSmallTerms];
+};
+
+static_assert(sizeof(SmallRun) <= 4000, "kernel argument too large");
+
+__global__ __launch_bounds__(1 << (kSmallQb - 1)) void k_rot_small(
+	double2 *__restrict__ amp, uint32_t nqb, const SmallRun R)
+{
+	__shared__ double2 a[1 << kSmallQb];
+	const uint32_t half = 1u << (nqb - 1), t = threadIdx.x;
+	const bool on = t < half;
+	if (on) {
+		a[t] = amp[t];
+		a[t + half] = amp[t + half];
+	}
+	for (uint32_t k = 0; k < R.n; k++) {
+		const uint32_t x = R.t[k].x, z = R.t[k].z;
+		const double c = R.t[k].c, s = R.t[k].s;
+		__syncthreads();
+		if (!on)
+			continue;
+		if (x == 0) {
+			double2 u = a[t], v = a[t + half];
+			rot_diag(u, __popc(t & z) & 1, c, s);
+			rot_diag(v, __popc((t + half) & z) & 1, c, s);
+			a[t] = u;
+			a[t + half] = v;
+		} else {
+			const uint32_t i = (uint32_t)insert_zero(t, R.t[k].h);
+			double2 u = a[i], v = a[i ^ x];
+			rot_pair(u, v, (int)((R.t[k].y + 2 *
+				(__popc(i & z) & 1)) & 3), c, s);
+			a[i] = u;
+			a[i ^ x] = v;
+		}
+	}
+	__syncthreads();
+	if (on) {
+		amp[t] = a[t];
+		amp[t + half] = a[t + half];
 	}
 }
 
@@ -1149,6 +1214,35 @@ __global__ __launch_bounds__(kBlock) void k_gather(
 		out[k] = a[idx[k]];
 }
 
+// Up to kFew indices as kernel arguments: no copy in, and with out in pinned
+// host memory no copy back.
+constexpr uint32_t kFew = 64;
+
+struct FewIdx {
+	uint64_t idx[kFew];
+};
+
+struct FewSet {
+	uint64_t idx[kFew];
+	double val[2 * kFew];
+};
+
+__global__ __launch_bounds__(kFew) void k_gather_few(
+	const double2 *__restrict__ a, const FewIdx I, double2 *__restrict__ out,
+	uint32_t n)
+{
+	if (threadIdx.x < n)
+		out[threadIdx.x] = a[I.idx[threadIdx.x]];
+}
+
+__global__ __launch_bounds__(kFew) void k_scatter_few(
+	double2 *__restrict__ a, const FewSet S, uint32_t n)
+{
+	const uint32_t t = threadIdx.x;
+	if (t < n)
+		a[S.idx[t]] = make_double2(S.val[2 * t], S.val[2 * t + 1]);
+}
+
 __global__ __launch_bounds__(kBlock) void k_scatter_set(
 	double2 *__restrict__ a, const uint64_t *__restrict__ idx,
 	const double2 *__restrict__ val, uint64_t n)
@@ -1479,12 +1573,51 @@ int prof_end(hipEvent_t stop)
 	return 0;
 }
 
+// Pinned host memory that kernels read indices from and write small results
+// to: a result of a few amplitudes then costs one launch and one wait (11 us
+// measured) instead of two allocations, two copies, a launch and a wait
+// (27 us).  One block per process, used by one call at a time (the holder of
+// the lock, to the end of its wait); also covers g_red.  Released by
+// ph2hip_shutdown.
+constexpr size_t kStageN = 8192;      // indices or amplitudes of a call
+constexpr size_t kStageBytes = kStageN * 24 + 64;
+std::mutex g_stage_mu;
+char *g_stage = nullptr;
+
+// The block (nullptr if there is none); call with the lock held.
+char *stage()
+{
+	if (!g_stage && hipHostMalloc(reinterpret_cast<void **>(&g_stage),
+				kStageBytes, hipHostMallocDefault) != hipSuccess) {
+		(void)hipGetLastError();
+		g_stage = nullptr;
+	}
+	return g_stage;
+}
+
 int ensure_red()
 {
 	if (g_red)
 		return 0;
 	HIPCHK(hipMalloc(&g_red, sizeof(double2) * (kRedBlocks + 1)));
 	g_red_cap = kRedBlocks + 1;
+	return 0;
+}
+
+// Second stage of a reduction over nb partials in g_red, its result waited
+// for and copied to out (two doubles).  Call with the stage lock held.
+int reduce_out(uint32_t nb, double *out)
+{
+	double2 *partial = reinterpret_cast<double2 *>(g_red);
+	char *p = stage();
+	double2 *to = p ? reinterpret_cast<double2 *>(p) : partial + kRedBlocks;
+	hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(kBlock), 0, g_stream,
+		partial, nb, to);
+	HIPCHK(hipGetLastError());
+	if (!p)
+		return ph2hip_d2h(out, to, sizeof(double2));
+	HIPCHK(hipStreamSynchronize(g_stream));
+	memcpy(out, p, sizeof(double2));
 	return 0;
 }
 
@@ -1785,19 +1918,28 @@ int build_pass_mode(FusedPass &P, const struct ph2hip_rot *r, size_t len,
 	uint32_t gk[PH2HIP_PASS_MAX + 1];   // group boundaries
 	uint32_t sup[PH2HIP_PASS_MAX];      // tile bits touched by each span
 	for (size_t k = 0; k < len;) {
-		size_t e = k + 1;
-		uint32_t u[8];
-		while (e < len && reduce32(xt + k, e + 1 - k, u, D) <= D)
-			e++;
-		const uint32_t d = reduce32(xt + k, e - k, u, D);
-		uint32_t sp = 0;
-		for (uint32_t m = 0; m < (1u << d); m++) {
-			uint32_t v = 0;
+		// extend the group while its span has at most D dimensions
+		size_t e = k;
+		uint32_t u[8], d = 0;
+		for (; e < len; e++) {
+			uint32_t x = xt[e];
+			for (uint32_t i = 0; i < d && x; i++)
+				if (x >> (31 - __builtin_clz(u[i])) & 1)
+					x ^= u[i];
+			if (!x)
+				continue;
+			if (d == D)
+				break;
+			const int p = 31 - __builtin_clz(x);
 			for (uint32_t i = 0; i < d; i++)
-				if (m >> i & 1)
-					v ^= u[i];
-			sp |= v;
+				if (u[i] >> p & 1)
+					u[i] ^= x;
+			u[d++] = x;
 		}
+		// every bit of a basis vector is a bit of some vector of the span
+		uint32_t sp = 0;
+		for (uint32_t i = 0; i < d; i++)
+			sp |= u[i];
 		gk[ng] = (uint32_t)k;
 		sup[ng++] = sp;
 		k = e;
@@ -2203,11 +2345,18 @@ uint64_t g_replay_clock = 0, g_replay_hits = 0;
 bool g_replay_init = false;
 uint32_t g_replay_max_qb = 20;
 
-uint64_t fnv_bytes(uint64_t h, const void *p, size_t n)
+// FNV-1a over 64-bit words (a byte at a time took 20 us for 537 terms, as
+// much as two passes of a 16-qubit sweep); n is a multiple of 4.  Only a
+// filter: matches are compared in full.
+uint64_t fnv_words(uint64_t h, const void *p, size_t n)
 {
 	const unsigned char *b = static_cast<const unsigned char *>(p);
-	for (size_t i = 0; i < n; i++)
-		h = (h ^ b[i]) * UINT64_C(0x100000001b3);
+	for (size_t i = 0; i < n; i += 8) {
+		uint64_t w = 0;
+		memcpy(&w, b + i, n - i < 8 ? 4 : 8);
+		h = (h ^ w) * UINT64_C(0x100000001b3);
+		h ^= h >> 32;
+	}
 	return h;
 }
 
@@ -2242,10 +2391,10 @@ bool replay_same(const ReplaySlot &r, uint64_t key, void *amp, uint32_t nqb,
 ReplaySlot *replay_slot(void *amp, uint32_t nqb, const struct ph2hip_rot *rot,
 	size_t n, const uint32_t *const sch[3], size_t npass, bool *seen)
 {
-	uint64_t key = fnv_bytes(UINT64_C(0xcbf29ce484222325), rot,
+	uint64_t key = fnv_words(UINT64_C(0xcbf29ce484222325), rot,
 		sizeof *rot * n);
 	for (int a = 0; a < 3; a++)
-		key = fnv_bytes(key, sch[a], sizeof(uint32_t) * npass);
+		key = fnv_words(key, sch[a], sizeof(uint32_t) * npass);
 	ReplaySlot *old = &g_replay[0];
 	for (ReplaySlot &r : g_replay) {
 		if (replay_same(r, key, amp, nqb, rot, n, sch, npass)) {
@@ -2507,9 +2656,15 @@ void ph2hip_shutdown(void)
 	for (ReplaySlot &r : g_replay)
 		replay_clear(r);
 	rg_clear();
-	if (g_red)
-		(void)hipFree(g_red);
-	g_red = nullptr;
+	{
+		std::lock_guard<std::mutex> lock(g_stage_mu);
+		if (g_red)
+			(void)hipFree(g_red);
+		g_red = nullptr;
+		if (g_stage)
+			(void)hipHostFree(g_stage);
+		g_stage = nullptr;
+	}
 	(void)hipStreamDestroy(g_stream);
 	g_stream = nullptr;
 }
@@ -2614,6 +2769,42 @@ int ph2hip_rotate_plain(void *amp, uint32_t nqb, const struct ph2hip_rot *rot,
 		}
 		if (rc || prof_end(stop))
 			return -1;
+	}
+	return 0;
+}
+
+int ph2hip_rotate_small(void *amp, uint32_t nqb, const struct ph2hip_rot *rot,
+	size_t n)
+{
+	if (ensure_init())
+		return -1;
+	if (nqb == 0 || nqb > kSmallQb)
+		return fail("rotate_small: nqb=%u outside 1..%u", nqb, kSmallQb);
+	for (size_t k = 0; k < n; k++)
+		if (rot[k].x >> nqb)
+			return fail("rotate_small: term %zu flips qubit >= %u", k,
+				nqb);
+	if (g_prof)   // one record per term, as the plain sweep keeps them
+		return ph2hip_rotate_plain(amp, nqb, rot, n);
+	for (size_t k0 = 0; k0 < n; k0 += kSmallTerms) {
+		SmallRun R;
+		R.n = (uint32_t)(n - k0 < kSmallTerms ? n - k0 : kSmallTerms);
+		for (uint32_t k = 0; k < R.n; k++) {
+			const struct ph2hip_rot &r = rot[k0 + k];
+			SmallTerm &T = R.t[k];
+			T.c = r.c;
+			T.s = r.s;
+			T.x = (uint16_t)r.x;
+			// phase bits beyond the register meet no index bit
+			T.z = (uint16_t)(r.z & ((UINT64_C(1) << nqb) - 1));
+			T.h = r.x ? (uint8_t)top_bit(r.x) : 0;
+			T.y = (uint8_t)(__builtin_popcountll(r.x & r.z) & 3);
+			T.pad = 0;
+		}
+		hipLaunchKernelGGL(k_rot_small, dim3(1),
+			dim3(1u << (kSmallQb - 1)), 0, g_stream, (double2 *)amp,
+			nqb, R);
+		HIPCHK(hipGetLastError());
 	}
 	return 0;
 }
@@ -2773,6 +2964,32 @@ int ph2hip_gather(const void *amp, uint32_t nqb, const uint64_t *idx,
 		if (idx[k] >= namp)
 			return fail("gather: index %llu beyond 2^%u",
 				(unsigned long long)idx[k], nqb);
+	if (n <= kStageN) {
+		std::lock_guard<std::mutex> lock(g_stage_mu);
+		if (char *p = stage()) {
+			double2 *res = reinterpret_cast<double2 *>(p);
+			if (n <= kFew) {
+				FewIdx I;
+				memset(&I, 0, sizeof I);
+				memcpy(I.idx, idx, sizeof(uint64_t) * n);
+				hipLaunchKernelGGL(k_gather_few, dim3(1),
+					dim3(kFew), 0, g_stream,
+					(const double2 *)amp, I, res, (uint32_t)n);
+			} else {
+				uint64_t *in = reinterpret_cast<uint64_t *>(p +
+					sizeof(double2) * kStageN);
+				memcpy(in, idx, sizeof(uint64_t) * n);
+				hipLaunchKernelGGL(k_gather,
+					dim3(grid_for(n, kBlock, kMaxGrid)),
+					dim3(kBlock), 0, g_stream,
+					(const double2 *)amp, in, res, (uint64_t)n);
+			}
+			HIPCHK(hipGetLastError());
+			HIPCHK(hipStreamSynchronize(g_stream));
+			memcpy(out, p, sizeof(double2) * n);
+			return 0;
+		}
+	}
 	uint64_t *didx = nullptr;
 	double2 *dout = nullptr;
 	HIPCHK(hipMalloc(&didx, sizeof(uint64_t) * n));
@@ -2942,7 +3159,10 @@ int ph2hip_sc_scatter(void *amp, uint32_t nqb, const struct ph2hip_sc *sc,
 int ph2hip_sc_inner(const void *amp, uint32_t nqb, const struct ph2hip_sc *sc,
 	uint32_t n_sites, double weight, int tapered, double *out)
 {
-	if (ensure_init() || sc_check(sc, nqb, n_sites, tapered) || ensure_red())
+	if (ensure_init() || sc_check(sc, nqb, n_sites, tapered))
+		return -1;
+	std::lock_guard<std::mutex> lock(g_stage_mu);
+	if (ensure_red())
 		return -1;
 	const uint64_t total = (uint64_t)sc->Ma * sc->Mb;
 	const uint32_t nb = grid_for(total, kBlock, kRedBlocks);
@@ -2952,10 +3172,7 @@ int ph2hip_sc_inner(const void *amp, uint32_t nqb, const struct ph2hip_sc *sc,
 		(uint64_t)sc->Ma, (uint64_t)sc->Mb, n_sites, weight, tapered,
 		partial);
 	HIPCHK(hipGetLastError());
-	hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(kBlock), 0, g_stream,
-		partial, nb, partial + kRedBlocks);
-	HIPCHK(hipGetLastError());
-	return ph2hip_d2h(out, partial + kRedBlocks, sizeof(double2));
+	return reduce_out(nb, out);
 }
 
 int ph2hip_prof_enable(int on)
@@ -3114,11 +3331,18 @@ int ph2hip_sample_cdf(size_t nstream, const double *const *cdf,
 	    hipMalloc(&dout, sizeof(uint32_t) * (nout ? nout : 1)) !=
 		    hipSuccess)
 		rc = fail("sample_cdf: hipMalloc");
-	for (size_t k = 0; k < nstream && !rc; k++)
-		if (hipMemcpyAsync(dtab + hj[k].cdf_off, cdf[k],
-			    sizeof(double) * len[k], hipMemcpyHostToDevice,
-			    g_stream) != hipSuccess)
-			rc = fail("sample_cdf: copy of table %zu", k);
+	// the tables in one copy: one at a time they cost 12 us each
+	double *htab = static_cast<double *>(malloc(sizeof(double) * ntab));
+	if (!rc && !htab)
+		rc = fail("sample_cdf: out of host memory");
+	if (!rc) {
+		for (size_t k = 0; k < nstream; k++)
+			memcpy(htab + hj[k].cdf_off, cdf[k],
+				sizeof(double) * len[k]);
+		if (hipMemcpyAsync(dtab, htab, sizeof(double) * ntab,
+			    hipMemcpyHostToDevice, g_stream) != hipSuccess)
+			rc = fail("sample_cdf: copy of the tables");
+	}
 	if (!rc && hipMemcpyAsync(dj, hj, sizeof(DrawJob) * nstream,
 			   hipMemcpyHostToDevice, g_stream) != hipSuccess)
 		rc = fail("sample_cdf: copy of the streams");
@@ -3143,13 +3367,17 @@ int ph2hip_sample_cdf(size_t nstream, const double *const *cdf,
 	(void)hipFree(dtab);
 	(void)hipFree(dj);
 	(void)hipFree(dout);
+	free(htab);
 	free(hj);
 	return rc;
 }
 
 int ph2hip_norm2(const void *amp, uint32_t nqb, double *out)
 {
-	if (ensure_init() || ensure_red())
+	if (ensure_init())
+		return -1;
+	std::lock_guard<std::mutex> lock(g_stage_mu);
+	if (ensure_red())
 		return -1;
 	const uint64_t namp = UINT64_C(1) << nqb;
 	const uint32_t nb = grid_for(namp, kBlock * 8, kRedBlocks);
@@ -3157,11 +3385,8 @@ int ph2hip_norm2(const void *amp, uint32_t nqb, double *out)
 	hipLaunchKernelGGL(k_norm2, dim3(nb), dim3(kBlock), 0, g_stream,
 		(const double2 *)amp, namp, partial);
 	HIPCHK(hipGetLastError());
-	hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(kBlock), 0, g_stream,
-		partial, nb, partial + kRedBlocks);
-	HIPCHK(hipGetLastError());
 	double r[2];
-	if (ph2hip_d2h(r, partial + kRedBlocks, sizeof r))
+	if (reduce_out(nb, r))
 		return -1;
 	*out = r[0];
 	return 0;
@@ -3181,7 +3406,10 @@ int ph2hip_fill_hash(void *amp, uint64_t namp, uint64_t seed)
 int ph2hip_count_unequal(const void *a, const void *b, uint64_t namp,
 	uint64_t *count)
 {
-	if (ensure_init() || ensure_red())
+	if (ensure_init())
+		return -1;
+	std::lock_guard<std::mutex> lock(g_stage_mu);
+	if (ensure_red())
 		return -1;
 	unsigned long long *dc = (unsigned long long *)g_red;
 	hipLaunchKernelGGL(k_fill, dim3(1), dim3(kBlock), 0, g_stream,
@@ -3450,6 +3678,27 @@ int ph2hip_scatter_set(void *amp, uint64_t namp_total, const uint64_t *idx,
 			return fail("scatter_set: index %llu beyond %llu",
 				(unsigned long long)idx[k],
 				(unsigned long long)namp_total);
+	if (n <= kFew) {
+		// as kernel arguments, nothing to wait for; later entries win
+		FewSet S;
+		memset(&S, 0, sizeof S);
+		uint32_t m = 0;
+		for (size_t k = 0; k < n; k++) {
+			size_t j = k + 1;
+			while (j < n && idx[j] != idx[k])
+				j++;
+			if (j < n)
+				continue;
+			S.idx[m] = idx[k];
+			S.val[2 * m] = val[2 * k];
+			S.val[2 * m + 1] = val[2 * k + 1];
+			m++;
+		}
+		hipLaunchKernelGGL(k_scatter_few, dim3(1), dim3(kFew), 0,
+			g_stream, (double2 *)amp, S, m);
+		HIPCHK(hipGetLastError());
+		return 0;
+	}
 	// later entries win: keep the last occurrence of every index
 	size_t *ord = (size_t *)malloc(sizeof(size_t) * n);
 	uint64_t *ui = (uint64_t *)malloc(sizeof(uint64_t) * n);
@@ -3472,6 +3721,25 @@ int ph2hip_scatter_set(void *amp, uint64_t namp_total, const uint64_t *idx,
 		uv[2 * m] = val[2 * ord[k]];
 		uv[2 * m + 1] = val[2 * ord[k] + 1];
 		m++;
+	}
+	if (m <= kStageN) {
+		std::lock_guard<std::mutex> lock(g_stage_mu);
+		if (char *p = stage()) {
+			uint64_t *pi = reinterpret_cast<uint64_t *>(p +
+				sizeof(double2) * kStageN);
+			memcpy(p, uv, sizeof(double2) * m);
+			memcpy(pi, ui, sizeof(uint64_t) * m);
+			free(ord);
+			free(ui);
+			free(uv);
+			hipLaunchKernelGGL(k_scatter_set,
+				dim3(grid_for(m, kBlock, kMaxGrid)), dim3(kBlock),
+				0, g_stream, (double2 *)amp, pi,
+				reinterpret_cast<const double2 *>(p), (uint64_t)m);
+			HIPCHK(hipGetLastError());
+			HIPCHK(hipStreamSynchronize(g_stream));
+			return 0;
+		}
 	}
 	uint64_t *di = nullptr;
 	double2 *dv = nullptr;

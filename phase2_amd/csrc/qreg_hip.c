@@ -29,14 +29,32 @@
 #include "phase2/world.h"
 #include "phase2_hip.h"
 
+/* A block of rotations as the register last saw it: its codes and angles,
+ * and from them the rotations with their sines and cosines and the greedy
+ * schedule.  A Trotter step applies the same blocks every step; for 1024
+ * terms the sines take 15 us and the schedule 10, and the device of a
+ * narrow register waits for them. */
+#define BLOCKS 8
+#define BLOCK_MAX 4096	/* larger ones share the first slot */
+struct block {
+	size_t n, cap;
+	struct paulis *codes;
+	double *phis;
+	struct ph2hip_rot *rot;
+	struct ph2_sched sched;
+	int scheduled;	/* sched is the greedy one of the settings below */
+	uint32_t tile, low, half;
+	uint64_t used;
+};
+
 struct qreg_hip {
 	void *damp;
 	int err;
 	int mode;
 	uint32_t tile_bits, low_bits;
-	struct ph2hip_rot *rot;
-	size_t rot_cap;
-	struct ph2_sched sched;
+	struct block blocks[BLOCKS];	/* least recently used out */
+	uint64_t clock;
+	struct ph2_sched sched;		/* of a schedule function */
 	/* state a caller above the register keeps with it (the multidet
 	 * overlap plan of circ.c), released by qreg_free */
 	void *aux;
@@ -49,6 +67,7 @@ struct qreg_hip {
 	 * holds them with the queued writes applied; win_n = 0: none */
 	double *win;
 	uint64_t win_lo, win_n;
+	int reads;	/* single reads since the buffer last changed */
 };
 
 /* One amplitude moved by itself costs a synchronous device copy (about
@@ -163,6 +182,7 @@ void ph2_sched_install(ph2_sched_fn fn, void *ctx)
 static int settle(struct qreg_hip *h, uint64_t namp)
 {
 	h->win_n = 0;
+	h->reads = 0;
 	if (h->nq == 0)
 		return 0;
 	const int rc = ph2hip_scatter_set(h->damp, namp, h->qidx, h->qval,
@@ -202,9 +222,11 @@ int qreg_error(const struct qreg *reg)
 	/* a queued write fails, if at all, when it lands: land it now */
 	if (h->nq) {
 		const uint64_t lo = h->win_lo, n = h->win_n;
+		const int reads = h->reads;
 		settle(h, reg->namp);
 		h->win_lo = lo;
 		h->win_n = n;
+		h->reads = reads;
 	}
 	return h->err;
 }
@@ -285,7 +307,12 @@ void qreg_free(struct qreg *reg)
 		if (h->aux && h->aux_free)
 			h->aux_free(h->aux);
 		ph2hip_free(h->damp);
-		free(h->rot);
+		for (int i = 0; i < BLOCKS; i++) {
+			free(h->blocks[i].codes);
+			free(h->blocks[i].phis);
+			free(h->blocks[i].rot);
+			ph2_sched_free(&h->blocks[i].sched);
+		}
 		ph2_sched_free(&h->sched);
 		free(h->qidx);
 		free(h->qval);
@@ -318,8 +345,21 @@ void qreg_getamp(struct qreg *reg, uint64_t i, _Complex double *z)
 	if (!in_range(reg, i, "qreg_getamp"))
 		return;
 	if (!h->win_n || i - h->win_lo >= h->win_n) {
+		const int reads = h->reads;
 		if (settle(h, reg->namp) < 0)
 			return;
+		/* the first read after a change is often the only one: it
+		 * takes the amplitude alone (11 us), the next the window
+		 * (30 us) */
+		h->reads = reads + 1;
+		if (reads == 0) {
+			double v[2];
+			if (ph2hip_gather(h->damp, reg->qb_lo, &i, 1, v) < 0)
+				set_err(reg, "qreg_getamp");
+			else
+				*z = CMPLX(v[0], v[1]);
+			return;
+		}
 		if (!h->win && !(h->win = malloc(AMP_WIN * 16))) {
 			log_error("qreg_getamp: alloc");
 			h->err = -1;
@@ -384,6 +424,7 @@ void qreg_zero(struct qreg *reg)
 	struct qreg_hip *h = reg->backend;
 	h->nq = 0; /* every queued write would be overwritten */
 	h->win_n = 0;
+	h->reads = 0;
 	if (ph2hip_zero(h->damp, reg->namp) < 0)
 		set_err(reg, "qreg_zero");
 }
@@ -399,6 +440,7 @@ void qreg_sync_host_to_device(struct qreg *reg)
 	}
 	h->nq = 0; /* every queued write would be overwritten */
 	h->win_n = 0;
+	h->reads = 0;
 	if (ph2hip_h2d(h->damp, reg->amp, reg->namp * 16) < 0)
 		set_err(reg, "qreg_sync_host_to_device");
 }
@@ -418,6 +460,83 @@ void qreg_sync_device_to_host(struct qreg *reg)
 		set_err(reg, "qreg_sync_device_to_host");
 }
 
+/* The block of these codes and angles: an earlier one, compared in full, or
+ * the least recently used one made theirs.  NULL: out of memory. */
+static struct block *block_of(struct qreg_hip *h, const struct paulis *codes,
+	const double *phis, size_t n)
+{
+	struct block *old = &h->blocks[0];
+	for (int i = 0; i < BLOCKS; i++) {
+		struct block *b = &h->blocks[i];
+		if (b->used && b->n == n &&
+		    memcmp(b->phis, phis, sizeof *phis * n) == 0 &&
+		    memcmp(b->codes, codes, sizeof *codes * n) == 0) {
+			b->used = ++h->clock;
+			return b;
+		}
+		if (b->used < old->used)
+			old = b;
+	}
+	if (n > BLOCK_MAX)
+		old = &h->blocks[0];
+	old->used = 0;
+	old->scheduled = 0;
+	if (n > old->cap) {
+		free(old->codes);
+		free(old->phis);
+		free(old->rot);
+		old->codes = malloc(sizeof *old->codes * n);
+		old->phis = malloc(sizeof *old->phis * n);
+		old->rot = malloc(sizeof *old->rot * n);
+		old->cap = old->codes && old->phis && old->rot ? n : 0;
+		if (!old->cap)
+			return NULL;
+	}
+	memcpy(old->codes, codes, sizeof *codes * n);
+	memcpy(old->phis, phis, sizeof *phis * n);
+	for (size_t k = 0; k < n; k++) {
+		old->rot[k].x = codes[k].pak[0];
+		old->rot[k].z = codes[k].pak[1];
+		sincos(phis[k], &old->rot[k].s, &old->rot[k].c);
+	}
+	old->n = n;
+	old->used = ++h->clock;
+	return old;
+}
+
+/* The fused sweep of a block: the schedule function's cut, else greedy. */
+static int rotate_block(struct qreg_hip *h, uint32_t nqb, struct block *b)
+{
+	const struct ph2_sched *s = &h->sched;
+	int rc = -1;
+	if (g_sched_fn)
+		rc = g_sched_fn(g_sched_ctx, b->rot, b->n, nqb, &h->sched);
+	if (rc < 0) {
+		const uint32_t tile = h->tile_bits ? h->tile_bits :
+			auto_tile(nqb);
+		const uint32_t low = h->tile_bits ? h->low_bits :
+			auto_low(nqb, h->low_bits);
+		/* the cut at tile 13 depends on the half-tile setting */
+		const uint32_t half = ph2hip_fused_half_mask();
+		s = &b->sched;
+		rc = 0;
+		if (!b->scheduled || b->tile != tile || b->low != low ||
+		    b->half != half) {
+			b->scheduled = 0;
+			rc = ph2_sched_greedy(b->rot, b->n, nqb, tile, low,
+				&b->sched);
+			b->tile = tile;
+			b->low = low;
+			b->half = half;
+			b->scheduled = rc == 0;
+		}
+	}
+	if (rc == 0)
+		rc = ph2hip_rotate_fused(h->damp, nqb, b->rot, b->n, s->len,
+			s->tile_bits, s->npass, s->low_bits);
+	return rc;
+}
+
 void qreg_paulirot(struct qreg *reg, struct paulis code_hi,
 	const struct paulis *codes_lo, const double *phis, size_t ncodes)
 {
@@ -431,40 +550,20 @@ void qreg_paulirot(struct qreg *reg, struct paulis code_hi,
 		return;
 	if (settle(h, reg->namp) < 0)
 		return;
-	if (ncodes > h->rot_cap) {
-		struct ph2hip_rot *r = realloc(h->rot, sizeof *r * ncodes);
-		if (!r) {
-			log_error("qreg_paulirot: alloc");
-			h->err = -1;
-			return;
-		}
-		h->rot = r;
-		h->rot_cap = ncodes;
-	}
-	for (size_t k = 0; k < ncodes; k++) {
-		h->rot[k].x = codes_lo[k].pak[0];
-		h->rot[k].z = codes_lo[k].pak[1];
-		sincos(phis[k], &h->rot[k].s, &h->rot[k].c);
+	struct block *b = block_of(h, codes_lo, phis, ncodes);
+	if (!b) {
+		log_error("qreg_paulirot: alloc");
+		h->err = -1;
+		return;
 	}
 	const uint32_t nqb = reg->qb_lo;
 	int rc;
-	if (h->mode == QREG_HIP_PLAIN || nqb < PH2HIP_TILE_MIN) {
-		rc = ph2hip_rotate_plain(h->damp, nqb, h->rot, ncodes);
-	} else {
-		rc = -1;
-		if (g_sched_fn)
-			rc = g_sched_fn(g_sched_ctx, h->rot, ncodes, nqb,
-				&h->sched);
-		if (rc < 0)
-			rc = ph2_sched_greedy(h->rot, ncodes, nqb,
-				h->tile_bits ? h->tile_bits : auto_tile(nqb),
-				h->tile_bits ? h->low_bits :
-					auto_low(nqb, h->low_bits), &h->sched);
-		if (rc == 0)
-			rc = ph2hip_rotate_fused(h->damp, nqb, h->rot, ncodes,
-				h->sched.len, h->sched.tile_bits, h->sched.npass,
-				h->sched.low_bits);
-	}
+	if (h->mode == QREG_HIP_PLAIN)
+		rc = ph2hip_rotate_plain(h->damp, nqb, b->rot, ncodes);
+	else if (nqb < PH2HIP_TILE_MIN)
+		rc = ph2hip_rotate_small(h->damp, nqb, b->rot, ncodes);
+	else
+		rc = rotate_block(h, nqb, b);
 	if (rc < 0)
 		set_err(reg, "qreg_paulirot");
 }

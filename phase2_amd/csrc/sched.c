@@ -5,6 +5,7 @@
  */
 #include <stdint.h>
 #include <stdlib.h>
+#include <string.h>
 
 #include "phase2/qreg_hip.h"
 #include "phase2_hip.h"
@@ -123,30 +124,23 @@ int ph2_sched_greedy(const struct ph2hip_rot *rot, size_t n, uint32_t nqb,
 		low_bits = tile_bits - 1;
 	const uint64_t lowmask = (UINT64_C(1) << low_bits) - 1;
 	const uint32_t gmax = tile_bits - low_bits;
-	uint64_t basis[64];
-	int piv[64];
+	uint64_t basis[64] = { 0 };	/* by leading bit */
 	uint32_t g = 0, len = 0;
 	for (size_t k = 0; k < n; k++) {
 		uint64_t v = rot[k].x & ~lowmask;
-		for (uint32_t b = 0; b < g && v; b++)
-			if (v >> piv[b] & 1)
-				v ^= basis[b];
-		const int grows = v != 0;
-		if (len == PH2HIP_PASS_MAX || (grows && g == gmax)) {
+		while (v && basis[topbit(v)])
+			v ^= basis[topbit(v)];
+		if (len == PH2HIP_PASS_MAX || (v && g == gmax)) {
 			if (push(out, rot + k - len, len, tile_bits, low_bits) <
 				0)
 				return -1;
+			memset(basis, 0, sizeof basis);
 			g = 0;
 			len = 0;
 			v = rot[k].x & ~lowmask;
 		}
 		if (v) {
-			const int p = topbit(v);
-			for (uint32_t b = 0; b < g; b++)
-				if (basis[b] >> p & 1)
-					basis[b] ^= v;
-			basis[g] = v;
-			piv[g] = p;
+			basis[topbit(v)] = v;
 			g++;
 		}
 		len++;
