@@ -216,8 +216,13 @@ void ph2hip_round_graph_stats(uint64_t *builds, uint64_t *replays);
 
 /* amp[idx[k]] = (val[2k], val[2k+1]) with idx < namp_total (host arrays);
  * for repeated indices the last entry wins, as sequential qreg_setamp
- * calls would leave it. */
+ * calls would leave it.  Returns when the values are in place. */
 int ph2hip_scatter_set(void *amp, uint64_t namp_total, const uint64_t *idx,
+	const double *val, size_t n);
+
+/* The same, queued on the library stream: the host arrays are free on
+ * return, and up to 64 values are not waited for. */
+int ph2hip_scatter_queue(void *amp, uint64_t namp_total, const uint64_t *idx,
 	const double *val, size_t n);
 
 /* out[2k], out[2k+1] = amp[idx[k]], idx < namp_total. */

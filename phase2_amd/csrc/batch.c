@@ -315,7 +315,7 @@ static int prep_round(struct batch *B, size_t r, size_t lim)
 			m++;
 		}
 	}
-	return m ? ph2hip_scatter_set(B->amp, B->namp, B->idx, B->val, m) : 0;
+	return m ? ph2hip_scatter_queue(B->amp, B->namp, B->idx, B->val, m) : 0;
 }
 
 static void set_rot(struct ph2hip_rot *o, const struct paulis op, double phi)

@@ -1588,7 +1588,7 @@ char *g_stage = nullptr;
 char *stage()
 {
 	if (!g_stage && hipHostMalloc(reinterpret_cast<void **>(&g_stage),
-				kStageBytes, hipHostMallocDefault) != hipSuccess) {
+				kStageBytes, hipHostMallocPortable) != hipSuccess) {
 		(void)hipGetLastError();
 		g_stage = nullptr;
 	}
@@ -3666,7 +3666,7 @@ int ph2hip_rotate_batched(void *amp, uint64_t namp_total,
 	return rc;
 }
 
-int ph2hip_scatter_set(void *amp, uint64_t namp_total, const uint64_t *idx,
+int ph2hip_scatter_queue(void *amp, uint64_t namp_total, const uint64_t *idx,
 	const double *val, size_t n)
 {
 	if (ensure_init())
@@ -3679,7 +3679,8 @@ int ph2hip_scatter_set(void *amp, uint64_t namp_total, const uint64_t *idx,
 				(unsigned long long)idx[k],
 				(unsigned long long)namp_total);
 	if (n <= kFew) {
-		// as kernel arguments, nothing to wait for; later entries win
+		// as kernel arguments: nothing of the caller's or the stage
+		// is read later, so nothing to wait for; later entries win
 		FewSet S;
 		memset(&S, 0, sizeof S);
 		uint32_t m = 0;
@@ -3767,6 +3768,17 @@ int ph2hip_scatter_set(void *amp, uint64_t namp_total, const uint64_t *idx,
 	free(ui);
 	free(uv);
 	return rc;
+}
+
+int ph2hip_scatter_set(void *amp, uint64_t namp_total, const uint64_t *idx,
+	const double *val, size_t n)
+{
+	if (ph2hip_scatter_queue(amp, namp_total, idx, val, n))
+		return -1;
+	if (n == 0 || n > kFew)   // a longer one has waited
+		return 0;
+	HIPCHK(hipStreamSynchronize(g_stream));
+	return 0;
 }
 
 int ph2hip_gather_abs(const void *amp, uint64_t namp_total,

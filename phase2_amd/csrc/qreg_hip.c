@@ -63,6 +63,7 @@ struct qreg_hip {
 	uint64_t *qidx;
 	double *qval;
 	size_t nq, qcap;
+	int flying;	/* writes sent to the stream and not waited for */
 	/* host copy of amplitudes [win_lo, win_lo + win_n) as the device
 	 * holds them with the queued writes applied; win_n = 0: none */
 	double *win;
@@ -185,9 +186,10 @@ static int settle(struct qreg_hip *h, uint64_t namp)
 	h->reads = 0;
 	if (h->nq == 0)
 		return 0;
-	const int rc = ph2hip_scatter_set(h->damp, namp, h->qidx, h->qval,
+	const int rc = ph2hip_scatter_queue(h->damp, namp, h->qidx, h->qval,
 		h->nq);
 	h->nq = 0;
+	h->flying = 1;
 	if (rc < 0) {
 		h->err = -1;
 		log_error("qreg_setamp: %s", ph2hip_strerror());
@@ -195,14 +197,19 @@ static int settle(struct qreg_hip *h, uint64_t namp)
 	return rc;
 }
 
-/* The caller may read or change the buffer through the pointer, so the
- * queued writes land first and the read window goes. */
+/* The caller may read or change the buffer through the pointer, on a stream
+ * of its own too, so the queued writes land first and the read window goes. */
 void *qreg_hip_device_ptr(struct qreg *reg)
 {
 	struct qreg_hip *h = reg->backend;
 	if (!h)
 		return NULL;
 	settle(h, reg->namp);
+	if (h->flying) {
+		h->flying = 0;
+		if (ph2hip_synchronize() < 0)
+			h->err = -1;
+	}
 	return h->damp;
 }
 
