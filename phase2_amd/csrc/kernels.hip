@@ -1009,9 +1009,19 @@ __device__ __forceinline__ cHead arg_head()
 // workgroup w = 8 l + x runs tile start(x) + l, where XCD x owns
 // q + (x < r) tiles (q = ntiles / 8, r = ntiles mod 8).  A bijection on
 // [0, ntiles); measured 4.5% faster per fused pass at 33 qubits than tile w.
+// From 2^14 tiles (a power of two; 27 qubits at tile 13) the ranges are 64
+// tiles long and follow each other: the XCDs then work within one window of
+// 512 tiles, on an eighth of the DRAM pages and not at equal offsets of
+// eight distant ranges.  1024-term sweeps, ranges of an eighth / of 64: 62.4
+// / 62.0 ms at 27 qubits, 130.1 / 127.8 at 28, 264.4 / 262.7 at 29, 539.8 /
+// 536.1 and 593.6 / 582.2 at 30; with fewer tiles 3324 / 3344 us at 23,
+// 6508 / 6566 at 24, 15177 / 15368 at 25.  Ranges of 16 and of 256 tiles
+// gain less (130.1 and 129.5 ms at 28).
 __device__ __forceinline__ uint64_t xcd_tile(uint64_t w, uint64_t ntiles)
 {
 	const uint64_t q = ntiles >> 3, r = ntiles & 7, x = w & 7, l = w >> 3;
+	if (ntiles >> 14)
+		return l >> 6 << 9 | x << 6 | (l & 63);
 	return x * q + (x < r ? x : r) + l;
 }
 
