@@ -1836,10 +1836,6 @@ int plain_one(double2 *a, uint32_t nqb, const struct ph2hip_rot &r)
 	return 0;
 }
 
-// Descriptor of one fused pass over terms r[0..len) (global term index k0
-// for messages) in tiles of 2^tb amplitudes.  0, or -1 if the pass does not
-// fit its tile; with half set, 1 if the pass has no half-tile form (some
-// exchange between consecutive groups has no split bit).
 // Rank over GF(2) of v[0..n) masked by m.
 uint32_t gf2_rank(const uint32_t *v, uint32_t n, uint32_t m)
 {
@@ -1869,8 +1865,72 @@ uint32_t half_bank(uint32_t t)
 	return (v ^ (v >> 4) ^ (v >> 5) ^ (v >> 7)) & 15u;
 }
 
+// The gathered coordinates of a pass in the basis of its own flip masks:
+// y[0..n) are the masks in the coordinates of the echelon basis w[0..g),
+// whose span they fill; replaces w and y.  The basis keeps the order of its
+// leading bits, so that lanes still take the lowest rows.
+void mask_basis(uint64_t *w, uint32_t g, uint32_t *y, size_t n)
+{
+	uint32_t nb[PH2HIP_TILE_MAX], row[32], m = 0;
+	memset(row, 0, sizeof row);
+	for (size_t k = 0; k < n && m < g; k++) {
+		uint32_t v = y[k];
+		while (v && row[31 - __builtin_clz(v)])
+			v ^= row[31 - __builtin_clz(v)];
+		if (v) {
+			row[31 - __builtin_clz(v)] = v;
+			nb[m++] = y[k];
+		}
+	}
+	std::sort(nb, nb + m);
+	// rows of an elimination with the basis vectors each one sums
+	uint32_t sum[32];
+	memset(row, 0, sizeof row);
+	for (uint32_t b = 0; b < m; b++) {
+		uint32_t v = nb[b], c = 1u << b;
+		while (row[31 - __builtin_clz(v)]) {
+			const int p = 31 - __builtin_clz(v);
+			v ^= row[p];
+			c ^= sum[p];
+		}
+		row[31 - __builtin_clz(v)] = v;
+		sum[31 - __builtin_clz(v)] = c;
+	}
+	for (size_t k = 0; k < n; k++) {
+		uint32_t v = y[k], c = 0;
+		while (v) {
+			const int p = 31 - __builtin_clz(v);
+			v ^= row[p];
+			c ^= sum[p];
+		}
+		y[k] = c;
+	}
+	uint64_t nw[PH2HIP_TILE_MAX];
+	for (uint32_t b = 0; b < m; b++) {
+		nw[b] = 0;
+		for (uint32_t i = 0; i < g; i++)
+			if (nb[b] >> i & 1)
+				nw[b] ^= w[i];
+	}
+	memcpy(w, nw, sizeof *w * m);
+}
+
+// Descriptor of one fused pass over terms r[0..len) (global term index k0
+// for messages) in tiles of 2^tb amplitudes.  0, or -1 if the pass does not
+// fit its tile; with half set, 1 if the pass has no half-tile form (some
+// exchange between consecutive groups has no split bit).  own: the gathered
+// tile bits stand for flip masks of the pass (mask_basis) instead of the
+// echelon basis of their span.  An independent mask then touches one tile
+// bit, so two consecutive groups rarely touch all of them; tried at tile 13
+// where the echelon basis leaves an exchange without a split bit, as dense
+// masks often do.  Such a pass was cut to keep the half-tile form: blocks
+// of 1024 random terms took 96, 91, 93 and 80 passes at 22, 24, 25 and 28
+// qubits (low 2) and 2492, 9441, 20354 and 152604 us, and take 79, 76, 76
+// and 73 passes and 2143, 8278, 17180 and 142041 us.  Tile 12 has a
+// whole-tile form as fast (two 64 KiB workgroups per CU): with it 0.97 to
+// 1.02 of the time, so it stays.
 int build_pass_mode(FusedPass &P, const struct ph2hip_rot *r, size_t len,
-	uint32_t tb, uint32_t low_bits, size_t k0, bool half)
+	uint32_t tb, uint32_t low_bits, size_t k0, bool half, bool own = false)
 {
 	memset(&P, 0, sizeof P);
 	// Grow the contiguous low part L while the gathered rank g fits:
@@ -1892,29 +1952,34 @@ int build_pass_mode(FusedPass &P, const struct ph2hip_rot *r, size_t len,
 	P.L = (uint8_t)L;
 	P.g = (uint8_t)g;
 	P.nterms = (uint8_t)len;
-	for (uint32_t b = 0; b < g; b++) {
-		P.w[b] = w[b];
+	for (uint32_t b = 0; b < g; b++)
 		P.piv[b] = (uint8_t)top_bit(w[b]);
-	}
 	const uint64_t lm = (UINT64_C(1) << L) - 1;
 	uint32_t xt[PH2HIP_PASS_MAX];
 	for (size_t k = 0; k < len; k++) {
-		const uint64_t x = r[k].x, z = r[k].z;
-		uint32_t xk = (uint32_t)(x & lm), zk = (uint32_t)(z & lm);
-		uint64_t rest = x & ~lm;
-		for (uint32_t b = 0; b < g; b++) {
-			if (x >> P.piv[b] & 1) {
-				xk |= 1u << (L + b);
+		uint64_t rest = r[k].x & ~lm;
+		xt[k] = 0;
+		for (uint32_t b = 0; b < g; b++)
+			if (r[k].x >> P.piv[b] & 1) {
+				xt[k] |= 1u << b;
 				rest ^= w[b];
 			}
-			if (__builtin_popcountll(w[b] & z) & 1)
-				zk |= 1u << (L + b);
-		}
 		if (rest) {
 			return fail("rotate_fused: term %zu outside its tile",
 				k0 + k);
 		}
-		xt[k] = xk;
+	}
+	if (own)
+		mask_basis(w, g, xt, len);
+	for (uint32_t b = 0; b < g; b++)
+		P.w[b] = w[b];
+	for (size_t k = 0; k < len; k++) {
+		const uint64_t x = r[k].x, z = r[k].z;
+		uint32_t zk = (uint32_t)(z & lm);
+		for (uint32_t b = 0; b < g; b++)
+			if (__builtin_popcountll(w[b] & z) & 1)
+				zk |= 1u << (L + b);
+		xt[k] = xt[k] << L | (uint32_t)(x & lm);
 		FusedTerm &T = P.t[k];
 		T.z = z;
 		T.zt = zk;
@@ -1965,8 +2030,9 @@ int build_pass_mode(FusedPass &P, const struct ph2hip_rot *r, size_t len,
 	if (half) {
 		for (uint32_t q = 0; q + 1 < ng; q++) {
 			const uint32_t fr = ((1u << tb) - 1) & ~(sup[q] | sup[q + 1]);
-			if (!fr)
-				return 1;   // no split bit: not a half-tile pass
+			if (!fr)            // no split bit
+				return own || tb < 13 ? 1 : build_pass_mode(P, r,
+					len, tb, low_bits, k0, true, true);
 			uint32_t h;
 			if (q > 0 && (fr >> xh[q - 1] & 1)) {
 				h = xh[q - 1];
@@ -2019,7 +2085,9 @@ int build_pass_mode(FusedPass &P, const struct ph2hip_rot *r, size_t len,
 			u[d++] = x;
 		}
 		if (d < D)
-			return half ? 1 : fail("rotate_fused: group padding");
+			return !half ? fail("rotate_fused: group padding") :
+				own || tb < 13 ? 1 : build_pass_mode(P, r, len,
+					tb, low_bits, k0, true, true);
 		for (uint32_t i = 1; i < d; i++)   // ascending pivots
 			for (uint32_t j = i; j > 0 && __builtin_clz(u[j - 1]) <
 				__builtin_clz(u[j]); j--) {

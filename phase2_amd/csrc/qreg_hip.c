@@ -43,6 +43,7 @@ struct block {
 	struct ph2hip_rot *rot;
 	struct ph2_sched sched;
 	int scheduled;	/* sched is the greedy one of the settings below */
+	int chosen;	/* the tile and low bits are automatic */
 	uint32_t tile, low, half;
 	uint64_t used;
 };
@@ -89,46 +90,58 @@ static uint32_t g_tile = 0, g_low = 3;
 static ph2_sched_fn g_sched_fn;
 static void *g_sched_ctx;
 
-/* Tile width when none is set, from 1024-term blocks of lex-ordered sweeps
- * timed at every tile width (us per block at the widths beside each line):
- *   to 18 qubits, tile 10: 300, 349 and 416 at 13, 16 and 18 qubits
- *     against 323, 369 and 421 at tile 11.  A few dozen workgroups, bound
- *     by each pass's chain of terms and exchanges;
- *   19 to 21, tile 11: 464, 676, 997 at 19, 20, 21 against 521, 786, 1257
- *     at tile 10 and 609, 722, 1047 at tile 12;
- *   22 and 23, tile 12: 1730 and 3371 against 1991 and 3749 at tile 11 and
- *     1770 and 3385 at tile 13;
- *   from 24, tile 13: 6748 and 15112 at 24 and 25 against 6841 and 17452 at
- *     tile 12.  HBM traffic per pass weighs most and wider tiles need fewer
- *     passes.
+/* Tile width when none is set, from 1024-term blocks timed at every tile
+ * width, lex-ordered sweeps and random draws (us per block, sweep / draw):
+ *   to 18 qubits, tile 10: 346 / 366 at 16 qubits and 405 / 450 at 18
+ *     against 367 / 404 and 415 / 474 at tile 11, 118 against 147 at tile 9
+ *     at 10 qubits.  A few dozen workgroups, bound by each pass's chain of
+ *     terms and exchanges;
+ *   19 to 21, tile 11: 674 / 853 at 20 and 988 / 894 at 21 against
+ *     781 / 910 and 1205 / 1003 at tile 10, 721 / 896 and 1034 / 991 at 12;
+ *   from 22, tile 13: 1732 / 1467 at 22, 6404 / 4707 at 24, 14744 / 9765 at
+ *     25, 128310 / 75068 at 28 against 1773 / 1489, 6755 / 4825, 16834 /
+ *     9901 and 143945 / 77109 at tile 12.  Traffic per pass weighs most and
+ *     wider tiles need fewer passes.
  * Without replay of captured sweeps (ph2hip_replay_max_qb, 20 qubits by
  * default) launches weigh more below: 12 from 17 qubits, nqb - 5 under
  * that (at 16 qubits a Trotter step took 0.476 ms at tile 11, 0.503 at 10,
- * 0.532 at 9 and 0.564 at 12).  Never above nqb - 2 in the replayed
- * range. */
+ * 0.532 at 9 and 0.564 at 12). */
 static uint32_t auto_tile(uint32_t nqb)
 {
 	uint32_t t;
 	if (nqb <= ph2hip_replay_max_qb()) {
-		t = nqb >= 19 ? 11 : 10;
-		if (t + 2 > nqb)
-			t = nqb > 2 ? nqb - 2 : 0;
+		t = nqb >= 22 ? 13 : nqb >= 19 ? 11 : 10;
+		if (t > nqb)
+			t = nqb;
 	} else {
-		t = nqb >= 24 ? 13 : nqb == 21 ? 11 : nqb > 16 ? 12 :
+		t = nqb >= 22 ? 13 : nqb == 21 ? 11 : nqb > 16 ? 12 :
 			(nqb > 5 ? nqb - 5 : 0);
 	}
 	return t < PH2HIP_TILE_MIN ? PH2HIP_TILE_MIN : t;
 }
 
 /* Contiguous low bits the cut asks for under the automatic tile width: at
- * most `low`, and 2 from 24 qubits, where rows of 64 bytes leave one more
- * dimension to gather.  Same sweeps, low 2 against 3 at tile 13: 6547 and
- * 6748 us at 24 qubits, 14874 and 15112 at 25, 62623 and 63233 at 27,
- * 130562 and 134986 at 28, 538698 and 551383 at 30; low 1 is slower from
- * 30.  Below 24 qubits the two are within 1%. */
-static uint32_t auto_low(uint32_t nqb, uint32_t low)
+ * most `low`, and at most 2, where rows of 64 bytes leave one more
+ * dimension to gather than rows of 128.  Low 2 against 3: random draws 366
+ * and 393 us at 16 qubits, 450 and 493 at 18, 850 and 918 at 20; sweeps 346
+ * and 348, 406 and 415, 673 and 675; 6547 and 6748 at 24, 130562 and 134986
+ * at 28.  Low 1 is slower from 30. */
+static uint32_t auto_low(uint32_t low)
 {
-	return nqb >= 24 && low > 2 ? 2 : low;
+	return low > 2 ? 2 : low;
+}
+
+/* Up to 18 qubits the state lies in the L2s, where short rows cost less
+ * than passes: with no low bits asked for, sweeps (whose masks have an even
+ * number of flips, so that single low bits are dimensions none of them
+ * needs) take a third fewer passes and 324 us instead of 347 at 16 qubits,
+ * 290 / 311 at 14, 389 / 405 at 18, but random draws a fifth fewer and 378
+ * instead of 366, 392 / 368 and 471 / 450.  So both cuts are made, and the
+ * one without low bits is taken if it saves a quarter of the passes; to 12
+ * qubits always (271 / 281 and 211 / 218). */
+static int no_low(uint32_t nqb, size_t passes, size_t passes0)
+{
+	return nqb <= 12 || 4 * passes0 <= 3 * passes;
 }
 
 static void load_defaults(void)
@@ -522,19 +535,28 @@ static int rotate_block(struct qreg_hip *h, uint32_t nqb, struct block *b)
 		const uint32_t tile = h->tile_bits ? h->tile_bits :
 			auto_tile(nqb);
 		const uint32_t low = h->tile_bits ? h->low_bits :
-			auto_low(nqb, h->low_bits);
+			auto_low(h->low_bits);
 		/* the cut at tile 13 depends on the half-tile setting */
 		const uint32_t half = ph2hip_fused_half_mask();
 		s = &b->sched;
 		rc = 0;
 		if (!b->scheduled || b->tile != tile || b->low != low ||
-		    b->half != half) {
+		    b->half != half || b->chosen != !h->tile_bits) {
 			b->scheduled = 0;
 			rc = ph2_sched_greedy(b->rot, b->n, nqb, tile, low,
 				&b->sched);
+			if (rc == 0 && !h->tile_bits && nqb <= 18 && low > 0 &&
+			    (rc = ph2_sched_greedy(b->rot, b->n, nqb, tile, 0,
+				     &h->sched)) == 0 &&
+			    no_low(nqb, b->sched.npass, h->sched.npass)) {
+				const struct ph2_sched t = b->sched;
+				b->sched = h->sched;
+				h->sched = t;
+			}
 			b->tile = tile;
 			b->low = low;
 			b->half = half;
+			b->chosen = !h->tile_bits;
 			b->scheduled = rc == 0;
 		}
 	}
