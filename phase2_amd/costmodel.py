@@ -221,7 +221,7 @@ def collect(reg, xm, zm, phi, blocks, rng, log=print):
         s = slice(b * 1024, (b + 1) * 1024)
         bx, bz, bp = (np.ascontiguousarray(xm[s]), np.ascontiguousarray(zm[s]),
                       np.ascontiguousarray(phi[s]))
-        lens, tbs, lbs = random_schedule(bx, rng)
+        lens, tbs, lbs = random_schedule(bx, rng, lows=(2, 3, 4, 5))
         rc = L.ph2_reg_rotate_sched(
             C.c_void_p(reg.h), C.c_size_t(len(bx)),
             bx.ctypes.data_as(C.POINTER(C.c_uint64)),
@@ -294,7 +294,8 @@ def load(path=PARAMS_PATH):
 
 def install(params, low=3, min_qb=26):
     """Use the learned schedule for fused registers of >= min_qb qubits
-    (passes with low .. low + 2 contiguous low bits)."""
+    (passes with three counts of contiguous low bits: from low - 1, or from
+    low itself if it is 2 or less)."""
     p = np.ascontiguousarray(params, np.float32)
     if p.size != n_params():
         raise ValueError(f"{p.size} parameters, the network has "

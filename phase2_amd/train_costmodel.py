@@ -4,7 +4,7 @@
     python -m phase2_amd.train_costmodel --out DIR --eval-only PARAMS
 
 1. Records: random cuts (phase2_amd.costmodel.random_schedule: random pass
-   length, tile width 12/13 and 3..5 contiguous low bits per pass) of
+   length, tile width 12/13 and 2..5 contiguous low bits per pass) of
    1024-term blocks of lexicographically sorted synthetic Hamiltonians at 28
    (two seeds), 30 and 33 qubits, timed per pass with HIP events
    (ph2hip_prof_records), plus any record files given with --extra-records.
