@@ -14,9 +14,10 @@
  * Defaults come from PHASE2_HIP_MODE (plain|fused), PHASE2_HIP_TILE (tile
  * bits, 9..13) and PHASE2_HIP_LOW (contiguous low bits); otherwise fused,
  * automatic tile width and 3.  Tile width 0 (the automatic one) is 13 from
- * 22 qubits, 11 from 19, 10 below (at least 9); it also lowers the
- * contiguous low bits to 2, and to 0 up to 18 qubits for blocks that this
- * saves a quarter of their passes.  Fused registers narrower than 9 qubits take ph2hip_rotate_small.
+ * 22 qubits (to 27 qubits 12 for blocks that 13 saves no passes), 11 from
+ * 19, 10 below (at least 9); it also lowers the contiguous low bits to 2,
+ * and to 0 up to 18 qubits for blocks that this saves a quarter of their
+ * passes.  Fused registers narrower than 9 qubits take ph2hip_rotate_small.
  */
 
 #include <stddef.h>

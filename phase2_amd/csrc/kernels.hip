@@ -6,9 +6,10 @@
 //
 // Arithmetic contract (bit identity with the reference CPU backend,
 // phase2/qreg_qreg.c:149-160): built with -ffp-contract=off and every
-// product/sum goes through mul()/add() below, so each component update is
-// round(round(c*x) + round(+-s*y)) with c, s computed by the host libm.
-// Negations and component swaps are exact.  Nothing here is FMA-contracted.
+// product/sum goes through mul()/add() below or the fused passes' assembly,
+// so each component update is round(round(c*x) + round(+-s*y)) with c, s
+// computed by the host libm.  Negations and component swaps are exact, and
+// the one fma (by a factor +-1.0) rounds as the sum it stands for.
 //
 // Kernels:
 //   k_rot_pair    plain pass, one thread per amplitude pair (i, i^x), i<j
@@ -277,13 +278,15 @@ __global__ __launch_bounds__(1 << (kSmallQb - 1)) void k_rot_small(
 // ---------------------------------------------------------------------------
 //
 // Tile: the coset  base ^ span{e_0..e_{L-1}, w_0..w_{g-1}}  of 2^TB
-// amplitudes (TB = L + g), held in LDS.  The w_b have zero low L bits,
-// distinct leading bits p_b (ascending in b) and zeros at every other p_b'.
+// amplitudes (TB = L + g), in registers and LDS.  The w_b have zero low L
+// bits: the reduced echelon basis of the masks beyond them, with leading bits
+// p_b (pivots), or for some tile-13 passes masks of the pass (mask_basis).
 // Tile coordinate v: bits [0,L) are index bits 0..L-1, bit L+b selects w_b;
 // the tile index spreads over the index bits that are neither low nor
 // pivots.  In these coordinates a term with flip mask x has xt, and
-//   parity(i & z) = parity(base & z) ^ parity(v & zt),   i < i^x <=> v < v^xt,
-// so the plain update runs unchanged on v.
+//   parity(i & z) = parity(base & z) ^ parity(v & zt),
+// so the plain update runs unchanged on v (it is the same seen from either
+// amplitude of a pair: the phase seen from i^x is the conjugate).
 //
 // Inside the tile the terms of the pass are cut into micro-groups whose xt
 // span at most D dimensions.  A group has its own basis u_0..u_{D-1} (tile
@@ -333,7 +336,7 @@ struct FusedGroup {
 
 struct FusedPass {
 	uint64_t w[PH2HIP_TILE_MAX];   // gathered basis vectors
-	uint32_t piv[PH2HIP_TILE_MAX]; // their leading bits, ascending
+	uint32_t piv[PH2HIP_TILE_MAX]; // pivots of their span, ascending
 	uint8_t L, g, ngroups, nterms;
 	// bit 0: the first group loads its cosets from HBM (the tile is not
 	// staged in LDS first); bit 1: the last group stores them to HBM;

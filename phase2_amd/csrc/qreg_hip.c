@@ -131,17 +131,41 @@ static uint32_t auto_low(uint32_t low)
 	return low > 2 ? 2 : low;
 }
 
-/* Up to 18 qubits the state lies in the L2s, where short rows cost less
- * than passes: with no low bits asked for, sweeps (whose masks have an even
+/* Under the automatic setting a block of a register of up to 18 or of 22 to 27
+ * qubits is cut twice, and the number of passes says which cut it takes.
+ *
+ * To 18 qubits the state lies in the L2s, where short rows cost less than
+ * passes: with no low bits asked for, sweeps (whose masks have an even
  * number of flips, so that single low bits are dimensions none of them
  * needs) take a third fewer passes and 324 us instead of 347 at 16 qubits,
  * 290 / 311 at 14, 389 / 405 at 18, but random draws a fifth fewer and 378
- * instead of 366, 392 / 368 and 471 / 450.  So both cuts are made, and the
- * one without low bits is taken if it saves a quarter of the passes; to 12
- * qubits always (271 / 281 and 211 / 218). */
-static int no_low(uint32_t nqb, size_t passes, size_t passes0)
+ * instead of 366, 392 / 368 and 471 / 450.  The second cut, without low
+ * bits, is taken if it saves a quarter of the passes; to 12 qubits always
+ * (271 / 281 and 211 / 218).
+ *
+ * From 22 to 27 qubits a tile-12 pass is the shorter one: blocks of 1 to 40
+ * terms that need as many passes at either width took 1.06, 1.05, 1.05,
+ * 1.03, 1.015 and 1.07 times as long at tile 13 (22 to 27 qubits, mean of
+ * 13 to 17 blocks each; 825 us against 1312 in one of nine terms at 27), 0.99
+ * at 28 and 1.00 at 30.  The second cut, at tile 12, is taken unless tile 13
+ * saves a twentieth of its passes; blocks of 1024 terms save a twelfth or more
+ * (at 22 qubits 41 passes instead of 45, 1467 us instead of 1489). */
+static int second_cut(uint32_t nqb, uint32_t *tile, uint32_t *low)
 {
-	return nqb <= 12 || 4 * passes0 <= 3 * passes;
+	if (nqb <= 18 && *low > 0)
+		*low = 0;
+	else if (nqb >= 22 && nqb <= 27 && *tile == 13)
+		*tile = 12;
+	else
+		return 0;
+	return 1;
+}
+
+static int take_second(uint32_t nqb, size_t first, size_t second)
+{
+	if (nqb <= 18)
+		return nqb <= 12 || 4 * second <= 3 * first;
+	return 20 * first > 19 * second;
 }
 
 static void load_defaults(void)
@@ -532,12 +556,14 @@ static int rotate_block(struct qreg_hip *h, uint32_t nqb, struct block *b)
 	if (g_sched_fn)
 		rc = g_sched_fn(g_sched_ctx, b->rot, b->n, nqb, &h->sched);
 	if (rc < 0) {
-		const uint32_t tile = h->tile_bits ? h->tile_bits :
-			auto_tile(nqb);
 		const uint32_t low = h->tile_bits ? h->low_bits :
 			auto_low(h->low_bits);
-		/* the cut at tile 13 depends on the half-tile setting */
+		/* the cut at tile 13 depends on the half-tile setting; without
+		 * that form tile 13 runs one workgroup per CU */
 		const uint32_t half = ph2hip_fused_half_mask();
+		uint32_t tile = h->tile_bits ? h->tile_bits : auto_tile(nqb);
+		if (!h->tile_bits && tile == 13 && !(half >> 13 & 1))
+			tile = 12;
 		s = &b->sched;
 		rc = 0;
 		if (!b->scheduled || b->tile != tile || b->low != low ||
@@ -545,10 +571,12 @@ static int rotate_block(struct qreg_hip *h, uint32_t nqb, struct block *b)
 			b->scheduled = 0;
 			rc = ph2_sched_greedy(b->rot, b->n, nqb, tile, low,
 				&b->sched);
-			if (rc == 0 && !h->tile_bits && nqb <= 18 && low > 0 &&
-			    (rc = ph2_sched_greedy(b->rot, b->n, nqb, tile, 0,
+			uint32_t tile2 = tile, low2 = low;
+			if (rc == 0 && !h->tile_bits &&
+			    second_cut(nqb, &tile2, &low2) &&
+			    (rc = ph2_sched_greedy(b->rot, b->n, nqb, tile2, low2,
 				     &h->sched)) == 0 &&
-			    no_low(nqb, b->sched.npass, h->sched.npass)) {
+			    take_second(nqb, b->sched.npass, h->sched.npass)) {
 				const struct ph2_sched t = b->sched;
 				b->sched = h->sched;
 				h->sched = t;

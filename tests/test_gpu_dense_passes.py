@@ -110,3 +110,39 @@ def test_automatic_low_bits(oracle, n):
     finally:
         nat.prof_enable(False)
         reg.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [21, 22, 24])
+def test_automatic_tile(n):
+    """A block of few terms at the width that costs its pass least, a sweep
+    at the width that takes the fewest, without the half-tile form never 13;
+    all equal to the plain sweep."""
+    hm = synth.hamiltonian(n, 400, seed=n)
+    lex = nat.sort_lex(hm.xm, hm.zm)
+    a, b = nat.Register(n, nat.FUSED, 0, 3), nat.Register(n, nat.PLAIN)
+    tiles = []
+    try:
+        for r in (a, b):
+            r.fill_hash(n)
+        for k, half in ((lex[300:304], nat.HALF_TILES),
+                        (lex[200:], nat.HALF_TILES), (lex[200:], 0)):
+            phi = 0.1 * hm.cf[k] / np.max(np.abs(hm.cf))
+            nat.set_fused_half(half)
+            nat.prof_enable(True)
+            nat.prof_records(reset=True)
+            a.rotate(hm.xm[k], hm.zm[k], phi)
+            rec = nat.prof_records(reset=True)
+            nat.prof_enable(False)
+            tiles.append(set(rec["tile_bits"].tolist()))
+            b.rotate(hm.xm[k], hm.zm[k], phi)
+        assert a.count_unequal(b) == 0
+        if n == 21:
+            assert tiles == [{11}] * 3
+        else:
+            assert tiles[0] == {12} and tiles[2] == {12}
+    finally:
+        nat.prof_enable(False)
+        nat.set_fused_half(nat.HALF_TILES)
+        a.free()
+        b.free()
