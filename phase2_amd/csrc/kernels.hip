@@ -2405,13 +2405,38 @@ int launch_batch(double2 *amp, const uint8_t *descs, const BatchItem *items,
 // The first time a call is seen it is remembered (a copy of its
 // arguments); the second time its launches are captured into a hipGraph
 // (kernel nodes only: the pass descriptors are kernel arguments); from
-// then on the graph is replayed.  Calls match only if every argument is
-// equal, compared in full, so a replay launches exactly what the direct
-// path would.
+// then on the graph is replayed.  Calls match only if every argument and
+// every setting of the kernels' form is equal, compared in full, so a replay
+// launches exactly what the direct path would.
 constexpr int kReplaySlots = 32;
+
+// The settings that choose a fused pass's kernel, grid and descriptor.
+struct FusedForm {
+	uint64_t persist_wgs;
+	uint32_t direct, half, pipe, pad;
+	uint32_t hpipe_pf[PH2HIP_TILE_MAX + 1];
+	uint32_t hpipe_wpc[PH2HIP_TILE_MAX + 1];
+};
+
+FusedForm fused_form()
+{
+	static_assert(sizeof(FusedForm) == 24 + 8 * (PH2HIP_TILE_MAX + 1),
+		"compared as bytes: no gaps");
+	FusedForm f;
+	pipe_init();
+	f.direct = g_direct;
+	f.half = half_mask();
+	f.pipe = g_pipe_mask;
+	f.pad = 0;
+	f.persist_wgs = g_persist_wgs;
+	memcpy(f.hpipe_pf, g_hpipe_pf, sizeof f.hpipe_pf);
+	memcpy(f.hpipe_wpc, g_hpipe_wpc, sizeof f.hpipe_wpc);
+	return f;
+}
 
 struct ReplaySlot {
 	uint64_t key, used;
+	FusedForm form;
 	void *amp;
 	uint32_t nqb;
 	size_t n, npass;
@@ -2452,12 +2477,13 @@ void replay_clear(ReplaySlot &r)
 	r = ReplaySlot{};
 }
 
-bool replay_same(const ReplaySlot &r, uint64_t key, void *amp, uint32_t nqb,
-	const struct ph2hip_rot *rot, size_t n, const uint32_t *const sch[3],
-	size_t npass)
+bool replay_same(const ReplaySlot &r, uint64_t key, const FusedForm &form,
+	void *amp, uint32_t nqb, const struct ph2hip_rot *rot, size_t n,
+	const uint32_t *const sch[3], size_t npass)
 {
 	if (!r.rot || r.key != key || r.amp != amp || r.nqb != nqb ||
 	    r.n != n || r.npass != npass ||
+	    memcmp(&r.form, &form, sizeof form) != 0 ||
 	    memcmp(r.rot, rot, sizeof *rot * n) != 0)
 		return false;
 	for (int a = 0; a < 3; a++)
@@ -2476,9 +2502,10 @@ ReplaySlot *replay_slot(void *amp, uint32_t nqb, const struct ph2hip_rot *rot,
 		sizeof *rot * n);
 	for (int a = 0; a < 3; a++)
 		key = fnv_words(key, sch[a], sizeof(uint32_t) * npass);
+	const FusedForm form = fused_form();
 	ReplaySlot *old = &g_replay[0];
 	for (ReplaySlot &r : g_replay) {
-		if (replay_same(r, key, amp, nqb, rot, n, sch, npass)) {
+		if (replay_same(r, key, form, amp, nqb, rot, n, sch, npass)) {
 			r.used = ++g_replay_clock;
 			*seen = true;
 			return &r;
@@ -2499,6 +2526,7 @@ ReplaySlot *replay_slot(void *amp, uint32_t nqb, const struct ph2hip_rot *rot,
 	for (int a = 0; a < 3; a++)
 		memcpy(old->sched + a * npass, sch[a], sizeof(uint32_t) * npass);
 	old->key = key;
+	old->form = form;
 	old->amp = amp;
 	old->nqb = nqb;
 	old->n = n;
