@@ -71,8 +71,11 @@ typedef int (*ph2_sched_fn)(void *ctx, const struct ph2hip_rot *rot,
 	size_t n, uint32_t nqb, struct ph2_sched *out);
 void ph2_sched_install(ph2_sched_fn fn, void *ctx);
 
-/* Device pointer of the register's amplitudes (for the batched and
- * benchmark entry points). */
+/* Device pointer of the register's amplitudes, for the caller's own kernels
+ * and copies on any stream.  Returns when all work queued on the register so
+ * far is done (amplitude writes, zeroing, rotations); work queued later is
+ * not waited for: take the pointer again, or call ph2hip_synchronize, before
+ * looking. */
 void *qreg_hip_device_ptr(struct qreg *reg);
 
 #ifdef __cplusplus

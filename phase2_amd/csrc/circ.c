@@ -326,7 +326,7 @@ _Complex double circ_measure(struct circ *ct)
 			log_error("circ_measure: no overlap plan");
 			return 0.0;
 		}
-		if (ph2hip_gather(qreg_hip_device_ptr(&ct->reg),
+		if (ph2hip_gather(qreg_hip_buffer(&ct->reg),
 			    ct->reg.qb_lo, p->idx, p->n, p->amp) < 0) {
 			log_error("circ_measure: %s", ph2hip_strerror());
 			return 0.0;

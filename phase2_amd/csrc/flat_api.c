@@ -105,7 +105,7 @@ static void results(const struct circ *ct, double *out, double *state)
 		out[2 * i + 1] = cimag(ct->vals.z[i]);
 	}
 	if (state)
-		ph2hip_d2h(state, qreg_hip_device_ptr((struct qreg *)&ct->reg),
+		ph2hip_d2h(state, qreg_hip_buffer((struct qreg *)&ct->reg),
 			ct->reg.namp * 16);
 }
 
@@ -194,7 +194,7 @@ int ph2_rotate(double *state, uint32_t nqb, size_t n, const uint64_t *xm,
 	if (qreg_init(&reg, nqb) < 0)
 		return -1;
 	qreg_hip_configure(&reg, mode, tile_bits, low_bits);
-	void *d = qreg_hip_device_ptr(&reg);
+	void *d = qreg_hip_buffer(&reg);
 	int rc = ph2hip_h2d(d, state, reg.namp * 16);
 	struct paulis codes[1024];
 	const struct paulis hi = { .pak = { 0, 0 } };
@@ -239,7 +239,7 @@ int ph2_expand(uint32_t nqb, uint32_t n_sites, uint32_t n_alpha,
 	cm.C_beta = closed_shell ? NULL : Cb;
 	int rc = state_prep_coeff_expand_all(&reg, &sc, &cm);
 	if (rc == 0)
-		rc = ph2hip_d2h(state, qreg_hip_device_ptr(&reg), reg.namp * 16);
+		rc = ph2hip_d2h(state, qreg_hip_buffer(&reg), reg.namp * 16);
 	state_prep_coeff_scratch_free(&sc);
 	qreg_free(&reg);
 	return rc;
@@ -259,7 +259,7 @@ int ph2_inner(uint32_t nqb, uint32_t n_sites, uint32_t n_alpha,
 		qreg_free(&reg);
 		return -1;
 	}
-	int rc = ph2hip_h2d(qreg_hip_device_ptr(&reg), state, reg.namp * 16);
+	int rc = ph2hip_h2d(qreg_hip_buffer(&reg), state, reg.namp * 16);
 	_Complex double z = 0.0;
 	if (rc == 0)
 		rc = state_prep_coeff_inner(&reg, &sc, Ca,
@@ -368,7 +368,7 @@ int ph2_reg_rotate_sched(void *r, size_t n, const uint64_t *xm,
 		rot[k].z = zm[k];
 		sincos(phi[k], &rot[k].s, &rot[k].c);
 	}
-	const int rc = ph2hip_rotate_fused(qreg_hip_device_ptr(reg), reg->qb_lo,
+	const int rc = ph2hip_rotate_fused(qreg_hip_buffer(reg), reg->qb_lo,
 		rot, n, pass_len, tile_bits, npass, low_bits);
 	free(rot);
 	return rc;
@@ -386,7 +386,7 @@ int ph2_reg_overlap_multidet(void *r, size_t ndet, const uint64_t *didx,
 		/* indices beyond the register are refused by the gather */
 		for (size_t d = 0; d < ndet; d++)
 			idx[d] = didx[d];
-		rc = ph2hip_gather(qreg_hip_device_ptr(reg), reg->qb_lo, idx,
+		rc = ph2hip_gather(qreg_hip_buffer(reg), reg->qb_lo, idx,
 			ndet, a);
 	}
 	if (rc == 0) {
@@ -405,25 +405,25 @@ int ph2_reg_overlap_multidet(void *r, size_t ndet, const uint64_t *didx,
 int ph2_reg_norm2(void *r, double *out)
 {
 	struct qreg *reg = r;
-	return ph2hip_norm2(qreg_hip_device_ptr(reg), reg->qb_lo, out);
+	return ph2hip_norm2(qreg_hip_buffer(reg), reg->qb_lo, out);
 }
 
 int ph2_reg_read(void *r, double *state)
 {
 	struct qreg *reg = r;
-	return ph2hip_d2h(state, qreg_hip_device_ptr(reg), reg->namp * 16);
+	return ph2hip_d2h(state, qreg_hip_buffer(reg), reg->namp * 16);
 }
 
 int ph2_reg_gather(void *r, size_t n, const uint64_t *idx, double *out)
 {
 	struct qreg *reg = r;
-	return ph2hip_gather(qreg_hip_device_ptr(reg), reg->qb_lo, idx, n, out);
+	return ph2hip_gather(qreg_hip_buffer(reg), reg->qb_lo, idx, n, out);
 }
 
 int ph2_reg_fill_hash(void *r, uint64_t seed)
 {
 	struct qreg *reg = r;
-	return ph2hip_fill_hash(qreg_hip_device_ptr(reg), reg->namp, seed);
+	return ph2hip_fill_hash(qreg_hip_buffer(reg), reg->namp, seed);
 }
 
 int ph2_reg_count_unequal(void *r1, void *r2, uint64_t *count)
@@ -431,6 +431,6 @@ int ph2_reg_count_unequal(void *r1, void *r2, uint64_t *count)
 	struct qreg *a = r1, *b = r2;
 	if (a->namp != b->namp)
 		return -1;
-	return ph2hip_count_unequal(qreg_hip_device_ptr(a),
-		qreg_hip_device_ptr(b), a->namp, count);
+	return ph2hip_count_unequal(qreg_hip_buffer(a),
+		qreg_hip_buffer(b), a->namp, count);
 }

@@ -18,6 +18,10 @@ typedef int (*term_cmp)(const struct circ_hamil_term *,
 void *qreg_hip_aux(struct qreg *reg);
 int qreg_hip_set_aux(struct qreg *reg, void *aux, void (*aux_free)(void *));
 
+/* Device buffer of a register for work on the library's own stream
+ * (qreg_hip.c): qreg_hip_device_ptr without its wait. */
+void *qreg_hip_buffer(struct qreg *reg);
+
 /* Stable sort of a term array (circ.c). */
 int circ_terms_sort(struct circ_hamil_term *t, size_t n, term_cmp cmp);
 

@@ -64,7 +64,8 @@ struct qreg_hip {
 	uint64_t *qidx;
 	double *qval;
 	size_t nq, qcap;
-	int flying;	/* writes sent to the stream and not waited for */
+	int pending;	/* work on the buffer sent to the stream and not waited
+			 * for since */
 	/* host copy of amplitudes [win_lo, win_lo + win_n) as the device
 	 * holds them with the queued writes applied; win_n = 0: none */
 	double *win;
@@ -226,7 +227,7 @@ static int settle(struct qreg_hip *h, uint64_t namp)
 	const int rc = ph2hip_scatter_queue(h->damp, namp, h->qidx, h->qval,
 		h->nq);
 	h->nq = 0;
-	h->flying = 1;
+	h->pending = 1;
 	if (rc < 0) {
 		h->err = -1;
 		log_error("qreg_setamp: %s", ph2hip_strerror());
@@ -234,18 +235,35 @@ static int settle(struct qreg_hip *h, uint64_t namp)
 	return rc;
 }
 
-/* The caller may read or change the buffer through the pointer, on a stream
- * of its own too, so the queued writes land first and the read window goes. */
+/* For calls of this library, which queue their work behind the register's on
+ * the same stream: the queued amplitude writes are sent ahead and the read
+ * window goes, nothing is waited for. */
+void *qreg_hip_buffer(struct qreg *reg)
+{
+	struct qreg_hip *h = reg->backend;
+	if (!h)
+		return NULL;
+	settle(h, reg->namp);
+	h->pending = 1;
+	return h->damp;
+}
+
+/* The caller may read or change the buffer through the pointer on any
+ * stream, so everything queued on it is done first: amplitude writes,
+ * zeroing, rotations and the work of other calls of this library. */
 void *qreg_hip_device_ptr(struct qreg *reg)
 {
 	struct qreg_hip *h = reg->backend;
 	if (!h)
 		return NULL;
 	settle(h, reg->namp);
-	if (h->flying) {
-		h->flying = 0;
-		if (ph2hip_synchronize() < 0)
+	if (h->pending) {
+		h->pending = 0;
+		if (ph2hip_synchronize() < 0) {
 			h->err = -1;
+			log_error("qreg_hip_device_ptr: %s",
+				ph2hip_strerror());
+		}
 	}
 	return h->damp;
 }
@@ -469,6 +487,7 @@ void qreg_zero(struct qreg *reg)
 	h->nq = 0; /* every queued write would be overwritten */
 	h->win_n = 0;
 	h->reads = 0;
+	h->pending = 1;
 	if (ph2hip_zero(h->damp, reg->namp) < 0)
 		set_err(reg, "qreg_zero");
 }
@@ -615,6 +634,7 @@ void qreg_paulirot(struct qreg *reg, struct paulis code_hi,
 	}
 	const uint32_t nqb = reg->qb_lo;
 	int rc;
+	h->pending = 1;
 	if (h->mode == QREG_HIP_PLAIN)
 		rc = ph2hip_rotate_plain(h->damp, nqb, b->rot, ncodes);
 	else if (nqb < PH2HIP_TILE_MIN)

@@ -24,9 +24,9 @@
 #include "det_small.h"
 #include "log.h"
 #include "phase2/circ.h"
-#include "phase2/qreg_hip.h"
 #include "phase2/state_prep_coeff.h"
 #include "phase2_hip.h"
+#include "internal.h"
 
 struct sc_dev {
 	struct ph2hip_sc *tab;
@@ -224,7 +224,7 @@ int state_prep_coeff_expand(struct qreg *reg,
 		log_error("expand: device tables: %s", ph2hip_strerror());
 		return -1;
 	}
-	if (ph2hip_sc_scatter(qreg_hip_device_ptr(reg), reg->qb_lo, tab,
+	if (ph2hip_sc_scatter(qreg_hip_buffer(reg), reg->qb_lo, tab,
 		    sc->n_sites, weight, tapered, accumulate) < 0) {
 		log_error("expand: %s", ph2hip_strerror());
 		return -1;
@@ -259,7 +259,7 @@ int state_prep_coeff_inner(struct qreg *reg,
 {
 	struct ph2hip_sc *tab = device_tables(sc, C_alpha, C_beta);
 	double r[2];
-	if (!tab || ph2hip_sc_inner(qreg_hip_device_ptr(reg), reg->qb_lo, tab,
+	if (!tab || ph2hip_sc_inner(qreg_hip_buffer(reg), reg->qb_lo, tab,
 			    sc->n_sites, weight, tapered, r) < 0) {
 		log_error("inner: %s", ph2hip_strerror());
 		return -1;
