@@ -235,6 +235,17 @@ static int settle(struct qreg_hip *h, uint64_t namp)
 	return rc;
 }
 
+static void wait_pending(struct qreg_hip *h, const char *what)
+{
+	if (!h->pending)
+		return;
+	h->pending = 0;
+	if (ph2hip_synchronize() < 0) {
+		h->err = -1;
+		log_error("%s: %s", what, ph2hip_strerror());
+	}
+}
+
 /* For calls of this library, which queue their work behind the register's on
  * the same stream: the queued amplitude writes are sent ahead and the read
  * window goes, nothing is waited for. */
@@ -257,14 +268,7 @@ void *qreg_hip_device_ptr(struct qreg *reg)
 	if (!h)
 		return NULL;
 	settle(h, reg->namp);
-	if (h->pending) {
-		h->pending = 0;
-		if (ph2hip_synchronize() < 0) {
-			h->err = -1;
-			log_error("qreg_hip_device_ptr: %s",
-				ph2hip_strerror());
-		}
-	}
+	wait_pending(h, "qreg_hip_device_ptr");
 	return h->damp;
 }
 
@@ -281,7 +285,8 @@ int qreg_error(const struct qreg *reg)
 	struct qreg_hip *h = reg->backend;
 	if (!h)
 		return -1;
-	/* a queued write fails, if at all, when it lands: land it now */
+	/* a queued write fails, if at all, when it lands: land it now, and
+	 * wait for it (short ones are only sent to the stream) */
 	if (h->nq) {
 		const uint64_t lo = h->win_lo, n = h->win_n;
 		const int reads = h->reads;
@@ -289,6 +294,7 @@ int qreg_error(const struct qreg *reg)
 		h->win_lo = lo;
 		h->win_n = n;
 		h->reads = reads;
+		wait_pending(h, "qreg_error");
 	}
 	return h->err;
 }

@@ -32,11 +32,16 @@ def busy():
     reg.free()
 
 
-def _look(reg):
+def _ptr(reg):
     L = nat.lib()
     L.qreg_hip_device_ptr.restype = C.c_void_p
+    return L.qreg_hip_device_ptr(C.c_void_p(reg.h))
+
+
+def _look(reg, ptr=None):
+    L = nat.lib()
     got = np.zeros(1 << reg.nqb, complex)
-    ptr = L.qreg_hip_device_ptr(C.c_void_p(reg.h))
+    ptr = ptr or _ptr(reg)
     # the runtime that the library is linked with
     assert L.hipMemcpy(C.c_void_p(got.ctypes.data), C.c_void_p(ptr),
                        C.c_size_t(got.nbytes), C.c_int(2)) == 0
@@ -102,3 +107,24 @@ def test_after_calls_of_the_library(busy):
     finally:
         a.free()
         b.free()
+
+
+@pytest.mark.parametrize("count", [1, 64, 65])
+def test_error_check_waits_for_writes(busy, count):
+    """qreg_error reports on writes that have landed: they are in the buffer
+    when it returns, also the short ones that are sent without a wait."""
+    reg, st = _start(N)
+    L = nat.lib()
+    L.qreg_setamp.argtypes = [C.c_void_p, C.c_uint64, C.c_double, C.c_double]
+    L.qreg_error.argtypes = [C.c_void_p]
+    L.qreg_error.restype = C.c_int
+    try:
+        ptr = _ptr(reg)
+        busy()
+        for i in range(count):
+            L.qreg_setamp(reg.h, 10 + i, 0.25, float(i))
+            st[10 + i] = 0.25 + 1j * i
+        assert L.qreg_error(reg.h) == 0
+        assert np.array_equal(_look(reg, ptr), st)
+    finally:
+        reg.free()
