@@ -15,9 +15,12 @@
  * bits, 9..13) and PHASE2_HIP_LOW (contiguous low bits); otherwise fused,
  * automatic tile width and 3.  Tile width 0 (the automatic one) is 13 from
  * 22 qubits (to 27 qubits 12 for blocks that 13 saves no passes), 11 from
- * 19, 10 below (at least 9); it also lowers the contiguous low bits to 2,
- * and to 0 up to 18 qubits for blocks that this saves a quarter of their
- * passes.  Fused registers narrower than 9 qubits take ph2hip_rotate_small.
+ * 19, 10 below (at least 9); beyond the qubits of ph2hip_replay_max_qb (20
+ * by default) 11 at 21, 12 from 17, nqb - 5 below.  With it, low bits 3
+ * (the default) stand for the library's choice: 2, and 0 up to 18 qubits for
+ * blocks that this saves a quarter of their passes (to 12 qubits always);
+ * any other value is used as given.  Fused registers narrower than 9 qubits
+ * take ph2hip_rotate_small.
  */
 
 #include <stddef.h>

@@ -44,7 +44,7 @@ struct block {
 	struct ph2_sched sched;
 	int scheduled;	/* sched is the greedy one of the settings below */
 	int chosen;	/* the tile and low bits are automatic */
-	uint32_t tile, low, half;
+	uint32_t tile, low, half;	/* low as asked for */
 	uint64_t used;
 };
 
@@ -86,7 +86,7 @@ struct qreg_hip {
 #define AMP_QMAX ((size_t)1 << 20)   /* 24 MiB of queued writes */
 
 static int g_mode = -1;
-/* tile 0: auto_tile() and auto_low() */
+/* tile 0: auto_tile(), with low 3 auto_low() */
 static uint32_t g_tile = 0, g_low = 3;
 static ph2_sched_fn g_sched_fn;
 static void *g_sched_ctx;
@@ -121,15 +121,16 @@ static uint32_t auto_tile(uint32_t nqb)
 	return t < PH2HIP_TILE_MIN ? PH2HIP_TILE_MIN : t;
 }
 
-/* Contiguous low bits the cut asks for under the automatic tile width: at
- * most `low`, and at most 2, where rows of 64 bytes leave one more
- * dimension to gather than rows of 128.  Low 2 against 3: random draws 366
- * and 393 us at 16 qubits, 450 and 493 at 18, 850 and 918 at 20; sweeps 346
- * and 348, 406 and 415, 673 and 675; 6547 and 6748 at 24, 130562 and 134986
- * at 28.  Low 1 is slower from 30. */
+/* Contiguous low bits the cut asks for under the automatic tile width: those
+ * the caller set, but for the default (LOW_AUTO) 2, where rows of 64 bytes
+ * leave one more dimension to gather than rows of 128.  Low 2 against 3:
+ * random draws 366 and 393 us at 16 qubits, 450 and 493 at 18, 850 and 918
+ * at 20; sweeps 346 and 348, 406 and 415, 673 and 675; 6547 and 6748 at 24,
+ * 130562 and 134986 at 28.  Low 1 is slower from 30. */
+#define LOW_AUTO 3
 static uint32_t auto_low(uint32_t low)
 {
-	return low > 2 ? 2 : low;
+	return low == LOW_AUTO ? 2 : low;
 }
 
 /* Under the automatic setting a block of a register of up to 18 or of 22 to 27
@@ -142,7 +143,7 @@ static uint32_t auto_low(uint32_t low)
  * 290 / 311 at 14, 389 / 405 at 18, but random draws a fifth fewer and 378
  * instead of 366, 392 / 368 and 471 / 450.  The second cut, without low
  * bits, is taken if it saves a quarter of the passes; to 12 qubits always
- * (271 / 281 and 211 / 218).
+ * (271 / 281 and 211 / 218).  Low bits that the caller set stay.
  *
  * From 22 to 27 qubits a tile-12 pass is the shorter one: blocks of 1 to 40
  * terms that need as many passes at either width took 1.06, 1.05, 1.05,
@@ -151,9 +152,10 @@ static uint32_t auto_low(uint32_t low)
  * at 28 and 1.00 at 30.  The second cut, at tile 12, is taken unless tile 13
  * saves a twentieth of its passes; blocks of 1024 terms save a twelfth or more
  * (at 22 qubits 41 passes instead of 45, 1467 us instead of 1489). */
-static int second_cut(uint32_t nqb, uint32_t *tile, uint32_t *low)
+static int second_cut(uint32_t nqb, uint32_t asked, uint32_t *tile,
+	uint32_t *low)
 {
-	if (nqb <= 18 && *low > 0)
+	if (nqb <= 18 && asked == LOW_AUTO)
 		*low = 0;
 	else if (nqb >= 22 && nqb <= 27 && *tile == 13)
 		*tile = 12;
@@ -591,14 +593,15 @@ static int rotate_block(struct qreg_hip *h, uint32_t nqb, struct block *b)
 			tile = 12;
 		s = &b->sched;
 		rc = 0;
-		if (!b->scheduled || b->tile != tile || b->low != low ||
+		if (!b->scheduled || b->tile != tile ||
+		    b->low != h->low_bits ||
 		    b->half != half || b->chosen != !h->tile_bits) {
 			b->scheduled = 0;
 			rc = ph2_sched_greedy(b->rot, b->n, nqb, tile, low,
 				&b->sched);
 			uint32_t tile2 = tile, low2 = low;
 			if (rc == 0 && !h->tile_bits &&
-			    second_cut(nqb, &tile2, &low2) &&
+			    second_cut(nqb, h->low_bits, &tile2, &low2) &&
 			    (rc = ph2_sched_greedy(b->rot, b->n, nqb, tile2, low2,
 				     &h->sched)) == 0 &&
 			    take_second(nqb, b->sched.npass, h->sched.npass)) {
@@ -607,7 +610,7 @@ static int rotate_block(struct qreg_hip *h, uint32_t nqb, struct block *b)
 				h->sched = t;
 			}
 			b->tile = tile;
-			b->low = low;
+			b->low = h->low_bits;
 			b->half = half;
 			b->chosen = !h->tile_bits;
 			b->scheduled = rc == 0;
