@@ -16,9 +16,9 @@
  * as y = ln(ms) - (nqb - 30) ln 2 (time per 2^30 amplitudes).  For a block of
  * terms the scheduler enumerates passes [i, j) that end where the next term
  * would widen the tile (or at the longest feasible end), for tile widths 12
- * and 13 and for three counts of contiguous low bits (low_bits - 1 and the
- * next two; from low_bits itself if it is 2 or less), predicts them all in
- * one batch on the GPU and picks the cut, tile and low bits of every pass
+ * and 13 and for three counts of contiguous low bits (low_bits - 1, low_bits
+ * and low_bits + 1; 0, 1 and 2 if it is 0), predicts them all in one batch on
+ * the GPU and picks the cut, tile and low bits of every pass
  * with the smallest predicted total by dynamic programming.  Schedules are
  * cached per block (flip and phase masks, width), so repeated Trotter sweeps
  * pay for scheduling once.  The order of terms never changes, so the state
@@ -45,8 +45,8 @@ void ph2_learned_features(const struct ph2hip_rot *rot, size_t n,
 
 /* Load parameters (packed as ph2hip_mlp) of a PH2_LM_NIN -> nhid -> nhid
  * -> 1 network, and install the learned schedule for fused registers of at
- * least min_qb qubits (narrower ones keep the greedy cut).  low_bits centres
- * the contiguous low parts that passes may request, as above. */
+ * least min_qb qubits (narrower ones keep the greedy cut).  low_bits is the
+ * middle one of the contiguous low parts that passes may request. */
 int ph2_learned_install(const float *params, uint32_t nhid, uint32_t low_bits,
 	uint32_t min_qb);
 void ph2_learned_uninstall(void);

@@ -294,8 +294,8 @@ def load(path=PARAMS_PATH):
 
 def install(params, low=3, min_qb=26):
     """Use the learned schedule for fused registers of >= min_qb qubits
-    (passes with three counts of contiguous low bits: from low - 1, or from
-    low itself if it is 2 or less)."""
+    (passes with low - 1, low or low + 1 contiguous low bits; with 0, 1 or 2
+    if low is 0)."""
     p = np.ascontiguousarray(params, np.float32)
     if p.size != n_params():
         raise ValueError(f"{p.size} parameters, the network has "

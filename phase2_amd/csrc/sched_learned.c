@@ -36,16 +36,17 @@ static struct {
 /* candidate tile widths: both have the half-tile form (tile 11 was rarely
  * chosen once tile 12 had it) */
 static const uint32_t TILES[] = { 12, 13 };
-/* Contiguous low bits of the candidates: NLOW counts from one below the low
- * bits asked for, but not below 2.  With the default 3 as the first count,
- * 2 was never tried, and from 28 qubits rows of 64 bytes, which leave one
- * more dimension to gather, are the better ones: 1024-term sweeps took
- * 130.3 and 131.8 ms at 28 qubits, 551 and 614 at 30, 1151 and 1227 at 31,
- * and take 126.6 and 125.5, 536 and 587, 1098 and 1217. */
+/* Contiguous low bits of the candidates: NLOW counts, the middle one as asked
+ * for (the default 3: 2, 3 and 4; 0 and 1 alike: 0, 1 and 2).  With 3, 4 and
+ * 5, as the default once was, 2 was never tried, and from 28 qubits rows of
+ * 64 bytes, which leave one more dimension to gather, are the better ones:
+ * 1024-term sweeps took 130.3 and 131.8 ms at 28 qubits, 551 and 614 at 30,
+ * 1151 and 1227 at 31, and took 126.6 and 125.5, 536 and 587, 1098 and 1217
+ * with 2, 3 and 4. */
 #define NLOW 3
 static uint32_t first_low(uint32_t low)
 {
-	return low > 2 ? low - 1 : low;
+	return low ? low - 1 : 0;
 }
 
 void ph2_learned_features(const struct ph2hip_rot *rot, size_t n,
