@@ -246,10 +246,18 @@ def plain_rate(nat, nqb, xm, zm, phi):
                 diag_launches=pp["plain_diag"]["launches"])
 
 
+def tiles_run(kernels, asked):
+    """Tile width of the fused passes that ran, from the launch counts per
+    kernel (launches_per_kernel): a list if there were several, the width
+    asked for if there were none."""
+    t = sorted({int(k.split("<")[1].split(",")[0]) for k in kernels})
+    return t[0] if len(t) == 1 else t or asked
+
+
 def auto_tile(tile, nqb, replay_max_qb=20):
-    """The library's tile width for a requested one (0: automatic), with
-    graph replay of repeated sweeps on for registers of at most
-    replay_max_qb qubits (the library's default)."""
+    """A tile width by register width alone, as the library once chose it
+    (0: automatic).  The library now looks at every block's passes too
+    (include/phase2/qreg_hip.h), so results report tiles_run instead."""
     if tile:
         return tile
     if nqb <= replay_max_qb:
@@ -731,8 +739,8 @@ def main(argv=None):
     plain = r["plain"]
     cfg = dict(r["config"])
     cfg.update(schedule=schedule, low_bits=args.low,
-               tile_bits=auto_tile(args.tile, r["nqb"]) if r["nqb"]
-               else args.tile)
+               tile_bits=tiles_run(r["extra"]["launches_per_kernel"],
+                                   args.tile))
     out = {
         "metric": METRIC,
         "value": value,
