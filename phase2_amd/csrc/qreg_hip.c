@@ -92,21 +92,24 @@ static ph2_sched_fn g_sched_fn;
 static void *g_sched_ctx;
 
 /* Tile width when none is set, from 1024-term blocks timed at every tile
- * width, lex-ordered sweeps and random draws (us per block, sweep / draw):
- *   to 18 qubits, tile 10: 346 / 366 at 16 qubits and 405 / 450 at 18
- *     against 367 / 404 and 415 / 474 at tile 11, 118 against 147 at tile 9
- *     at 10 qubits.  A few dozen workgroups, bound by each pass's chain of
- *     terms and exchanges;
- *   19 to 21, tile 11: 674 / 853 at 20 and 988 / 894 at 21 against
- *     781 / 910 and 1205 / 1003 at tile 10, 721 / 896 and 1034 / 991 at 12;
- *   from 22, tile 13: 1732 / 1467 at 22, 6404 / 4707 at 24, 14744 / 9765 at
- *     25, 128310 / 75068 at 28 against 1773 / 1489, 6755 / 4825, 16834 /
- *     9901 and 143945 / 77109 at tile 12.  Traffic per pass weighs most and
- *     wider tiles need fewer passes.
+ * width, lex-ordered sweeps and random draws at low bits 2 (us per block,
+ * sweep / draw; settings in turn, median of seven):
+ *   to 18 qubits, tile 10: 351 / 373 at 16 qubits and 411 / 458 at 18
+ *     against 384 / 416 and 432 / 486 at tile 11, 119 / 198 against 155 /
+ *     245 at tile 9 at 10 qubits.  A few dozen workgroups, bound by each
+ *     pass's chain of terms and exchanges;
+ *   19 to 21, tile 11: 680 / 862 at 20 and 998 / 945 at 21 against
+ *     774 / 909 and 1221 / 1036 at tile 10, 751 / 907 and 1045 / 1002 at 12;
+ *   from 22, tile 13: 1768 / 1497 at 22, 6664 / 4919 at 24, 14922 / 9928 at
+ *     25, 125907 / 76237 at 28 against 1757 / 1529, 6973 / 4928, 16880 /
+ *     10136 and 141426 / 78530 at tile 12.  Traffic per pass weighs most and
+ *     wider tiles need fewer passes; at 22 the two are even.
  * Without replay of captured sweeps (ph2hip_replay_max_qb, 20 qubits by
- * default) launches weigh more below: 12 from 17 qubits, nqb - 5 under
- * that (at 16 qubits a Trotter step took 0.476 ms at tile 11, 0.503 at 10,
- * 0.532 at 9 and 0.564 at 12). */
+ * default): 12 from 17 qubits, nqb - 5 under that, as fitted when a launch
+ * cost more than a pass of the kernels.  It no longer does: the widths above
+ * are the faster ones there too (394 us at tile 10 against 411 at 11 for a
+ * sweep at 16 qubits, 447 against 613 at 12 at 18, 701 at 11 against 766 at
+ * 12 at 20). */
 static uint32_t auto_tile(uint32_t nqb)
 {
 	uint32_t t;
@@ -124,9 +127,9 @@ static uint32_t auto_tile(uint32_t nqb)
 /* Contiguous low bits the cut asks for under the automatic tile width: those
  * the caller set, but for the default (LOW_AUTO) 2, where rows of 64 bytes
  * leave one more dimension to gather than rows of 128.  Low 2 against 3:
- * random draws 366 and 393 us at 16 qubits, 450 and 493 at 18, 850 and 918
- * at 20; sweeps 346 and 348, 406 and 415, 673 and 675; 6547 and 6748 at 24,
- * 130562 and 134986 at 28.  Low 1 is slower from 30. */
+ * random draws 373 and 401 us at 16 qubits, 458 and 502 at 18, 862 and 930
+ * at 20; sweeps 351 and 353, 411 and 420, 680 and 680; 6664 and 6745 at 24,
+ * 125907 and 130379 at 28.  Low 1 is slower from 30. */
 #define LOW_AUTO 3
 static uint32_t auto_low(uint32_t low)
 {
@@ -139,19 +142,22 @@ static uint32_t auto_low(uint32_t low)
  * To 18 qubits the state lies in the L2s, where short rows cost less than
  * passes: with no low bits asked for, sweeps (whose masks have an even
  * number of flips, so that single low bits are dimensions none of them
- * needs) take a third fewer passes and 324 us instead of 347 at 16 qubits,
- * 290 / 311 at 14, 389 / 405 at 18, but random draws a fifth fewer and 378
- * instead of 366, 392 / 368 and 471 / 450.  The second cut, without low
+ * needs) take a third fewer passes and 328 us instead of 351 at 16 qubits,
+ * 295 / 316 at 14, 394 / 411 at 18, but random draws a fifth fewer and 384
+ * instead of 373, 401 / 378 and 479 / 458.  The second cut, without low
  * bits, is taken if it saves a quarter of the passes; to 12 qubits always
- * (271 / 281 and 211 / 218).  Low bits that the caller set stay.
+ * (276 / 286 and 218 / 225).  Low bits that the caller set stay.
  *
  * From 22 to 27 qubits a tile-12 pass is the shorter one: blocks of 1 to 40
- * terms that need as many passes at either width took 1.06, 1.05, 1.05,
- * 1.03, 1.015 and 1.07 times as long at tile 13 (22 to 27 qubits, mean of
- * 13 to 17 blocks each; 825 us against 1312 in one of nine terms at 27), 0.99
- * at 28 and 1.00 at 30.  The second cut, at tile 12, is taken unless tile 13
- * saves a twentieth of its passes; blocks of 1024 terms save a twelfth or more
- * (at 22 qubits 41 passes instead of 45, 1467 us instead of 1489). */
+ * terms that need as many passes at either width took 1.075, 1.078, 1.077,
+ * 1.039, 1.018 and 1.030 times as long at tile 13 (22 to 27 qubits,
+ * geometric mean of 17 to 23 blocks each, 0.99 at 28 and 1.01 at 29; a
+ * setting timed twice, all in turn, differed by 0.1 to 0.6% in the mean).
+ * Single blocks range from 0.87 to 1.32, and one of nine terms at 27 qubits
+ * took 1331 us against 815.  The second cut, at tile 12, is taken unless
+ * tile 13 saves a twentieth of its passes; blocks of 1024 terms save a
+ * twelfth or more (at 22 qubits 41 passes instead of 45, 1497 us instead of
+ * 1529). */
 static int second_cut(uint32_t nqb, uint32_t asked, uint32_t *tile,
 	uint32_t *low)
 {
