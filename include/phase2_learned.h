@@ -13,6 +13,8 @@
  *   f[85]      first micro-group reads HBM directly (0/1)
  *   f[86]      last micro-group writes HBM directly (0/1)
  *   f[87]      half-tile form (0/1)
+ * (f[85] and f[86] are 1 for every pass unless ph2hip_set_fused_direct is
+ * off and the pass is not in the half-tile form)
  * as y = ln(ms) - (nqb - 30) ln 2 (time per 2^30 amplitudes).  For a block of
  * terms the scheduler enumerates passes [i, j) that end where the next term
  * would widen the tile (or at the longest feasible end), for tile widths 12

@@ -11,12 +11,12 @@
 2. Training: the library's FP32 network (88 -> 64 -> 64 -> 1), Adam, on the
    GPU, 10% held out.
 3. Evaluation on 33-qubit blocks never used for training: the same blocks
-   are swept with (a) the greedy cut at tile 12 / low 3, (b) the greedy cut
+   are swept with (a) the library's automatic greedy cut, (b) the greedy cut
    at four tile/low settings, keeping the fastest (exhaustive tuning of the
    fixed setting), and (c) the learned schedule; wall time per block after
-   a synchronisation, and predicted-vs-measured error per pass.
+   a synchronisation, all in turn, and predicted-vs-measured error per pass.
 4. Evaluation on the composite integrator at 30 qubits (synth.cmpsit_n30):
-   greedy, exhaustive and learned schedules over whole cmpsit steps, with
+   automatic, exhaustive and learned schedules over whole cmpsit steps, with
    the overlaps compared bit for bit.
 Writes costmodel_params.npz, records.npy and train.json (steps 1-2), and
 report.json and report_cmpsit.json (steps 3-4) into DIR.
@@ -59,68 +59,78 @@ def collect_width(nqb, hm, blocks, rng):
     return rec
 
 
-def time_blocks(reg, xm, zm, phi, blocks, what=""):
-    out = []
-    for b in blocks:
-        s = slice(b * 1024, (b + 1) * 1024)
-        nat.synchronize()
-        t0 = time.perf_counter()
-        reg.rotate(xm[s], zm[s], phi[s])
-        nat.synchronize()
-        out.append(time.perf_counter() - t0)
-    log(f"eval {what}: {sum(out):.3f}s")
-    return out
+# greedy settings of the evaluations; (0, 3) is the library's default, the
+# automatic cut (13 / 2 from 28 qubits)
+AUTO = (0, 3)
+SETTINGS = (AUTO, (12, 3), (12, 4), (13, 3), (13, 4))
+
+
+def name(tb, low):
+    return "automatic_s" if (tb, low) == AUTO else f"greedy_{tb}_{low}_s"
+
+
+def in_turn(runs, rounds):
+    """Times of runs (name -> function returning seconds), one after the
+    other and back again, each round the other way: the card is faster in
+    its first seconds (the same passes took 17.9 s at first and 18.8 s
+    later).  One untimed round first; the least of each."""
+    best = {}
+    for k in range(rounds + 1):
+        for n in list(runs)[::-1 if k % 2 else 1]:
+            t = runs[n]()
+            if k:
+                best[n] = min(best.get(n, 1e300), t)
+    return best
 
 
 def eval_cmpsit(params, steps=1, log=log):
     """Composite integrator at 30 qubits (synth.cmpsit_n30, `steps` steps):
-    greedy 12/3, greedy at four tile/low settings (exhaustive tuning of the
-    fixed setting), learned; overlaps must agree bit for bit."""
+    the automatic cut, greedy at four tile/low settings (exhaustive tuning of
+    the fixed setting), learned; overlaps must agree bit for bit."""
     w = synth.cmpsit_n30()
     hm = w["hm"]
     prep = dict(det_idx=w["det_idx"], det_cf=w["det_cf"])
+    outs = {}
 
-    def run():
+    def run(key, tb, low, learned=False, prof=False):
+        nat.set_default(nat.FUSED, tb, low)
+        if learned:
+            cm.install(params, min_qb=28)
+        nat.prof_enable(prof)
+        nat.prof_records(reset=True)
         nat.synchronize()
         t0 = time.perf_counter()
-        out, _ = nat.cmpsit(hm, prep, 1, steps, w["length"], w["depth"],
-                            w["angle_det"], w["angle_rand"], w["seed"],
-                            want_state=False)
+        outs[key], _ = nat.cmpsit(hm, prep, 1, steps, w["length"], w["depth"],
+                                  w["angle_det"], w["angle_rand"], w["seed"],
+                                  want_state=False)
         nat.synchronize()
-        return out, time.perf_counter() - t0
+        t = time.perf_counter() - t0
+        log(f"cmpsit {key}: {t:.3f}s")
+        if prof:
+            nat.prof_enable(False)
+            return nat.prof_records(reset=True), cm.stats()
+        cm.uninstall()
+        return t
 
-    res = {}
-    outs = {}
-    best = (None, 1e300)
-    for tb, low in ((12, 3), (12, 4), (13, 3), (13, 4)):
-        nat.set_default(nat.FUSED, tb, low)
-        outs[(tb, low)], t = run()
-        res[f"greedy_{tb}_{low}_s"] = t
-        log(f"cmpsit greedy {tb}/{low}: {t:.3f}s")
-        if t < best[1]:
-            best = ((tb, low), t)
-    nat.set_default(nat.FUSED, 12, 3)
-    cm.install(params, min_qb=28)
-    nat.prof_enable(True)
-    nat.prof_records(reset=True)
-    out_l, t_l = run()
-    lrec = nat.prof_records(reset=True)
-    nat.prof_enable(False)
-    hits, misses = cm.stats()
+    runs = {name(*a): (lambda a=a: run(name(*a), *a)) for a in SETTINGS}
+    runs["learned_s"] = lambda: run("learned_s", *AUTO, learned=True)
+    res = in_turn(runs, 2)
+    lrec, (hits, misses) = run("learned_s", *AUTO, learned=True, prof=True)
     cm.uninstall()
-    log(f"cmpsit learned: {t_l:.3f}s")
+    nat.set_default(nat.FUSED, *AUTO)
     Xl, yl, _ = cm.features_from_records(lrec)
     m = cm.MLP()
     m.set_params(params)
     pl = m.forward(Xl)
     m.close()
     err = np.abs(np.exp(pl - yl) - 1.0)
-    same = all(np.array_equal(o, out_l) for o in outs.values())
+    same = all(np.array_equal(o, outs["learned_s"]) for o in outs.values())
+    fixed = min((name(*a) for a in SETTINGS[1:]), key=res.get)
     res.update(
-        steps=steps, learned_s=t_l,
-        learned_vs_greedy=res["greedy_12_3_s"] / t_l,
-        exhaustive_best=dict(tile=best[0][0], low=best[0][1], s=best[1]),
-        learned_vs_exhaustive=best[1] / t_l,
+        steps=steps,
+        learned_vs_automatic=res["automatic_s"] / res["learned_s"],
+        best_fixed=fixed,
+        learned_vs_best_fixed=res[fixed] / res["learned_s"],
         overlaps_bit_identical=bool(same),
         pass_median_rel_err=float(np.median(err)) if len(err) else None,
         pass_p90_rel_err=float(np.quantile(err, 0.9)) if len(err) else None,
@@ -132,34 +142,48 @@ EVAL_BLOCKS = [9, 27, 44, 61, 78, 95]
 
 
 def eval_n33(params, log=log):
-    """Held-out 33-qubit sweep blocks: greedy 12/3, greedy at four tile/low
-    settings (exhaustive tuning of the fixed setting), learned."""
+    """Held-out 33-qubit sweep blocks: the automatic cut, greedy at four
+    tile/low settings (exhaustive tuning of the fixed setting), learned
+    (schedules made beforehand, timed as scheduling_s)."""
     w = synth.trott_n33()
     xm33, zm33, phi33 = sorted_terms(w["hm"])
-    reg = nat.Register(33, nat.FUSED, 12, 4)
+    blocks = [tuple(np.ascontiguousarray(a[b * 1024:(b + 1) * 1024])
+                    for a in (xm33, zm33, phi33)) for b in EVAL_BLOCKS]
+    reg = nat.Register(33, nat.FUSED, *AUTO)
     reg.prep_multidet(w["det_idx"], w["det_cf"])
-    res = {}
-    best = (None, 1e300)
-    for tb, low in ((12, 3), (12, 4), (13, 3), (13, 4)):
-        reg.configure(nat.FUSED, tb, low)
-        t = time_blocks(reg, xm33, zm33, phi33, EVAL_BLOCKS,
-                        f"greedy {tb}/{low}")
-        res[f"greedy_{tb}_{low}_s"] = t
-        if sum(t) < best[1]:
-            best = ((tb, low), sum(t))
-    reg.configure(nat.FUSED, 12, 3)
     cm.install(params, min_qb=28)
-    # first sweep computes and caches the schedules, the second is timed
-    t_first = time_blocks(reg, xm33, zm33, phi33, EVAL_BLOCKS,
-                          "learned, first visit")
+    t0 = time.perf_counter()
+    scheds = [cm.schedule(x, z, 33) for x, z, _ in blocks]
+    t_sched = time.perf_counter() - t0
+    cm.uninstall()
+
+    def greedy(tb, low):
+        reg.configure(nat.FUSED, tb, low)
+        t = 0.0
+        for b in blocks:
+            nat.synchronize()
+            t0 = time.perf_counter()
+            reg.rotate(*b)
+            nat.synchronize()
+            t += time.perf_counter() - t0
+        log(f"eval {name(tb, low)}: {t:.3f}")
+        return t
+
+    def learned():
+        t = sum(time_sched(reg, *b, s, reps=1)
+                for b, s in zip(blocks, scheds))
+        log(f"eval learned_s: {t:.3f}")
+        return t
+
+    runs = {name(*a): (lambda a=a: greedy(*a)) for a in SETTINGS}
+    runs["learned_s"] = learned
+    res = in_turn(runs, 2)
     nat.prof_enable(True)
     nat.prof_records(reset=True)
-    t_learned = time_blocks(reg, xm33, zm33, phi33, EVAL_BLOCKS, "learned")
+    learned()
     lrec = nat.prof_records(reset=True)
     nat.prof_enable(False)
     ov_l = reg.overlap(w["det_idx"], w["det_cf"])
-    hits, misses = cm.stats()
-    cm.uninstall()
     reg.free()
     Xl, yl, lrec = cm.features_from_records(lrec)
     m = cm.MLP()
@@ -167,14 +191,12 @@ def eval_n33(params, log=log):
     pl = m.forward(Xl)
     m.close()
     err = np.abs(np.exp(pl - yl) - 1.0)
-    g = sum(res["greedy_12_3_s"])
+    fixed = min((name(*a) for a in SETTINGS[1:]), key=res.get)
     res.update(
-        learned_s=t_learned, learned_first_visit_s=t_first,
-        greedy_total_s=g, learned_total_s=float(sum(t_learned)),
-        learned_vs_greedy=float(g / sum(t_learned)),
-        exhaustive_best=dict(tile=best[0][0], low=best[0][1],
-                             total_s=best[1]),
-        learned_vs_exhaustive=float(best[1] / sum(t_learned)),
+        scheduling_s=t_sched,
+        learned_vs_automatic=res["automatic_s"] / res["learned_s"],
+        best_fixed=fixed,
+        learned_vs_best_fixed=res[fixed] / res["learned_s"],
         eval_blocks=EVAL_BLOCKS,
         learned_passes=int(len(lrec)),
         learned_low_bits=np.bincount(lrec["low_bits"], minlength=13
@@ -183,7 +205,6 @@ def eval_n33(params, log=log):
                                       ).tolist(),
         eval_pass_median_rel_err=float(np.median(err)),
         eval_pass_p90_rel_err=float(np.quantile(err, 0.9)),
-        cache_hits=hits, cache_misses=misses,
         overlap_after_learned=[ov_l.real, ov_l.imag])
     return res
 
@@ -246,22 +267,22 @@ def eval_dp(params, nqb=26, blocks=(3, 9, 15), log=log):
                        optimum_sum_ms=opt_ms, learned_sum_ms=float(lrn_ms),
                        optimum_passes=int(len(opt[0])),
                        learned_passes=int(len(lrn[0])))
-            for name, sch in (("greedy_12_3", cm.schedule(bx, bz, nqb,
+            for what, sch in (("greedy_12_3", cm.schedule(bx, bz, nqb,
                                                            greedy=(12, 3))),
-                              ("greedy_13_3", cm.schedule(bx, bz, nqb,
-                                                           greedy=(13, 3))),
+                              ("greedy_13_2", cm.schedule(bx, bz, nqb,
+                                                           greedy=(13, 2))),
                               ("learned", lrn), ("optimum", opt)):
-                row[name + "_s"] = time_sched(reg, bx, bz, bp, sch)
+                row[what + "_s"] = time_sched(reg, bx, bz, bp, sch)
             log(f"dp: {row}")
             rows.append(row)
     finally:
         cm.uninstall()
         reg.free()
     tot = {k: float(sum(r[k] for r in rows)) for k in
-           ("greedy_12_3_s", "greedy_13_3_s", "learned_s", "optimum_s")}
+           ("greedy_12_3_s", "greedy_13_2_s", "learned_s", "optimum_s")}
     return dict(nqb=nqb, blocks=list(blocks), rows=rows, totals=tot,
                 learned_vs_optimum=tot["optimum_s"] / tot["learned_s"],
-                learned_vs_greedy=tot["greedy_12_3_s"] / tot["learned_s"])
+                learned_vs_greedy=tot["greedy_13_2_s"] / tot["learned_s"])
 
 
 def main(argv=None):
