@@ -236,6 +236,10 @@ int ph2hip_gather_abs(const void *amp, uint64_t namp_total,
 int ph2hip_gather(const void *amp, uint32_t nqb, const uint64_t *idx,
 	size_t n, double *out);
 
+/* out[2k], out[2k+1] = amp[lo + k] for k < n.  Up to 2^13 amplitudes come
+ * through pinned memory: one launch and one wait. */
+int ph2hip_read(const void *amp, uint64_t lo, uint64_t n, double *out);
+
 /* ph2hip_gather without any device allocation: the indices and gathered
  * amplitudes pass through a fixed device array of the library (24 B per
  * entry for PH2HIP_GATHER_NOALLOC_MAX entries, 1.5 MiB on each device the

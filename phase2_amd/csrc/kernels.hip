@@ -1248,6 +1248,15 @@ __global__ __launch_bounds__(kFew) void k_gather_few(
 		out[threadIdx.x] = a[I.idx[threadIdx.x]];
 }
 
+// n neighbouring amplitudes to pinned host memory.
+__global__ __launch_bounds__(kBlock) void k_read(
+	const double2 *__restrict__ a, double2 *__restrict__ out, uint32_t n)
+{
+	const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+	if (k < n)
+		out[k] = a[k];
+}
+
 __global__ __launch_bounds__(kFew) void k_scatter_few(
 	double2 *__restrict__ a, const FewSet S, uint32_t n)
 {
@@ -3059,6 +3068,29 @@ int ph2hip_set_replay(uint32_t max_qb)
 uint64_t ph2hip_replay_hits(void)
 {
 	return g_replay_hits;
+}
+
+int ph2hip_read(const void *amp, uint64_t lo, uint64_t n, double *out)
+{
+	if (ensure_init())
+		return -1;
+	const double2 *a = (const double2 *)amp + lo;
+	if (n == 0)
+		return 0;
+	if (n <= kStageN) {
+		std::lock_guard<std::mutex> lock(g_stage_mu);
+		if (char *p = stage()) {
+			hipLaunchKernelGGL(k_read,
+				dim3(((uint32_t)n + kBlock - 1) / kBlock),
+				dim3(kBlock), 0, g_stream, a,
+				reinterpret_cast<double2 *>(p), (uint32_t)n);
+			HIPCHK(hipGetLastError());
+			HIPCHK(hipStreamSynchronize(g_stream));
+			memcpy(out, p, sizeof(double2) * n);
+			return 0;
+		}
+	}
+	return ph2hip_d2h(out, a, sizeof(double2) * n);
 }
 
 int ph2hip_gather(const void *amp, uint32_t nqb, const uint64_t *idx,

@@ -70,7 +70,10 @@ struct qreg_hip {
 	 * holds them with the queued writes applied; win_n = 0: none */
 	double *win;
 	uint64_t win_lo, win_n;
-	int reads;	/* single reads since the buffer last changed */
+	/* reads since the buffer last changed: the first one's window, whether
+	 * others left it; and whether they did between the two changes before */
+	uint64_t first_lo;
+	int reads, spread, wide;
 };
 
 /* One amplitude moved by itself costs a synchronous device copy (about
@@ -79,10 +82,15 @@ struct qreg_hip {
  * 10^5 amplitudes per second.  Writes are queued on the host and land in
  * one scatter (later writes to an index win) before anything else touches
  * the device buffer; reads are served from a host copy of an aligned
- * window of AMP_WIN amplitudes, taken after the queue has landed, kept
- * current by later qreg_setamp calls and dropped by every operation that
- * may change the buffer. */
+ * window, taken after the queue has landed, kept current by later
+ * qreg_setamp calls and dropped by every operation that may change the
+ * buffer.  AMP_WIN amplitudes cost 30 us to fetch, AMP_FIRST through pinned
+ * memory little more than one alone (11 us), and often one is all that is
+ * read between two changes: the first read after a change takes AMP_FIRST,
+ * one outside them AMP_WIN, and where reads spread like that the next change
+ * is followed by AMP_WIN at once. */
 #define AMP_WIN (UINT64_C(1) << 14)  /* 256 KiB */
+#define AMP_FIRST (UINT64_C(1) << 10)
 #define AMP_QMAX ((size_t)1 << 20)   /* 24 MiB of queued writes */
 
 static int g_mode = -1;
@@ -224,12 +232,10 @@ void ph2_sched_install(ph2_sched_fn fn, void *ctx)
 	g_sched_ctx = ctx;
 }
 
-/* Put the queued writes on the device and drop the read window: called
- * before anything else reads or changes the device buffer. */
-static int settle(struct qreg_hip *h, uint64_t namp)
+/* Put the queued writes on the device: called before anything else reads or
+ * changes the device buffer.  The read window holds them already. */
+static int land(struct qreg_hip *h, uint64_t namp)
 {
-	h->win_n = 0;
-	h->reads = 0;
 	if (h->nq == 0)
 		return 0;
 	const int rc = ph2hip_scatter_queue(h->damp, namp, h->qidx, h->qval,
@@ -238,9 +244,26 @@ static int settle(struct qreg_hip *h, uint64_t namp)
 	h->pending = 1;
 	if (rc < 0) {
 		h->err = -1;
+		h->win_n = 0;
 		log_error("qreg_setamp: %s", ph2hip_strerror());
 	}
 	return rc;
+}
+
+/* The buffer is about to change: the read window goes. */
+static void forget(struct qreg_hip *h)
+{
+	h->win_n = 0;
+	if (h->reads)
+		h->wide = h->spread;
+	h->reads = 0;
+	h->spread = 0;
+}
+
+static int settle(struct qreg_hip *h, uint64_t namp)
+{
+	forget(h);
+	return land(h, namp);
 }
 
 static void wait_pending(struct qreg_hip *h, const char *what)
@@ -296,12 +319,7 @@ int qreg_error(const struct qreg *reg)
 	/* a queued write fails, if at all, when it lands: land it now, and
 	 * wait for it (short ones are only sent to the stream) */
 	if (h->nq) {
-		const uint64_t lo = h->win_lo, n = h->win_n;
-		const int reads = h->reads;
-		settle(h, reg->namp);
-		h->win_lo = lo;
-		h->win_n = n;
-		h->reads = reads;
+		land(h, reg->namp);
 		wait_pending(h, "qreg_error");
 	}
 	return h->err;
@@ -421,37 +439,29 @@ void qreg_getamp(struct qreg *reg, uint64_t i, _Complex double *z)
 	if (!in_range(reg, i, "qreg_getamp"))
 		return;
 	if (!h->win_n || i - h->win_lo >= h->win_n) {
-		const int reads = h->reads;
-		if (settle(h, reg->namp) < 0)
+		h->win_n = 0;
+		if (land(h, reg->namp) < 0)
 			return;
-		/* the first read after a change is often the only one: it
-		 * takes the amplitude alone (11 us), the next the window
-		 * (30 us) */
-		h->reads = reads + 1;
-		if (reads == 0) {
-			double v[2];
-			if (ph2hip_gather(h->damp, reg->qb_lo, &i, 1, v) < 0)
-				set_err(reg, "qreg_getamp");
-			else
-				*z = CMPLX(v[0], v[1]);
-			return;
-		}
-		if (!h->win && !(h->win = malloc(AMP_WIN * 16))) {
+		if (!h->win && !(h->win = malloc((reg->namp < AMP_WIN ?
+					reg->namp : AMP_WIN) * 16))) {
 			log_error("qreg_getamp: alloc");
 			h->err = -1;
 			return;
 		}
-		const uint64_t lo = i & ~(AMP_WIN - 1);
-		const uint64_t n = reg->namp - lo < AMP_WIN ? reg->namp - lo :
-							       AMP_WIN;
-		if (ph2hip_d2h(h->win, (const char *)h->damp + lo * 16,
-			    n * 16) < 0) {
+		const uint64_t size = h->reads || h->wide ? AMP_WIN : AMP_FIRST;
+		const uint64_t lo = i & ~(size - 1);
+		const uint64_t n = reg->namp - lo < size ? reg->namp - lo : size;
+		if (ph2hip_read(h->damp, lo, n, h->win) < 0) {
 			set_err(reg, "qreg_getamp");
 			return;
 		}
 		h->win_lo = lo;
 		h->win_n = n;
+		if (!h->reads)
+			h->first_lo = i & ~(AMP_FIRST - 1);
+		h->reads = 1;
 	}
+	h->spread |= i - h->first_lo >= AMP_FIRST;
 	const double *v = h->win + 2 * (i - h->win_lo);
 	*z = CMPLX(v[0], v[1]);
 }
@@ -463,12 +473,8 @@ void qreg_setamp(struct qreg *reg, uint64_t i, _Complex double z)
 		return;
 	if (h->nq == h->qcap) {
 		if (h->qcap >= AMP_QMAX) {
-			/* the window already holds these writes: keep it */
-			const uint64_t lo = h->win_lo, n = h->win_n;
-			if (settle(h, reg->namp) < 0)
+			if (land(h, reg->namp) < 0)
 				return;
-			h->win_lo = lo;
-			h->win_n = n;
 		} else {
 			const size_t cap = h->qcap ? 2 * h->qcap : 1024;
 			uint64_t *qi = realloc(h->qidx, sizeof *qi * cap);
@@ -499,8 +505,7 @@ void qreg_zero(struct qreg *reg)
 {
 	struct qreg_hip *h = reg->backend;
 	h->nq = 0; /* every queued write would be overwritten */
-	h->win_n = 0;
-	h->reads = 0;
+	forget(h);
 	h->pending = 1;
 	if (ph2hip_zero(h->damp, reg->namp) < 0)
 		set_err(reg, "qreg_zero");
@@ -516,8 +521,7 @@ void qreg_sync_host_to_device(struct qreg *reg)
 		return;
 	}
 	h->nq = 0; /* every queued write would be overwritten */
-	h->win_n = 0;
-	h->reads = 0;
+	forget(h);
 	if (ph2hip_h2d(h->damp, reg->amp, reg->namp * 16) < 0)
 		set_err(reg, "qreg_sync_host_to_device");
 }
