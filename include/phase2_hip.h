@@ -63,8 +63,9 @@ int ph2hip_rotate_plain(void *amp, uint32_t nqb, const struct ph2hip_rot *rot,
 	size_t n);
 
 /* The same on a register of 1..8 qubits, one workgroup that keeps it in LDS
- * for up to 128 terms per launch.  Bit-identical to ph2hip_rotate_plain,
+ * for up to PH2HIP_SMALL_TERMS terms per launch.  Bit-identical to ph2hip_rotate_plain,
  * which it calls while profiling is enabled (a record per term). */
+#define PH2HIP_SMALL_TERMS 128
 int ph2hip_rotate_small(void *amp, uint32_t nqb, const struct ph2hip_rot *rot,
 	size_t n);
 

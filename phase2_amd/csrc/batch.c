@@ -379,7 +379,8 @@ static int run_round(struct batch *B, size_t r, size_t lim, int mode,
 					    g->nrot)) < 0)
 				return -1;
 			B->launches += mode == PH2_BATCH_PLAIN_EACH ? g->nrot :
-				(g->nrot + 127) / 128;
+				(g->nrot + PH2HIP_SMALL_TERMS - 1) /
+					PH2HIP_SMALL_TERMS;
 			continue;
 		}
 		const uint32_t t = tb < nqb ? tb : nqb;

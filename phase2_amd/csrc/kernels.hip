@@ -219,7 +219,7 @@ __global__ __launch_bounds__(kBlock) void k_rot_diag(
 // pair.  The plain pass costs such a register a launch per term (2.3 us of
 // host time and as much on the device for a few hundred bytes of work);
 // here a term is one LDS round trip, and a launch takes kSmallTerms.
-constexpr uint32_t kSmallQb = 8, kSmallTerms = 128;
+constexpr uint32_t kSmallQb = 8, kSmallTerms = PH2HIP_SMALL_TERMS;
 
 struct SmallTerm {
 	double c, s;
