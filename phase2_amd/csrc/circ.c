@@ -244,7 +244,7 @@ int circ_prepst(struct circ *ct)
 		for (size_t d = 0; d < ct->md.len; d++)
 			qreg_setamp(&ct->reg, ct->md.dets[d].idx,
 				ct->md.dets[d].cf);
-		return qreg_error(&ct->reg);
+		return qreg_hip_send(&ct->reg);
 	}
 	if (ct->stprep_kind == STPREP_COEFF_MATRIX)
 		return state_prep_coeff_expand_all(&ct->reg, &ct->sp_scratch,

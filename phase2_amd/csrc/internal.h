@@ -19,8 +19,13 @@ void *qreg_hip_aux(struct qreg *reg);
 int qreg_hip_set_aux(struct qreg *reg, void *aux, void (*aux_free)(void *));
 
 /* Device buffer of a register for work on the library's own stream
- * (qreg_hip.c): qreg_hip_device_ptr without its wait. */
+ * (qreg_hip.c): qreg_hip_device_ptr without its wait for rotations. */
 void *qreg_hip_buffer(struct qreg *reg);
+
+/* Send the queued amplitude writes to the device; returns the error flag:
+ * qreg_error without its wait, so that the host plans the first rotations
+ * while the device zeroes and writes. */
+int qreg_hip_send(struct qreg *reg);
 
 /* Stable sort of a term array (circ.c). */
 int circ_terms_sort(struct circ_hamil_term *t, size_t n, term_cmp cmp);
