@@ -495,9 +495,11 @@ static int time_round(struct batch *B, size_t lim, int batched, int mode,
 /* Autotuner: time the first round of some registers under each tile width,
  * then the fastest with fewer and with more contiguous low bits (every
  * setting gives the same state), and keep the fastest.  At most TUNE_REGS
- * registers, and so few that the five rounds timed are at most a quarter of
- * the work to come: over nine settings and always 16 registers, a batch of
- * 40 registers and three samples spent 9 of its 17 ms here.  Tiles wider
+ * registers from the front of the list, and so few that the five rounds timed
+ * are at most a quarter of the rounds to come: over nine settings and always
+ * 16 registers, a batch of 40 registers and three samples spent 9 of its 17
+ * ms here.  Each setting is timed once, so that in a new process the first
+ * launch of its kernel counts against it.  Tiles wider
  * than the narrowest register take the batch off its pipeline (18 ms
  * instead of 7), so they are timed, as what they are, only where the
  * pipelined choice is a tile below 11. */
