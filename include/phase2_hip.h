@@ -129,8 +129,8 @@ int ph2hip_set_fused_prefetch(uint32_t tile_bits, uint32_t amps,
 /* Replay of repeated fused sweeps on registers of at most max_qb qubits
  * (default 20, or PHASE2_HIP_REPLAY_QB; 0 turns it off): a
  * ph2hip_rotate_fused call whose arguments (register, terms with their
- * c and s, schedule) all equal an earlier call's -- a Trotter step's
- * circ_cache block from the second step on -- has its launches captured
+ * c and s, schedule) and kernel form (ph2hip_set_fused_*) all equal an
+ * earlier call's -- a Trotter step's circ_cache block from the second step on -- has its launches captured
  * into a hipGraph on its second occurrence and replayed from the third,
  * so the passes of a block go out as one submission.  The state is the
  * same whatever the setting.  Not while profiling.  Setting it drops the
