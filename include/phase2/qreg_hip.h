@@ -78,7 +78,9 @@ void ph2_sched_install(ph2_sched_fn fn, void *ctx);
  * and copies on any stream.  Returns when all work queued on the register so
  * far is done (amplitude writes, zeroing, rotations); work queued later is
  * not waited for: take the pointer again, or call ph2hip_synchronize, before
- * looking. */
+ * looking.  Take it again before each change of the buffer, too: qreg_getamp
+ * keeps amplitudes on the host from one change that it knows of to the
+ * next. */
 void *qreg_hip_device_ptr(struct qreg *reg);
 
 #ifdef __cplusplus
